@@ -45,6 +45,7 @@
 
 #include "../../include/dmtz.h"
 #include "mismatch.h"
+#include "pairs.h"
 #include "repair.h"
 
 using namespace dmtz;
@@ -64,9 +65,10 @@ enum : int {
     K_STARS = 16,                               // star codes re-evaluated from dirty lists
     K_DSW = 17,                                 // 2-saddle wall mismatch list
     K_WOVF = 18,                                // wall walks that outgrew their visited set
-    K_ASNEXT = 19,                              // next branch of the work-stealing path walk
-    K_DTILES = 20,                              // tiles whose masks the last detection read
-    K_NCTR = 21
+    K_ASNEXT = 19,                              // next face of the work-stealing path walk
+    K_ASTOTAL = 20,                             // steps of the listed paths
+    K_DTILES = 21,                              // tiles whose masks the last detection read
+    K_NCTR = 22
 };
 
 constexpr uint8_t FROZEN = 7;  // counter value of a vertex restored to f by the finisher
@@ -197,7 +199,7 @@ __device__ __forceinline__ void block_emit(i64 base, const uint64_t (&lo)[EMIT_V
         const uint64_t key = (uint64_t)(base + (i64)k * BLOCK + threadIdx.x) << 7;
         if ((lo[k] & 1ull) && at[0] < out.cap) out.l[0][at[0]] = key | LC_VERT;
         at[0] += lo[k] & 1ull;
-        uint64_t m = (lo[k] >> 1) & 0x3FFFull;
+        uint64_t m = out.l[1] ? (lo[k] >> 1) & 0x3FFFull : 0;
         while (m) {
             const int b = __builtin_ctzll(m);
             m &= m - 1;
@@ -285,17 +287,20 @@ __device__ __forceinline__ bool code_g_at(const T* g, Dims d, i64 v, StarCode* c
     return ((old.w[0] ^ sc.w[0]) | (old.w[1] ^ sc.w[1]) | (old.w[2] ^ sc.w[2]) | (old.w[3] ^ sc.w[3])) != 0;
 }
 
-// Mark vertex v and the (up to 8) cubes that have it as a corner in the dirty bitmaps of the
-// path checks.
-__device__ __forceinline__ void mark_vertex(Dims d, uint32_t v, uint32_t* cubes, uint32_t* vbits) {
-    atomicOr(vbits + (v >> 5), 1u << (v & 31u));
+// Mark vertex v and the (up to 8) cubes that have it as a corner, each at the vertex it is anchored
+// at, in the bitmap of the path checks. Anchors v - k and v - k - 1 along x share a word mostly.
+__device__ __forceinline__ void mark_vertex(Dims d, uint32_t v, uint32_t* marks) {
     i64 x, y, z;
     vxyz(d, (i64)v, x, y, z);
-    for (int k = 0; k < 8; k++) {
-        const i64 ax = x - (k & 1), ay = y - ((k >> 1) & 1), az = z - ((k >> 2) & 1);
-        if (ax < 0 || ay < 0 || az < 0 || ax > d.W - 2 || ay > d.H - 2 || az > d.D - 2) continue;
-        const ull cube = (ull)(az * (d.W - 1) * (d.H - 1) + ay * (d.W - 1) + ax);
-        atomicOr(cubes + (cube >> 5), 1u << (cube & 31u));
+    for (int k = 0; k < 4; k++) {
+        if (y < (k & 1) || z < (k >> 1)) continue;
+        const i64 a = (i64)v - (k & 1) * d.W - (k >> 1) * d.W * d.H;
+        uint32_t m = 1u << (a & 31);
+        if (x > 0) {
+            if (a & 31) m |= m >> 1;
+            else atomicOr(marks + (a >> 5) - 1, 0x80000000u);
+        }
+        atomicOr(marks + (a >> 5), m);
     }
 }
 
@@ -313,15 +318,15 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_g(const T* g
 
 // The list length is read on the device (*n_ptr, written by the kernel that filled the list), so
 // the host launches it without waiting; the grid strides over the list. Block 0 adds the length
-// to *stars, the count of star codes re-evaluated in the run. With cubes != null, every vertex
+// to *stars, the count of star codes re-evaluated in the run. With marks != null, every vertex
 // whose code changed is marked for the path checks (their results read nothing but star codes).
 // tile_nz follows the masks whose nonzero-ness changes.
 template <class T>
 __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const T* g, Dims d, StarCode* code,
                                                                          const CritMask* crit_f, CritMask* mm,
                                                                          const uint32_t* list, const ull* n_ptr,
-                                                                         ull* stars, uint32_t* cubes,
-                                                                         uint32_t* vbits, uint32_t* tile_nz) {
+                                                                         ull* stars, uint32_t* marks,
+                                                                         uint32_t* tile_nz) {
     const ull n = *n_ptr;
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(stars, n);
     for (ull i = (ull)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (ull)gridDim.x * BLOCK) {
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const
         bool nz_old = false, nz_new = false;
         const bool changed = code_g_at(g, d, (i64)v, code, crit_f, mm, &nz_old, &nz_new);
         if (nz_old != nz_new) atomicAdd(tile_nz + (v / EMIT_TILE), nz_new ? 1u : 0xFFFFFFFFu);
-        if (changed && cubes) mark_vertex(d, v, cubes, vbits);
+        if (changed && marks) mark_vertex(d, v, marks);
     }
 }
 
@@ -441,8 +446,11 @@ __global__ __launch_bounds__(BLOCK) void k_detect(const CritMask* mm, i64 n, con
     }
 }
 
-// f-critical cells owned by each vertex in f; type_mask selects which types are listed.
-__global__ __launch_bounds__(BLOCK) void k_fcrit(const StarCode* cf, Counts c, Lists4 out, ull* ctr, int type_mask) {
+// Critical cells owned by each vertex, from the masks of owned critical cells (own, as k_code leaves
+// them) or, when own is null, from the star codes; type_mask selects which types count, and a
+// type whose list is null is counted but not listed.
+__global__ __launch_bounds__(BLOCK) void k_fcrit(const CritMask* own, const StarCode* cf, Counts c, Lists4 out,
+                                                 ull* ctr, int type_mask) {
     const i64 base = (i64)blockIdx.x * EMIT_TILE;
     uint64_t keep = 0;
     if (type_mask & 1) keep |= 1ull;
@@ -456,9 +464,15 @@ __global__ __launch_bounds__(BLOCK) void k_fcrit(const StarCode* cf, Counts c, L
         lo[k] = 0;
         hi[k] = 0;
         if (v < c.N) {
-            uint64_t ilo;
-            uint32_t ihi;
-            code_masks(cf[v], lo[k], hi[k], ilo, ihi);
+            if (own) {
+                const CritMask m = own[v];
+                lo[k] = m.lo;
+                hi[k] = m.hi;
+            } else {
+                uint64_t ilo;
+                uint32_t ihi;
+                code_masks(cf[v], lo[k], hi[k], ilo, ihi);
+            }
             lo[k] &= keep;
             if (!(type_mask & 8)) hi[k] = 0;
         }
@@ -1044,181 +1058,179 @@ struct NoSink {
     __device__ void operator()(i64) const {}
 };
 
-// The separatrix checks run in two steps: one thread per (start cell, branch) walks and writes
-// its result at a fixed position; a combine step per start cell applies the reference's
-// "first branch that fails" rule and appends to the list in convergent code.
+// The separatrix checks read the pairings of f and g from pair words (pairs.h). Where branches are
+// walked (connectivity mode), one thread per (start cell, branch) writes its result at a fixed
+// position and a combine step per start cell applies the reference's "first branch that fails"
+// rule and appends to the list in convergent code.
 
-// get_false_ds_vpath main_3d.cu:4837-4959 over the f-critical edges.
+// Pair words (pairs.h) of every vertex of a field. Bound by the reads of the values and of the
+// codes' first two words (the whole 32-byte codes, as lines go).
 template <class T>
-__global__ __launch_bounds__(BLOCK) void k_ds_geo(const uint64_t* fce, ull n, const T* f, const StarCode* cf, const T* g,
-                                                  const StarCode* cg, Dims d, Counts c, PathList out) {
-    const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    bool has = false;
-    i64 e = -1, rec = -1;
-    if (i < n) {
-        const uint64_t r = fce[i];
-        e = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-        Repair<T, NoSink> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NoSink{});
-        has = R.ds_geometry(e, rec);
+__global__ __launch_bounds__(BLOCK) void k_pairs(const T* fld, const StarCode* code, Dims d, i64 n, uint32_t* out) {
+    const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= n) return;
+    i64 x, y, z;
+    vxyz(d, v, x, y, z);
+    out[v] = pair_word(fld, code, d, v, x, y, z);
+}
+
+// Where the pairings of f and g differ (pairs.h pair_mismatch), one byte per vertex, for every
+// vertex. pg (nullable) receives g's pair words.
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_mism_full(const T* g, const StarCode* code, const uint32_t* pf, Dims d,
+                                                     i64 n, uint8_t* mis, uint32_t* pg) {
+    const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    if (v >= n) return;
+    i64 x, y, z;
+    vxyz(d, v, x, y, z);
+    const uint32_t w = pair_word(g, code, d, v, x, y, z);
+    mis[v] = (uint8_t)pair_mismatch(pf[v], w);
+    if (pg) pg[v] = w;
+}
+
+// The same for the marked vertices alone (mark_vertex: the cubes around every vertex whose g code
+// changed since the last check; a pair word reads nothing but star codes and, to find a tet's
+// owner, the order of the values, which cannot change without the codes). A block takes the marks of
+// 32 * BLOCK vertices, clears them, lists the marked vertices in LDS and spreads them over its
+// threads, so that a few marks cost a pass over the bitmap (N / 8 bytes).
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_mism_marked(const T* g, const StarCode* code, const uint32_t* pf, Dims d,
+                                                       i64 n, uint32_t* marks, uint8_t* mis) {
+    __shared__ uint16_t list[32 * BLOCK];
+    __shared__ int wsum[BLOCK / 64];
+    const i64 w = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    uint32_t m = w < (n + 31) / 32 ? marks[w] : 0u;
+    if (!__syncthreads_or(m != 0u)) return;
+    if (m) marks[w] = 0u;
+    int wt;
+    int at = wave_excl_scan(__popc(m), wt);
+    const int wv = (int)(threadIdx.x >> 6);
+    if (__lane_id() == 0) wsum[wv] = wt;
+    __syncthreads();
+    int total = 0;
+    for (int i = 0; i < BLOCK / 64; i++) {
+        at += i < wv ? wsum[i] : 0;
+        total += wsum[i];
     }
-    out.push_block(has, e, rec);
+    for (; m; m &= m - 1) list[at++] = (uint16_t)(threadIdx.x * 32 + __builtin_ctz(m));
+    __syncthreads();
+    const i64 base = (i64)blockIdx.x * BLOCK * 32;
+    for (int i = threadIdx.x; i < total; i += BLOCK) {
+        const i64 v = base + list[i];
+        i64 x, y, z;
+        vxyz(d, v, x, y, z);
+        mis[v] = (uint8_t)pair_mismatch(pf[v], pair_word(g, code, d, v, x, y, z));
+    }
 }
 
-// Descending geometry checks over per-edge data computed once per run: endpoints and their f
-// pairings (ds_geometry compares only those with g's). pairing -1 is stored as ~0u.
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_ds_prepare(const uint64_t* fce, ull n, const T* f, const StarCode* cf,
-                                                      Dims d, Counts c, uint4* dsv, uint32_t* dse) {
-    const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const uint64_t r = fce[i];
-    const i64 e = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-    FieldGrad<T> F(f, cf, d, c);
-    i64 v1, v2;
-    edge_verts(d, c, e, v1, v2);
-    const i64 p1 = F.pv(v1), p2 = F.pv(v2);
-    dsv[i] = make_uint4((uint32_t)v1, (uint32_t)v2, p1 < 0 ? ~0u : (uint32_t)p1, p2 < 0 ? ~0u : (uint32_t)p2);
-    dse[i] = (uint32_t)e;
+// The walks' table of the tet across each face, in LDS: a divergent read of it costs no memory
+// access. Every thread of the block must call this.
+__device__ __forceinline__ void load_across(uint8_t* across) {
+    if (threadIdx.x < 24) across[threadIdx.x] = PT.across[threadIdx.x];
+    __syncthreads();
+}
+__device__ __forceinline__ void load_slot_steps(const Dims& d, i64* step) {
+    if (threadIdx.x < 14) step[threadIdx.x] = slot_step(d, threadIdx.x);
+    __syncthreads();
 }
 
-// get_false_ds_vpath (main_3d.cu:4837-4959) as ds_geometry does it: an edge is re-evaluated when
-// full is set or one of its endpoints had its g lower star re-evaluated since the last check
-// (its g pairing depends on nothing else); res keeps each edge's recorded vertex (-1: none).
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_ds_check(ull n, const uint4* dsv, const uint32_t* dse, const T* g,
-                                                    const StarCode* cg, Dims d, Counts c, const uint32_t* vbits,
-                                                    int full, int64_t* res, PathList out) {
-    const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    i64 rec = -1, e = -1;
-    if (i < n) {
-        const uint4 q = dsv[i];
-        e = (i64)dse[i];
-        const bool redo = full != 0 || ((vbits[q.x >> 5] >> (q.x & 31u)) & 1u) || ((vbits[q.y >> 5] >> (q.y & 31u)) & 1u);
-        if (redo) {
-            FieldGrad<T> G(g, cg, d, c);
-            const i64 p1 = q.z == ~0u ? -1 : (i64)q.z, p2 = q.w == ~0u ? -1 : (i64)q.w;
-            const bool b1 = p1 != -1 && p1 != G.pv((i64)q.x);
-            const bool b2 = p2 != -1 && p2 != G.pv((i64)q.y);
-            rec = b1 ? (i64)q.x : (b2 ? (i64)q.y : -1);
-            res[i] = rec;
-        } else {
-            rec = res[i];
+// get_false_ds_vpath (main_3d.cu:4837-4959). The reference compares the f and g edges of both
+// end vertices of every f-critical edge (v1, v2), v1 > v2, and records v1 if they differ there, else
+// v2 if they do there. Taken from the vertices: each vertex that differs records its f-critical
+// edges (bits of its f-critical mask) except those whose larger end differs too and records them.
+// A thread tests 16 vertices with one load, so an edge costs nothing unless an end differs (the
+// pass reads N bytes; 512^3, 11 checks: 5.8 ms with a thread and 36 bytes per edge -> 0.4 ms).
+constexpr int DS_V = 16;
+__global__ __launch_bounds__(BLOCK) void k_ds_list(const uint8_t* mis, const CritMask* critf, Dims d, Counts c, i64 n,
+                                                   PathList out) {
+    __shared__ i64 step[16];
+    load_slot_steps(d, step);
+    const i64 v0 = ((i64)blockIdx.x * BLOCK + threadIdx.x) * DS_V;
+    uint32_t hit = 0;
+    if (v0 < n) {
+        const uint4 q = *reinterpret_cast<const uint4*>(mis + v0);
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int k = 0; k < DS_V; k++) hit |= ((w[k >> 2] >> (8 * (k & 3) + 6)) & 1u) << k;
+        if (n - v0 < DS_V) hit &= (1u << (n - v0)) - 1u;
+    }
+    // f-critical edges of vertex v that v records
+    auto edges = [&](i64 v) {
+        uint32_t e = (uint32_t)(critf[v].lo >> LC_EDGE) & 0x3FFFu;
+        for (uint32_t up = e & 0x1555u; up; up &= up - 1) {  // even slots lead to larger indices
+            const int s = __builtin_ctz(up);
+            if (mis[v + step[s]] & MIS_SLOT) e &= ~(1u << s);
+        }
+        return e;
+    };
+    int cnt = 0;
+    for (uint32_t h = hit; h; h &= h - 1) cnt += __popc(edges(v0 + __builtin_ctz(h)));
+    if (!__syncthreads_or(cnt)) return;
+    ull at = block_alloc(out.ctr, cnt);
+    for (uint32_t h = hit; h; h &= h - 1) {
+        const i64 v = v0 + __builtin_ctz(h);
+        i64 x, y, z;
+        vxyz(d, v, x, y, z);
+        for (uint32_t e = edges(v); e; e &= e - 1) {
+            if (at < out.cap) {
+                out.id[at] = edge_id_dir(d, c, x, y, z, __builtin_ctz(e));
+                out.rec[at] = v;
+            }
+            at++;
         }
     }
-    out.push_block(rec >= 0, e, rec);
 }
 
-// Ascending branch walks (is_false main_3d.cu:4437-4497), thread = (f-critical face, cofacet k).
-// Connectivity mode (maxlab != null) first compares g's reached maximum with f's label
-// (main_3d.cu:4821-4826). res[2*j] = start tet if the branch fails else -1, res[2*j+1] = the
-// divergent tet.
-// Connectivity mode compares g's maximum with f's label (get_false_as_vpath_connectivity
-// main_3d.cu:4761-4835): maxlab holds f's labels per start face; with lab_from_f the start faces
-// are g's critical faces and f's label is computed here (the maximum f reaches from the tet when
-// f leaves the face critical, -1 otherwise: labels exist only for f's critical faces,
-// main_3d.cu:4689-4759).
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_as_branch(const uint64_t* fcf, ull n, const int64_t* maxlab, int lab_from_f,
-                                                     const T* f, const StarCode* cf, const T* g, const StarCode* cg,
-                                                     Dims d, Counts c, int64_t* res, ull* walk_ctr) {
-    const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (j >= 2 * n) return;
-    const ull i = j >> 1;
-    const int k = (int)(j & 1);
-    const uint64_t r = fcf[i];
-    const i64 t = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-    Repair<T, NoSink> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NoSink{});
-    i64 q0, q1;
-    R.cofacets(t, q0, q1);
-    const i64 q = k ? q1 : q0;
-    bool ovf = false, found = false;
-    i64 dv = -1;
-    bool check = q >= 0;
-    if (check && maxlab) check = R.paired_max(q, 1, c.N, ovf) != maxlab[2 * i + k];
-    if (check && lab_from_f) {
-        const i64 lab = R.F.pf(t) == -1 ? R.paired_max(q, 0, c.N, ovf) : -1;
-        check = R.paired_max(q, 1, c.N, ovf) != lab;
-    }
-    if (check) R.as_walk(q, c.N, found, dv, ovf);
-    res[2 * j] = found ? q : -1;
-    res[2 * j + 1] = dv;
-    if (ovf) atomicAdd(walk_ctr, 1ull);
+// Ascending checks (is_false main_3d.cu:4437-4497 from both cofacets of every f-critical face) in
+// geometry mode. f does not change, so the tets of f's ascending paths are listed once per run: the
+// steps of face i, first cofacet's path then the second's, at [off[i], off[i + 1]), one word per
+// step. A check then asks for every step, independently of all others, whether f and g pair its tet
+// alike (k_as_bad: a coalesced 4-byte read and a byte of mis per step, one bit out), and the first
+// differing step of a face is its first set bit (k_as_list). No check walks a path, and a check
+// costs the same whatever changed: 512^3 fBm, 320 M steps, 11 checks: 42 ms when each branch was
+// walked by a thread over star codes -> 7 ms; a 33 x 32 x 34 mixture, whose longest path has some
+// hundred steps, 227 -> 9 us per check.
+// A step word is 12 v + 2 type + 1 for the first step of a path (12 N < 2^32).
+__device__ __forceinline__ uint32_t step_word(const TetAt& a, bool first) {
+    return (uint32_t)a.v * 12u + 2u * (uint32_t)a.type + (first ? 1u : 0u);
 }
 
-// Precomputed ascending paths (geometry mode). A branch j is (f-critical face j / 2, cofacet
-// j % 2); its comparison steps (Repair::as_fpath) are fixed for the whole run.
-// The first k steps of a branch are kept by the counting walk, so that only longer branches are
-// walked a second time to place their steps; k is chosen per run from a memory budget
-// (as_keep_steps), between AS_K_MIN and AS_K_MAX.
-constexpr int AS_K_MIN = 8, AS_K_MAX = 64;
-constexpr unsigned AS_WS_BLOCKS = 2048;  // blocks of the work-stealing walk (eight per CU)
+// The paths of all faces, counted (cnt[i] = steps of face i, *total their sum) or, with FILL,
+// listed. Path lengths are heavy-tailed, so a lane takes a new face whenever its walks end, and each
+// loop round every busy lane advances by one step: one 4-byte read (the pair word) and one LDS read.
+// A wave claims AS_WS_CHUNK faces at a time from the shared counter (*next) and hands them to its
+// idle lanes. Bound by the latency of the pair-word reads, which lie near one another (faces are
+// listed in about vertex order). Walking twice is cheaper than keeping the counted steps.
+// (512^3 fBm: the count 54 ms and the fill with its copies 19 ms over star codes.)
+constexpr unsigned AS_WS_BLOCKS = 2048;  // eight blocks per CU
 // Beside the repair sweeps (on a second stream) the walk takes half the wave slots: its waves
-// run until every branch is walked, so with all slots the sweeps' kernels would wait for it.
+// run until every face is walked, so with all slots the sweeps' kernels would wait for it.
 constexpr unsigned AS_WS_BLOCKS_SIDE = 1024;
-constexpr size_t AS_KEEP_BYTES = (size_t)4 << 30;
-struct StoreFirst {
-    uint2* p;
-    int k;
-    DMTZ_HD void operator()(i64 i, i64 cur, i64 t) const {
-        if (i < k) p[i] = make_uint2((uint32_t)cur, (uint32_t)t);
-    }
-};
-inline int as_keep_steps(ull nb) {
-    const ull k = nb ? (ull)(AS_KEEP_BYTES / sizeof(uint2)) / nb : (ull)AS_K_MAX;
-    return (int)(k < (ull)AS_K_MIN ? AS_K_MIN : (k > (ull)AS_K_MAX ? AS_K_MAX : k));
-}
-struct StoreSteps {
-    uint2* p;
-    DMTZ_HD void operator()(i64 i, i64 cur, i64 t) const { p[i] = make_uint2((uint32_t)cur, (uint32_t)t); }
-};
-
-template <class T>
-__device__ i64 branch_tet(const uint64_t* fcf, ull j, const T* f, const StarCode* cf, Dims d, Counts c) {
-    const uint64_t r = fcf[j >> 1];
-    const i64 t = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-    Repair<T, NoSink> R(f, cf, f, cf, d, c, nullptr, 0, 0, 0, NoSink{});
-    i64 q0, q1;
-    R.cofacets(t, q0, q1);
-    return (j & 1) ? q1 : q0;
-}
-
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_as_count(const uint64_t* fcf, ull nb, const T* f, const StarCode* cf,
-                                                    Dims d, Counts c, ull* cnt, uint2* first, int keep, ull* walk_ctr) {
-    const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (j >= nb) return;
-    const i64 q = branch_tet(fcf, j, f, cf, d, c);
-    Repair<T, NoSink> R(f, cf, f, cf, d, c, nullptr, 0, 0, 0, NoSink{});
-    bool ovf = false;
-    cnt[j] = (ull)R.as_fpath(q, c.N, ovf, StoreFirst{first + j * (ull)keep, keep});
-    if (ovf) atomicAdd(walk_ctr, 1ull);
-}
-
-// k_as_count with work stealing: path lengths are heavy-tailed, so instead of one branch per
-// thread, every lane takes a new branch whenever its walk ends, and the waves run until the
-// branches are exhausted. Each loop round every busy lane advances its walk by one step, so a
-// wave's lanes stay busy until the last branches. A wave claims AS_WS_CHUNK branches at a time
-// from the shared counter (*next) and hands them to its idle lanes, so the one counter sees an
-// atomic per chunk rather than one per round. Same per-branch results as k_as_count.
 constexpr ull AS_WS_CHUNK = 1024;
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_as_count_ws(const uint64_t* fcf, ull nb, const T* f, const StarCode* cf,
-                                                       Dims d, Counts c, ull* cnt, uint2* first, int keep, ull* next,
-                                                       ull* walk_ctr) {
-    Repair<T, NoSink> R(f, cf, f, cf, d, c, nullptr, 0, 0, 0, NoSink{});
+template <bool FILL>
+__global__ __launch_bounds__(BLOCK) void k_as_walk(const uint64_t* fcf, ull nf, const uint32_t* pw, Dims d, i64 cap,
+                                                   uint32_t* cnt, const uint32_t* off, uint32_t* steps, ull* next,
+                                                   ull* total, ull* walk_ctr) {
+    __shared__ uint8_t across[24];
+    __shared__ uint8_t start[72];
+    if (threadIdx.x >= 64 && threadIdx.x < 64 + 72) start[threadIdx.x - 64] = PT.start[(threadIdx.x - 64) >> 1][threadIdx.x & 1];
+    load_across(across);
     const int lane = __lane_id();
-    bool busy = false;
+    bool busy = false, first = false;
     ull j = 0;
-    i64 cur = -1, n = 0;
-    ull cb = 0, ce = 0;  // the wave's unclaimed branches [cb, ce) (wave-uniform)
-    bool dry = false;    // the shared counter has passed nb (wave-uniform)
+    TetAt a{-1, 0, 0, 0, 0}, b{-1, 0, 0, 0, 0};  // the tet being visited; the second path's start
+    uint32_t at = 0;                              // FILL: next position
+    i64 n = 0;
+    ull sum = 0;
+    ull cb = 0, ce = 0;  // the wave's unclaimed faces [cb, ce) (wave-uniform)
+    bool dry = false;    // the shared counter has passed nf (wave-uniform)
     for (;;) {
         const ull idle = __ballot(!busy);
         if (idle && !(dry && cb >= ce)) {
             const ull nid = (ull)__popcll(idle);
             const ull rank = (ull)__popcll(idle & ((1ull << lane) - 1ull));
             const ull avail = ce - cb;
-            ull jj = nb;  // this lane's new branch, if idle (nb: none)
+            ull jj = nf;  // this lane's new face, if idle (nf: none)
             if (nid <= avail) {
                 jj = cb + rank;
                 cb += nid;
@@ -1230,195 +1242,101 @@ __global__ __launch_bounds__(BLOCK) void k_as_count_ws(const uint64_t* fcf, ull 
                     const unsigned lo = __shfl((unsigned)(nc & 0xffffffffu), leader, 64);
                     const unsigned hi = __shfl((unsigned)(nc >> 32), leader, 64);
                     nc = ((ull)hi << 32) | lo;
-                    dry = nc >= nb;
+                    dry = nc >= nf;
                 }
                 if (rank < avail) jj = cb + rank;
                 else if (!dry) jj = nc + (rank - avail);
                 if (!dry) {
-                    ce = nc + AS_WS_CHUNK < nb ? nc + AS_WS_CHUNK : nb;
+                    ce = nc + AS_WS_CHUNK < nf ? nc + AS_WS_CHUNK : nf;
                     cb = nc + (nid - avail) < ce ? nc + (nid - avail) : ce;
                 } else {
                     cb = ce;
                 }
             }
-            if (!busy && jj < nb) {
+            if (!busy && jj < nf) {
                 j = jj;
-                cur = branch_tet(fcf, j, f, cf, d, c);
+                const uint64_t r = fcf[j];
+                const i64 v = (i64)(r >> 7);
+                const int lt = (int)(r & 127u) - LC_TRI;
+                i64 x, y, z;
+                vxyz(d, v, x, y, z);
+                a = start_tet(d, v, (int)x, (int)y, (int)z, start[2 * lt]);
+                b = start_tet(d, v, (int)x, (int)y, (int)z, start[2 * lt + 1]);
+                if (a.v < 0) {
+                    a = b;
+                    b.v = -1;
+                }
                 n = 0;
-                if (cur < 0) cnt[j] = 0;  // no cofacet on this side: an empty path
-                else busy = true;
+                first = true;
+                if (FILL) at = off[j];
+                busy = a.v >= 0;
+                if (!FILL && !busy) cnt[j] = 0;
             }
         }
         if (__ballot(busy) == 0 && dry && cb >= ce) break;
         if (busy) {
-            bool fin = R.as_fpath_step(cur, n, StoreFirst{first + j * (ull)keep, keep});
-            if (!fin && n > c.N) {  // as_fpath's cap
-                atomicAdd(walk_ctr, 1ull);
-                fin = true;
+            const uint32_t out = pw_out(pw[a.v], a.type);
+            bool end = out == PW_NONE;
+            if (!end) {
+                if (FILL) steps[at++] = step_word(a, first);
+                first = false;
+                n++;
+                cross_face(d, a, across[4 * a.type + (int)out]);
+                end = a.v < 0;
+                if (!end && n > 2 * cap) {  // no V-path is that long
+                    atomicAdd(walk_ctr, 1ull);
+                    end = true;
+                    b.v = -1;
+                }
             }
-            if (fin) {
-                cnt[j] = (ull)n;
-                busy = false;
+            if (end) {
+                a = b;
+                b.v = -1;
+                first = true;
+                busy = a.v >= 0;
+                if (!FILL && !busy) {
+                    cnt[j] = (uint32_t)n;
+                    sum += (ull)n;
+                }
             }
         }
     }
-}
-
-// Steps of thread t's branch at off[t]: copied from the counting walk's first keep steps, or
-// walked again. Thread t takes branch order[t] (the check order of k_len_scatter: a wave's walks
-// are alike; off then holds the offsets in that order) or branch t when order is null.
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_as_fill(const uint64_t* fcf, ull nb, const uint32_t* order, const T* f,
-                                                   const StarCode* cf, Dims d, Counts c, const ull* off,
-                                                   const uint2* first, int keep, uint2* steps) {
-    const ull t = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= nb) return;
-    const ull j = order ? (ull)order[t] : t;
-    const ull a = off[t], n = off[t + 1] - a;
-    if (n <= (ull)keep) {
-        for (ull k = 0; k < n; k++) steps[a + k] = first[j * (ull)keep + k];
-        return;
-    }
-    const i64 q = branch_tet(fcf, j, f, cf, d, c);
-    Repair<T, NoSink> R(f, cf, f, cf, d, c, nullptr, 0, 0, 0, NoSink{});
-    bool ovf = false;
-    R.as_fpath(q, c.N, ovf, StoreSteps{steps + a});
-}
-
-// is_false (main_3d.cu:4437-4497) over the precomputed steps: the first step whose g partner
-// face differs from f's. A branch keeps its previous result unless full is set or one of its
-// tets lies in a cube marked dirty since the last check (a tet's g pairing can only change when
-// one of its vertices had its lower star re-evaluated).
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_as_check(ull nb, const ull* off, const uint2* steps, const T* g,
-                                                    const StarCode* cg, Dims d, Counts c, const uint32_t* cubes,
-                                                    int full, int64_t* res) {
-    const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (j >= nb) return;
-    const ull a = off[j], b = off[j + 1];
-    bool redo = full != 0;
-    for (ull s = a; s < b && !redo; s++) {
-        const uint32_t cube = steps[s].x / 6u;
-        redo = ((cubes[cube >> 5] >> (cube & 31u)) & 1u) != 0;
-    }
-    if (!redo) return;
-    FieldGrad<T> G(g, cg, d, c);
-    i64 found = -1, dv = -1;
-    bool done = a >= b;
-    ull s = a;
-    while (!done) {
-        const uint2 st = steps[s];
-        if (G.pt((i64)st.x) != (i64)st.y) {
-            found = (i64)steps[a].x;
-            dv = (i64)st.x;
-        }
-        s++;
-        done = found >= 0 || s >= b;
-    }
-    res[2 * j] = found;
-    res[2 * j + 1] = dv;
-}
-
-// Compact copies for the dirty test of the checks below: 32-bit branch offsets and the cube of
-// every step (needs fewer than 2^32 steps). Thread per branch.
-__global__ __launch_bounds__(BLOCK) void k_as_compact(ull nb, const ull* off, const uint2* steps, uint32_t* off32,
-                                                      uint32_t* cube) {
-    const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (j >= nb) return;
-    off32[j] = (uint32_t)off[j];
-    if (j == nb - 1) off32[nb] = (uint32_t)off[nb];
-    for (ull s = off[j]; s < off[j + 1]; s++) cube[s] = steps[s].x / 6u;
-}
-
-// Step counts in check order (cnt of branch order[t] at t), and a zero at nb for the scan.
-__global__ __launch_bounds__(BLOCK) void k_as_gather_cnt(ull nb, const uint32_t* order, const ull* cnt, ull* out) {
-    const ull t = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (t < nb) out[t] = cnt[order[t]];
-    else if (t == nb) out[nb] = 0;
-}
-
-// Branch order of the checks: the branches without a step first (the checks skip them), then
-// the others in chunks of LEN_CHUNK_BLOCKS * CS_PER_BLOCK consecutive branches, within a chunk
-// grouped by step count (capped at 255) so that a wave's walks have similar lengths. The
-// f-critical faces are listed in about vertex order, so a chunk covers a few planes of the grid
-// and the checks read one region at a time: neighbouring branches share the values and star
-// codes they read while these are cached. (Grouped by length over the whole grid, most branches
-// being a few steps long, every region was read again for each length.)
-// A counting sort like k_class_hist / k_class_scatter, with the key read from the counts.
-constexpr int LEN_BINS = 256;
-constexpr ull LEN_CHUNK_BLOCKS = 64;
-__device__ __forceinline__ int len_bin(const ull* cnt, ull j) { return (int)(cnt[j] < 255 ? cnt[j] : 255); }
-
-// Position of (block blk, length bin) in the count table of nblk blocks: bin 0 of every block,
-// then the chunks in order, each bin-major (the last chunk may be shorter). Bin 1 of block 0
-// is at nblk, so the scan there is the number of branches without a step.
-__device__ __forceinline__ ull len_slot(ull blk, int bin, ull nblk) {
-    if (bin == 0) return blk;
-    const ull b0 = blk / LEN_CHUNK_BLOCKS * LEN_CHUNK_BLOCKS;
-    const ull w = nblk - b0 < LEN_CHUNK_BLOCKS ? nblk - b0 : LEN_CHUNK_BLOCKS;
-    return nblk + b0 * (LEN_BINS - 1) + (ull)(bin - 1) * w + (blk - b0);
-}
-
-__global__ __launch_bounds__(BLOCK) void k_len_hist(ull nb, const ull* cnt, ull nblk, uint32_t* hist) {
-    __shared__ uint32_t h[LEN_BINS];
-    h[threadIdx.x] = 0;  // BLOCK == LEN_BINS
-    __syncthreads();
-    const ull base = (ull)blockIdx.x * CS_PER_BLOCK;
-    for (int k = 0; k < CS_V; k++) {
-        const ull j = base + (ull)k * BLOCK + threadIdx.x;
-        (void)wave_bin_claim(j < nb ? len_bin(cnt, j) : -1, h);
-    }
-    __syncthreads();
-    hist[len_slot(blockIdx.x, threadIdx.x, nblk)] = h[threadIdx.x];
-}
-
-__global__ __launch_bounds__(BLOCK) void k_len_scatter(ull nb, const ull* cnt, ull nblk, const uint32_t* first,
-                                                       uint32_t* order) {
-    __shared__ uint32_t h[LEN_BINS];
-    h[threadIdx.x] = first[len_slot(blockIdx.x, threadIdx.x, nblk)];
-    __syncthreads();
-    const ull base = (ull)blockIdx.x * CS_PER_BLOCK;
-    for (int k = 0; k < CS_V; k++) {
-        const ull j = base + (ull)k * BLOCK + threadIdx.x;
-        const int bin = j < nb ? len_bin(cnt, j) : -1;
-        const uint32_t slot = wave_bin_claim(bin, h);
-        if (bin >= 0) order[slot] = (uint32_t)j;
+    if (!FILL) {
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_down((unsigned long long)sum, o, 64);
+        if (lane == 0 && sum) atomicAdd(total, sum);
     }
 }
-static_assert(BLOCK == LEN_BINS, "k_len_hist keeps one bin per thread");
 
-// Per-step dirty bits of the compact path copies: bit s of sd is set when the tet of step s
-// lies in a marked cube. Each wave covers 4 x 64 consecutive steps, lane l the steps
-// 64k + l (k = 0..3): the cube ids are read coalesced, 4 bytes per step, with four independent
-// loads in flight per lane, and each 64-step word is one ballot.
-constexpr int SD_WORDS_PER_WAVE = 4;
-
-__global__ __launch_bounds__(BLOCK) void k_as_step_dirty(ull total, const uint32_t* cube, const uint32_t* cubes,
-                                                         uint64_t* sd) {
+// Bit s of bad: f and g pair the tet of step s differently. Each wave covers AS_BAD_WORDS x 64
+// consecutive steps, lane l the steps 64 k + l, with that many independent reads in flight per lane;
+// a 64-step word is one ballot.
+constexpr int AS_BAD_WORDS = 8;
+__global__ __launch_bounds__(BLOCK) void k_as_bad(ull total, const uint32_t* steps, const uint8_t* mis, uint64_t* bad) {
     const ull w = (ull)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
     const int lane = (int)(threadIdx.x & 63u);
-    const ull base = w * (64 * SD_WORDS_PER_WAVE);
-    uint32_t q[SD_WORDS_PER_WAVE];
+    const ull base = w * (64 * AS_BAD_WORDS);
+    uint32_t q[AS_BAD_WORDS], m[AS_BAD_WORDS];
 #pragma unroll
-    for (int k = 0; k < SD_WORDS_PER_WAVE; k++) {
+    for (int k = 0; k < AS_BAD_WORDS; k++) {
         const ull s = base + 64 * k + lane;
-        q[k] = s < total ? cube[s] : 0u;
+        q[k] = s < total ? steps[s] : 0u;
     }
 #pragma unroll
-    for (int k = 0; k < SD_WORDS_PER_WAVE; k++) {
+    for (int k = 0; k < AS_BAD_WORDS; k++) m[k] = mis[q[k] / 12u];
+#pragma unroll
+    for (int k = 0; k < AS_BAD_WORDS; k++) {
         const ull s = base + 64 * k + lane;
-        const bool dq = s < total && ((cubes[q[k] >> 5] >> (q[k] & 31u)) & 1u) != 0;
-        const uint64_t m = __ballot(dq);
-        if (lane == 0 && base + 64 * k < total) sd[(base >> 6) + k] = m;
+        const uint64_t r = __ballot(s < total && ((m[k] >> ((q[k] % 12u) >> 1)) & 1u) != 0u);
+        if (lane == 0 && base + 64 * k < total) bad[(base >> 6) + k] = r;
     }
 }
 
-// First step in [s, b) whose dirty bit is set, or b.
-__device__ __forceinline__ uint32_t next_dirty(const uint64_t* sd, uint32_t s, uint32_t b) {
+// First set bit of bits in [s, b), or b.
+__device__ __forceinline__ uint32_t next_set(const uint64_t* bits, uint32_t s, uint32_t b) {
     uint32_t r = b;
     for (uint32_t w = s >> 6; s < b && w <= (b - 1) >> 6 && r == b; w++) {
         const uint32_t lo = w << 6;
-        uint64_t m = sd[w];
+        uint64_t m = bits[w];
         if (lo < s) m &= ~0ull << (s - lo);
         if (b - lo < 64) m &= (1ull << (b - lo)) - 1ull;
         if (m) r = lo + (uint32_t)__builtin_ctzll(m);
@@ -1426,57 +1344,85 @@ __device__ __forceinline__ uint32_t next_dirty(const uint64_t* sd, uint32_t s, u
     return r;
 }
 
-// k_as_check over the compact copies. Thread t checks branch order[t], whose steps are at
-// [off32[t], off32[t + 1]) (the copies are laid out in check order, so a wave's offsets and dirty
-// words are adjacent); results stay indexed by branch. Threads start at check position t0: the
-// positions before it hold the branches without a step, whose result stays empty. Unless full, a
-// branch with no dirty step keeps its last result, and a branch whose
-// last result was "no mismatch" compares only its dirty steps, in order: the others matched then
-// and read unchanged star codes now. A branch that had a mismatch and has a dirty step is walked
-// again from its start.
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_as_check32(ull t0, ull nb, const uint32_t* order, const uint32_t* off32,
-                                                      const uint64_t* sd, const uint2* steps, const T* g,
-                                                      const StarCode* cg, Dims d, Counts c, int full, int64_t* res,
-                                                      uint32_t* fails) {
-    const ull t = t0 + (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= nb) return;
-    const uint32_t a = off32[t], b = off32[t + 1];
-    uint32_t s = a;
-    bool sparse = false;  // visit dirty steps only
-    if (!full) {
-        s = next_dirty(sd, a, b);
-        if (s >= b) return;
-    }
-    const ull j = order[t];
-    if (!full) {
-        sparse = res[2 * j] < 0;
-        if (!sparse) s = a;
-    }
-    FieldGrad<T> G(g, cg, d, c);
-    i64 found = -1, dv = -1;
-    while (s < b && found < 0) {
-        const uint2 st = steps[s];
-        if (G.pt((i64)st.x) != (i64)st.y) {
-            found = (i64)steps[a].x;
-            dv = (i64)st.x;
+// The reference takes a face's first cofacet whose path differs, and the first differing tet on
+// that path: the first set bit among the face's steps. AS_FACES faces per thread and one list
+// claim per block.
+constexpr int AS_FACES = 8;
+__global__ __launch_bounds__(BLOCK) void k_as_list(ull nf, const uint32_t* off, const uint64_t* bad,
+                                                   const uint32_t* steps, Dims d, PathList out) {
+    uint32_t hit[AS_FACES];
+    int cnt = 0;
+#pragma unroll
+    for (int k = 0; k < AS_FACES; k++) {
+        const ull i = ((ull)blockIdx.x * AS_FACES + k) * BLOCK + threadIdx.x;
+        hit[k] = ~0u;
+        if (i < nf) {
+            const uint32_t a = off[i], b = off[i + 1];
+            const uint32_t p = next_set(bad, a, b);
+            if (p < b) {
+                hit[k] = p;
+                cnt++;
+            }
         }
-        s = sparse ? next_dirty(sd, s + 1, b) : s + 1;
     }
-    // fails bit j mirrors res[2 * j] >= 0 (zeroed before a full check)
-    const bool was = !full && !sparse, now = found >= 0;
-    if (was != now) atomicXor(fails + (j >> 5), 1u << (j & 31u));
-    res[2 * j] = found;
-    res[2 * j + 1] = dv;
+    if (!__syncthreads_or(cnt)) return;
+    ull at = block_alloc(out.ctr, cnt);
+#pragma unroll
+    for (int k = 0; k < AS_FACES; k++) {
+        if (hit[k] == ~0u) continue;
+        if (at < out.cap) {
+            uint32_t p = hit[k];
+            const uint32_t q = steps[p];
+            uint32_t s = q;
+            while (!(s & 1u)) s = steps[--p];  // back to the path's first tet
+            out.id[at] = tet_id_of_vertex(d, s / 12u, (int)((s % 12u) >> 1));
+            out.rec[at] = tet_id_of_vertex(d, q / 12u, (int)((q % 12u) >> 1));
+        }
+        at++;
+    }
 }
 
-// With fails != null (bit j set when branch j failed), faces with neither branch failing skip the
-// result reads.
-__global__ __launch_bounds__(BLOCK) void k_as_combine(const int64_t* res, ull n, PathList out, const uint32_t* fails) {
+// Ascending branch walks, thread = (face, cofacet k): connectivity mode, and geometry mode on
+// grids whose paths are not listed. maxlab (nullable) holds f's maximum per start: a branch whose
+// maximum in g equals it does not fail (get_false_as_vpath_connectivity main_3d.cu:4761-4835). With
+// lab_from_f the start faces are g's critical faces and f's label is found here (the maximum f
+// reaches from the tet when f leaves the face critical, -1 otherwise: labels exist only for f's
+// critical faces, main_3d.cu:4689-4759). res[2*j] = start tet if the branch fails else -1,
+// res[2*j+1] = the divergent tet. A chain of dependent 4-byte reads; over star codes and ids the
+// 129 x 96 x 111 mixture's checks took 3.1 ms each, now 0.5.
+__global__ __launch_bounds__(BLOCK) void k_as_branch(const uint64_t* fcf, ull n, const int64_t* maxlab, int lab_from_f,
+                                                     const CritMask* critf, const uint32_t* pf, const uint32_t* pg,
+                                                     Dims d, i64 cap, int64_t* res, ull* walk_ctr) {
+    __shared__ uint8_t across[24];
+    load_across(across);
+    const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
+    if (j >= 2 * n) return;
+    const uint64_t r = fcf[j >> 1];
+    const i64 v = (i64)(r >> 7);
+    const int lc = (int)(r & 127u);
+    i64 x, y, z;
+    vxyz(d, v, x, y, z);
+    const TetAt a = start_tet(d, v, (int)x, (int)y, (int)z, PT.start[lc - LC_TRI][j & 1]);
+    bool ovf = false, found = false;
+    TetAt div = a;
+    bool check = a.v >= 0;
+    if (check && maxlab) check = paired_max(d, pg, across, a, cap, ovf) != maxlab[j];
+    if (check && lab_from_f) {
+        const bool fcrit = ((critf[v].lo >> lc) & 1ull) != 0;
+        const i64 lab = fcrit ? paired_max(d, pf, across, a, cap, ovf) : -1;
+        check = paired_max(d, pg, across, a, cap, ovf) != lab;
+    }
+    if (check) found = path_mismatch(d, pf, pg, across, a, cap, div, ovf);
+    res[2 * j] = found ? tet_id_at(d, a) : -1;
+    res[2 * j + 1] = found ? tet_id_at(d, div) : -1;
+    if (ovf) atomicAdd(walk_ctr, 1ull);
+}
+
+__global__ __launch_bounds__(BLOCK) void k_as_combine(const int64_t* res, ull n, PathList out) {
     const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
     bool has = false;
     i64 a = -1, b = -1;
-    if (i < n && (!fails || ((fails[(2 * i) >> 5] >> ((2 * i) & 31u)) & 3u) != 0)) {
+    if (i < n) {
         const int64_t* p = res + 4 * i;
         has = p[0] >= 0 || p[2] >= 0;
         a = p[0] >= 0 ? p[0] : p[2];
@@ -1485,63 +1431,34 @@ __global__ __launch_bounds__(BLOCK) void k_as_combine(const int64_t* res, ull n,
     out.push_block(has, a, b);
 }
 
-// k_as_combine over the failure bits (bit j set when branch j failed; the bits mirror
-// res[2 * j] >= 0): one thread per 32 faces, the 64 branch bits of one word pair, so that a face
-// without a failing branch costs one bit instead of a thread. Faces whose bits are set are read
-// twice: once to count what the thread appends, once to append it.
-__global__ __launch_bounds__(BLOCK) void k_as_combine_bits(const int64_t* res, ull n, PathList out,
-                                                           const uint32_t* fails) {
-    const ull t = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    const ull f0 = t * 32;
-    uint64_t fm = 0;  // bit 2i: face f0 + i has a failing branch
-    if (f0 < n) {
-        uint64_t bits = (uint64_t)fails[2 * t] | ((uint64_t)fails[2 * t + 1] << 32);
-        const ull nf = n - f0 < 32 ? n - f0 : 32;
-        if (nf < 32) bits &= (1ull << (2 * nf)) - 1ull;
-        fm = (bits | (bits >> 1)) & 0x5555555555555555ull;
-    }
-    uint64_t hm = 0;  // faces that append
-    for (uint64_t m = fm; m; m &= m - 1) {
-        const int b = __builtin_ctzll(m);
-        const int64_t* p = res + 4 * (f0 + (ull)(b >> 1));
-        if (p[0] >= 0 || p[2] >= 0) hm |= 1ull << b;
-    }
-    ull at = block_alloc(out.ctr, __popcll(hm));
-    for (uint64_t m = hm; m; m &= m - 1) {
-        const int b = __builtin_ctzll(m);
-        const int64_t* p = res + 4 * (f0 + (ull)(b >> 1));
-        if (at < out.cap) {
-            out.id[at] = p[0] >= 0 ? p[0] : p[2];
-            out.rec[at] = p[0] >= 0 ? p[1] : p[3];
-        }
-        at++;
-    }
+// Endpoint k of the f-critical edge of a record: the larger index first.
+__device__ __forceinline__ i64 edge_end(const i64* step, uint64_t r, int k) {
+    const i64 v = (i64)(r >> 7), w = v + step[(int)(r & 127u) - LC_EDGE];
+    return k == 0 ? (v > w ? v : w) : (v > w ? w : v);
 }
 
 // Endpoint labels of f (get_orginal_saddle_min_pairs / _max_pairs, main_3d.cu:4613-4759), one
 // thread per (f-critical edge, endpoint) and per (f-critical face, cofacet); ascending labels
 // are indexed by face (resolution of the shadowed index at main_3d.cu:4750).
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_labels(const uint64_t* fce, ull ne, const uint64_t* fcf, ull nf, const T* f,
-                                                  const StarCode* cf, Dims d, Counts c, int64_t* minlab,
+__global__ __launch_bounds__(BLOCK) void k_labels(const uint64_t* fce, ull ne, const uint64_t* fcf, ull nf,
+                                                  const uint32_t* pf, Dims d, i64 cap, int64_t* minlab,
                                                   int64_t* maxlab, ull* walk_ctr) {
+    __shared__ uint8_t across[24];
+    __shared__ i64 step[16];
+    load_across(across);
+    load_slot_steps(d, step);
     const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    Repair<T, NoSink> R(f, cf, f, cf, d, c, nullptr, 0, 0, 0, NoSink{});
     bool ovf = false;
     if (j < 2 * ne) {
-        const uint64_t r = fce[j >> 1];
-        const i64 e = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-        i64 a, b;
-        edge_verts(d, c, e, a, b);
-        minlab[j] = R.f_min_label((j & 1) ? b : a, c.N, ovf);
+        minlab[j] = paired_min(pf, step, edge_end(step, fce[j >> 1], (int)(j & 1)), cap, ovf);
     } else if (j < 2 * ne + 2 * nf) {
         const ull jj = j - 2 * ne;
         const uint64_t r = fcf[jj >> 1];
-        const i64 t = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-        i64 q0, q1;
-        R.cofacets(t, q0, q1);
-        const i64 q = (jj & 1) ? q1 : q0;
-        maxlab[jj] = q >= 0 ? R.paired_max(q, 0, c.N, ovf) : -1;
+        const i64 v = (i64)(r >> 7);
+        i64 x, y, z;
+        vxyz(d, v, x, y, z);
+        const TetAt a = start_tet(d, v, (int)x, (int)y, (int)z, PT.start[(int)(r & 127u) - LC_TRI][jj & 1]);
+        maxlab[jj] = paired_max(d, pf, across, a, cap, ovf);
     }
     if (ovf) atomicAdd(walk_ctr, 1ull);
 }
@@ -1549,20 +1466,16 @@ __global__ __launch_bounds__(BLOCK) void k_labels(const uint64_t* fce, ull ne, c
 // get_false_ds_vpath_connectivity main_3d.cu:4961-5062: thread = (f-critical edge, endpoint)
 // walks g's descending path; res[4*i + 2*k] = reached g minimum, res[4*i + 2*k + 1] = first
 // vertex on the walk whose f and g pairings differ.
-template <class T>
-__global__ __launch_bounds__(BLOCK) void k_ds_branch(const uint64_t* fce, ull n, const T* f, const StarCode* cf,
-                                                     const T* g, const StarCode* cg, Dims d, Counts c, int64_t* res,
+__global__ __launch_bounds__(BLOCK) void k_ds_branch(const uint64_t* fce, ull n, const uint32_t* pf,
+                                                     const uint32_t* pg, Dims d, i64 cap, int64_t* res,
                                                      ull* walk_ctr) {
+    __shared__ i64 step[16];
+    load_slot_steps(d, step);
     const ull j = (ull)blockIdx.x * BLOCK + threadIdx.x;
     if (j >= 2 * n) return;
-    const uint64_t r = fce[j >> 1];
-    const i64 e = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-    Repair<T, NoSink> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NoSink{});
-    i64 a, b;
-    edge_verts(d, c, e, a, b);
     i64 trouble = -1;
     bool ovf = false;
-    res[2 * j] = R.g_min_walk((j & 1) ? b : a, trouble, c.N, ovf);
+    res[2 * j] = g_min_of(pf, pg, step, edge_end(step, fce[j >> 1], (int)(j & 1)), trouble, cap, ovf);
     res[2 * j + 1] = trouble;
     if (ovf) atomicAdd(walk_ctr, 1ull);
 }
@@ -1702,18 +1615,15 @@ struct dmtz_ctx {
     uint64_t* d_fsorted[3] = {nullptr, nullptr, nullptr};
     uint8_t* d_ftmp[3] = {nullptr, nullptr, nullptr};
     size_t fk_cap[3] = {0, 0, 0}, fsorted_cap[3] = {0, 0, 0}, ftmp_cap[3] = {0, 0, 0};
-    uint2* d_as_first = nullptr;     // first steps per branch from the counting walk
-    size_t as_first_cap = 0;
-    uint32_t* d_as_off32 = nullptr;  // 32-bit branch offsets and per-step cubes for the dirty test
-    uint32_t* d_as_cube = nullptr;
-    uint32_t* d_as_order = nullptr;  // branches in check order (first nb), sort input (second nb)
-    uint64_t* d_as_sd = nullptr;     // per-step dirty bits
-    uint32_t* d_as_fails = nullptr;  // per-branch bit: the last check found a mismatch
-    size_t as_off32_cap = 0, as_cube_cap = 0, as_order_cap = 0, as_sd_cap = 0, as_fails_cap = 0;
+    uint32_t* d_pairf = nullptr;     // pair words of f and, where branches are walked, of g
+    uint32_t* d_pairg = nullptr;
+    uint8_t* d_mis = nullptr;        // per vertex: where the pairings of f and g differ
+    uint32_t* d_marks = nullptr;     // vertices whose d_mis is to be refreshed at the next path check
+    uint64_t* d_as_bad = nullptr;    // per listed step: f and g pair its tet differently
+    size_t pairf_cap = 0, pairg_cap = 0, mis_cap = 0, marks_cap = 0, as_bad_cap = 0;
     hipStream_t as_stream = nullptr;  // the ascending-path precompute, overlapping the first sweeps
     hipEvent_t as_ev_fork = nullptr, as_ev_count = nullptr, as_ev_done = nullptr;
-    ull* h_as_total = nullptr;        // pinned: total steps of the precomputed paths, and (low
-                                      // half of [1]) the branches without a step
+    ull* h_as_total = nullptr;        // pinned: total steps of the listed paths
     uint32_t* d_wall_scr = nullptr;  // wall walks: per-thread visited sets and stacks
     size_t wall_scr_cap = 0;
     uint32_t* d_wall_ovf = nullptr;  // wall walks to repeat with more slots (two lists)
@@ -1735,17 +1645,11 @@ struct dmtz_ctx {
     double dirty_total = 0;  // star codes re-evaluated incrementally in the last correction
     int64_t stalls = 0, finished = 0, radius = 0;  // finisher outcome of the last correction
     // precomputed ascending separatrix paths of f (geometry mode)
-    ull* d_as_cnt = nullptr;   // comparison steps per branch, then scanned into d_as_off
-    ull* d_as_off = nullptr;
-    uint2* d_as_steps = nullptr;  // (tet, f partner face) per step
-    uint32_t* d_cubes = nullptr;  // dirty-cube bitmap since the last path check
-    uint32_t* d_vbits = nullptr;  // dirty-vertex bitmap since the last path check
-    uint4* d_dsv = nullptr;       // per f-critical edge: endpoints and their f pairings
-    uint32_t* d_dse = nullptr;    // per f-critical edge: its id
-    int64_t* d_ds_res = nullptr;  // per f-critical edge: recorded vertex of the last check
+    uint32_t* d_as_cnt = nullptr;  // steps per f-critical face, then scanned into d_as_off
+    uint32_t* d_as_off = nullptr;
+    uint32_t* d_as_steps = nullptr;
     void* d_scan_tmp = nullptr;
-    size_t as_cnt_cap = 0, as_off_cap = 0, as_steps_cap = 0, cubes_cap = 0, scan_tmp_cap = 0;
-    size_t vbits_cap = 0, dsv_cap = 0, dse_cap = 0, ds_res_cap = 0;
+    size_t as_cnt_cap = 0, as_off_cap = 0, as_steps_cap = 0, scan_tmp_cap = 0, labels_cap = 0, walk_cap = 0;
 };
 
 namespace {
@@ -1784,44 +1688,33 @@ void free_paths(dmtz_ctx* ctx) {
     (void)hipFree(ctx->d_as_cnt);
     (void)hipFree(ctx->d_as_off);
     (void)hipFree(ctx->d_as_steps);
-    (void)hipFree(ctx->d_cubes);
-    (void)hipFree(ctx->d_vbits);
-    (void)hipFree(ctx->d_dsv);
-    (void)hipFree(ctx->d_dse);
-    (void)hipFree(ctx->d_ds_res);
     (void)hipFree(ctx->d_scan_tmp);
-    (void)hipFree(ctx->d_as_first);
-    ctx->d_as_first = nullptr;
-    ctx->as_first_cap = 0;
-    (void)hipFree(ctx->d_as_off32);
-    (void)hipFree(ctx->d_as_cube);
-    (void)hipFree(ctx->d_as_order);
-    (void)hipFree(ctx->d_as_sd);
-    (void)hipFree(ctx->d_as_fails);
-    ctx->d_as_off32 = ctx->d_as_cube = ctx->d_as_order = ctx->d_as_fails = nullptr;
-    ctx->d_as_sd = nullptr;
-    ctx->as_off32_cap = ctx->as_cube_cap = ctx->as_order_cap = ctx->as_sd_cap = ctx->as_fails_cap = 0;
+    (void)hipFree(ctx->d_pairf);
+    (void)hipFree(ctx->d_pairg);
+    (void)hipFree(ctx->d_mis);
+    (void)hipFree(ctx->d_marks);
+    (void)hipFree(ctx->d_as_bad);
+    (void)hipFree(ctx->d_labels);
+    (void)hipFree(ctx->d_walk);
+    ctx->d_as_cnt = ctx->d_as_off = ctx->d_as_steps = ctx->d_pairf = ctx->d_pairg = ctx->d_marks = nullptr;
+    ctx->d_scan_tmp = nullptr;
+    ctx->d_mis = nullptr;
+    ctx->d_as_bad = nullptr;
+    ctx->d_labels = ctx->d_walk = nullptr;
+    ctx->as_cnt_cap = ctx->as_off_cap = ctx->as_steps_cap = ctx->scan_tmp_cap = 0;
+    ctx->pairf_cap = ctx->pairg_cap = ctx->mis_cap = ctx->marks_cap = ctx->as_bad_cap = 0;
+    ctx->labels_cap = ctx->walk_cap = 0;
     (void)hipFree(ctx->d_wall_scr);
     (void)hipFree(ctx->d_wall_ovf);
     ctx->d_wall_scr = ctx->d_wall_ovf = nullptr;
     ctx->wall_scr_cap = ctx->wall_ovf_cap = 0;
-    ctx->d_as_cnt = ctx->d_as_off = nullptr;
-    ctx->d_as_steps = nullptr;
-    ctx->d_cubes = ctx->d_vbits = ctx->d_dse = nullptr;
-    ctx->d_dsv = nullptr;
-    ctx->d_ds_res = nullptr;
-    ctx->d_scan_tmp = nullptr;
-    ctx->as_cnt_cap = ctx->as_off_cap = ctx->as_steps_cap = ctx->cubes_cap = ctx->scan_tmp_cap = 0;
-    ctx->vbits_cap = ctx->dsv_cap = ctx->dse_cap = ctx->ds_res_cap = 0;
 }
 
 void free_fc(dmtz_ctx* ctx) {
     (void)hipFree(ctx->d_fc);
     (void)hipFree(ctx->d_path);
-    (void)hipFree(ctx->d_labels);
-    (void)hipFree(ctx->d_walk);
     ctx->d_fc = nullptr;
-    ctx->d_path = ctx->d_labels = ctx->d_walk = nullptr;
+    ctx->d_path = nullptr;
     ctx->fc_cap = 0;
 }
 
@@ -1882,8 +1775,6 @@ int grow_fc(dmtz_ctx* ctx, ull need) {
     ull cap = need + need / 4 + 4096;
     CK(hipMalloc(&ctx->d_fc, sizeof(uint64_t) * 4 * cap));
     CK(hipMalloc(&ctx->d_path, sizeof(int64_t) * 6 * cap));
-    CK(hipMalloc(&ctx->d_labels, sizeof(int64_t) * 4 * cap));
-    CK(hipMalloc(&ctx->d_walk, sizeof(int64_t) * 4 * cap));
     ctx->fc_cap = cap;
     return 0;
 }
@@ -2187,7 +2078,7 @@ struct Driver {
         CK(hipGetLastError());
         k_code_list_g<T><<<stride_blocks(15 * est), BLOCK, 0, ctx->stream>>>(
             g, d, ctx->d_code_g, ctx->d_critf, ctx->d_mm, ctx->d_dirty, ctx->d_ctr + K_DIRTY, ctx->d_ctr + K_STARS,
-            as_ready ? ctx->d_cubes : nullptr, as_ready ? ctx->d_vbits : nullptr, ctx->d_tile_nz);
+            as_ready ? ctx->d_marks : nullptr, ctx->d_tile_nz);
         CK(hipGetLastError());
         return 0;
     }
@@ -2309,21 +2200,21 @@ struct Driver {
     const uint64_t* as_gfaces = nullptr;
     ull n_gfaces = 0;
 
-    // f-critical cells of the types in type_mask into the f-critical lists (grown on demand).
-    int fcrit(int type_mask) { return fcrit_of(ctx->d_code_f, type_mask); }
-
-    // Critical cells of the types in type_mask of the field whose star codes are given, into the
-    // f-critical lists (grown on demand).
-    int fcrit_of(const StarCode* codes, int type_mask) {
+    // Critical cells of the types in type_mask into the f-critical lists (grown on demand), from the
+    // star codes given or, with codes null, from f's owned critical cells, which lie in d_mm between
+    // f_codes() and g_codes(). Types outside list_mask are counted but not listed.
+    int fcrit(const StarCode* codes, int type_mask, int list_mask = 15) {
         if (ctx->fc_cap == 0) {
             int rc0 = grow_fc(ctx, (ull)(c.N / 16));
             if (rc0) return rc0;
         }
         for (;;) {
             Lists4 FL = fcrit_lists(ctx);
+            for (int k = 0; k < 4; k++)
+                if (!((list_mask >> k) & 1)) FL.l[k] = nullptr;
             CK(hipMemsetAsync(ctx->d_ctr + K_FC0, 0, sizeof(ull) * 4, ctx->stream));
             k_fcrit<<<(unsigned)((c.N + EMIT_TILE - 1) / EMIT_TILE), BLOCK, 0, ctx->stream>>>(
-                codes, c, FL, ctx->d_ctr + K_FC0, type_mask);
+                codes ? nullptr : ctx->d_mm, codes, c, FL, ctx->d_ctr + K_FC0, type_mask);
             CK(hipGetLastError());
             int rc = sync_ctr(ctx);
             if (rc) return rc;
@@ -2335,90 +2226,120 @@ struct Driver {
         return 0;
     }
 
-    int prepare_paths() {
-        int rc = fcrit(2 | 4);
+    // The start cells of the separatrix checks: f-critical faces, and edges (listed in connectivity
+    // mode only: the geometry checks find them from the vertices). codes as for fcrit().
+    int prepare_paths(const StarCode* codes) {
+        const bool conn = fl.preserve_geometry != 1;
+        int rc = fcrit(codes, 2 | 4, conn ? 15 : 4);
         if (rc) return rc;
         Lists4 FL = fcrit_lists(ctx);
         nfce = ctx->h_ctr[K_FC0 + 1];
         nfcf = ctx->h_ctr[K_FC0 + 2];
-        if (fl.preserve_vpath == 1 && fl.preserve_geometry == 0 && nfce + nfcf) {
-            k_labels<T><<<nblocks(2 * (nfce + nfcf)), BLOCK, 0, ctx->stream>>>(
-                FL.l[1], nfce, FL.l[2], nfcf, f, ctx->d_code_f, d, c, ctx->d_labels, ctx->d_labels + 2 * ctx->fc_cap,
+        if (conn) {
+            rc = pairs_of(f, ctx->d_code_f, ctx->d_pairf, ctx->pairf_cap, ctx->stream);
+            if (rc) return rc;
+        }
+        if (conn && nfce + nfcf) {
+            rc = grow_buf(ctx, ctx->d_labels, ctx->labels_cap, 2 * (nfce + nfcf));
+            if (rc) return rc;
+            k_labels<<<nblocks(2 * (nfce + nfcf)), BLOCK, 0, ctx->stream>>>(
+                FL.l[1], nfce, FL.l[2], nfcf, ctx->d_pairf, d, c.N, ctx->d_labels, ctx->d_labels + 2 * nfce,
                 ctx->d_ctr + K_WALK);
             CK(hipGetLastError());
         }
         return 0;
     }
 
+    int pairs_of(const T* fld, const StarCode* codes, uint32_t*& out, size_t& cap, hipStream_t st) {
+        int rc = grow_buf(ctx, out, cap, (size_t)c.N);
+        if (rc) return rc;
+        k_pairs<T><<<nblocks(c.N), BLOCK, 0, st>>>(fld, codes, d, c.N, out);
+        CK(hipGetLastError());
+        return 0;
+    }
+
     // Separatrix detection (main_3d.cu:6955-6970): fills the ds / as lists.
     int detect_paths() {
         CK(hipMemsetAsync(ctx->d_ctr + K_DS, 0, sizeof(ull) * 2, ctx->stream));
-        Lists4 FL = fcrit_lists(ctx);
-        const bool conn = fl.preserve_geometry != 1;
-        const bool pre = as_precomputable();
-        if (pre && !as_ready && as_stage) {
-            int rc = as_join();
-            if (rc) return rc;
-        }
-        if (pre && !as_ready) {
-            int rc = as_prepare();
-            if (rc) return rc;
-        }
-        if (nfcf && pre) {
-            int rc = as_check();
-            if (rc) return rc;
-        } else if (conn && as_gfaces) {
-            if (n_gfaces) {
-                k_as_branch<T><<<nblocks(2 * n_gfaces), BLOCK, 0, ctx->stream>>>(
-                    as_gfaces, n_gfaces, nullptr, 1, f, ctx->d_code_f, g, ctx->d_code_g, d, c, ctx->d_walk,
-                    ctx->d_ctr + K_WALK);
-                CK(hipGetLastError());
-            }
-        } else if (nfcf) {
-            const int64_t* lab = conn ? ctx->d_labels + 2 * ctx->fc_cap : nullptr;
-            k_as_branch<T><<<nblocks(2 * nfcf), BLOCK, 0, ctx->stream>>>(FL.l[2], nfcf, lab, 0, f, ctx->d_code_f, g,
-                                                                         ctx->d_code_g, d, c, ctx->d_walk,
-                                                                         ctx->d_ctr + K_WALK);
-            CK(hipGetLastError());
-        }
-        const ull nstarts = conn && as_gfaces ? n_gfaces : nfcf;
-        if (nstarts && pre && as_compact) {
-            k_as_combine_bits<<<nblocks((nstarts + 31) / 32), BLOCK, 0, ctx->stream>>>(ctx->d_walk, nstarts,
-                                                                                      path_list(1), ctx->d_as_fails);
-            CK(hipGetLastError());
-        } else if (nstarts) {
-            k_as_combine<<<nblocks(nstarts), BLOCK, 0, ctx->stream>>>(ctx->d_walk, nstarts, path_list(1), nullptr);
-            CK(hipGetLastError());
-        }
-        if (nfce && pre) {
-            int rc = ds_check();
-            if (rc) return rc;
-        } else if (nfce) {
-            if (!conn) {
-                k_ds_geo<T><<<nblocks(nfce), BLOCK, 0, ctx->stream>>>(FL.l[1], nfce, f, ctx->d_code_f, g, ctx->d_code_g,
-                                                                      d, c, path_list(0));
-                CK(hipGetLastError());
-            } else {
-                k_ds_branch<T><<<nblocks(2 * nfce), BLOCK, 0, ctx->stream>>>(FL.l[1], nfce, f, ctx->d_code_f, g,
-                                                                             ctx->d_code_g, d, c, ctx->d_walk,
-                                                                             ctx->d_ctr + K_WALK);
-                CK(hipGetLastError());
-                k_ds_combine<<<nblocks(nfce), BLOCK, 0, ctx->stream>>>(FL.l[1], nfce, ctx->d_walk, ctx->d_labels, d, c,
-                                                                       path_list(0));
-                CK(hipGetLastError());
-            }
-        }
-        if (pre) {
-            int rc = paths_checked();
-            if (rc) return rc;
-        }
+        int rc = fl.preserve_geometry == 1 ? check_geometry() : check_connectivity();
+        if (rc) return rc;
         if (fl.preserve_connectors == 1) {
-            int rc = walls();
+            rc = walls();
             if (rc) return rc;
         }
-        int rc = sync_ctr(ctx);
+        rc = sync_ctr(ctx);
         if (rc) return rc;
         return overflow_check(ctx);
+    }
+
+    // Walks both branches of the n start faces and combines their results into the as list.
+    int as_branches(const uint64_t* faces, ull n, const int64_t* lab, int lab_from_f) {
+        if (!n) return 0;
+        int rc = grow_buf(ctx, ctx->d_walk, ctx->walk_cap, 4 * n);
+        if (rc) return rc;
+        k_as_branch<<<nblocks(2 * n), BLOCK, 0, ctx->stream>>>(faces, n, lab, lab_from_f, ctx->d_critf, ctx->d_pairf,
+                                                               ctx->d_pairg, d, c.N, ctx->d_walk, ctx->d_ctr + K_WALK);
+        CK(hipGetLastError());
+        k_as_combine<<<nblocks(n), BLOCK, 0, ctx->stream>>>(ctx->d_walk, n, path_list(1));
+        CK(hipGetLastError());
+        return 0;
+    }
+
+    int check_connectivity() {
+        int rc = pairs_of(g, ctx->d_code_g, ctx->d_pairg, ctx->pairg_cap, ctx->stream);
+        if (rc) return rc;
+        Lists4 FL = fcrit_lists(ctx);
+        rc = as_gfaces ? as_branches(as_gfaces, n_gfaces, nullptr, 1)
+                       : as_branches(FL.l[2], nfcf, ctx->d_labels + 2 * nfce, 0);
+        if (rc || !nfce) return rc;
+        rc = grow_buf(ctx, ctx->d_walk, ctx->walk_cap, 4 * nfce);
+        if (rc) return rc;
+        k_ds_branch<<<nblocks(2 * nfce), BLOCK, 0, ctx->stream>>>(FL.l[1], nfce, ctx->d_pairf, ctx->d_pairg, d, c.N,
+                                                                  ctx->d_walk, ctx->d_ctr + K_WALK);
+        CK(hipGetLastError());
+        k_ds_combine<<<nblocks(nfce), BLOCK, 0, ctx->stream>>>(FL.l[1], nfce, ctx->d_walk, ctx->d_labels, d, c,
+                                                               path_list(0));
+        CK(hipGetLastError());
+        return 0;
+    }
+
+    int check_geometry() {
+        int rc = as_stage ? as_join() : (as_ready ? 0 : as_prepare());
+        if (rc) return rc;
+        const size_t words = (size_t)(c.N + 31) / 32;
+        if (as_full || !as_listed) {
+            if (!as_listed) {
+                rc = grow_buf(ctx, ctx->d_pairg, ctx->pairg_cap, (size_t)c.N);
+                if (rc) return rc;
+            }
+            CK(hipMemsetAsync(ctx->d_marks, 0, sizeof(uint32_t) * words, ctx->stream));
+            k_mism_full<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(g, ctx->d_code_g, ctx->d_pairf, d, c.N, ctx->d_mis,
+                                                                     as_listed ? nullptr : ctx->d_pairg);
+        } else {
+            k_mism_marked<T><<<nblocks(words), BLOCK, 0, ctx->stream>>>(g, ctx->d_code_g, ctx->d_pairf, d, c.N,
+                                                                         ctx->d_marks, ctx->d_mis);
+        }
+        CK(hipGetLastError());
+        as_full = false;
+        if (nfcf && as_listed) {
+            if (as_total) {
+                k_as_bad<<<nblocks((as_total + AS_BAD_WORDS - 1) / AS_BAD_WORDS), BLOCK, 0, ctx->stream>>>(
+                    as_total, ctx->d_as_steps, ctx->d_mis, ctx->d_as_bad);
+                CK(hipGetLastError());
+            }
+            k_as_list<<<nblocks((nfcf + AS_FACES - 1) / AS_FACES), BLOCK, 0, ctx->stream>>>(
+                nfcf, ctx->d_as_off, ctx->d_as_bad, ctx->d_as_steps, d, path_list(1));
+            CK(hipGetLastError());
+        } else {
+            rc = as_branches(fcrit_lists(ctx).l[2], nfcf, nullptr, 0);
+            if (rc) return rc;
+        }
+        if (nfce) {
+            k_ds_list<<<nblocks((c.N + DS_V - 1) / DS_V), BLOCK, 0, ctx->stream>>>(ctx->d_mis, ctx->d_critf, d, c, c.N,
+                                                                                   path_list(0));
+            CK(hipGetLastError());
+        }
+        return 0;
     }
 
     // 2-saddle walls (preserve_connectors, main_3d.cu:5064-5133) from every f-critical face
@@ -2466,41 +2387,30 @@ struct Driver {
         return 0;
     }
 
-    // Ascending geometry checks over precomputed f paths: in geometry mode, when tet and face
-    // ids fit 32 bits.
-    bool as_ready = false, as_full = true, as_compact = false;
-    ull as_total = 0;  // steps of the compact path copies
+    // Geometry checks: the pair words of f and the listed ascending paths (one word per step), made
+    // once per run. Paths are listed when step words and face ids fit 32 bits and there are fewer than
+    // 2^32 steps; otherwise every check walks them.
+    bool as_ready = false, as_full = true, as_listed = false;
+    ull as_total = 0;  // steps of the listed paths
 
-    bool as_precomputable() const {
-        return fl.preserve_geometry == 1 && c.T < ((i64)1 << 32) && c.F < ((i64)1 << 32) && c.E < ((i64)1 << 32) &&
-               c.N < ((i64)1 << 32);
-    }
+    bool as_listable() const { return fl.preserve_geometry == 1 && c.F < ((i64)1 << 32) && 12 * c.N < ((i64)1 << 32); }
 
-    // Per-run precomputation of the separatrix checks (geometry mode): the ascending paths of f
-    // (flat steps per branch), the descending per-edge data, and the dirty bitmaps.
     int as_prepare() {
-        const ull nb = 2 * nfcf;
-        Lists4 FL = fcrit_lists(ctx);
-        int rc = nb ? as_paths(FL, nb) : 0;
-        if (rc) return rc;
-        rc = as_bitmaps_and_ds(FL, (size_t)(c.N >> 5) + 1, ctx->stream);
+        int rc = as_count(ctx->stream);
         if (rc) return rc;
         CK(hipStreamSynchronize(ctx->stream));
+        rc = as_fill(ctx->stream);
+        if (rc) return rc;
         return as_begin();
     }
 
-    // The precomputed paths are in place: the checks start with a full one, and the branches
-    // without a step, which the compact checks skip, keep an empty result.
-    ull as_n0 = 0;  // branches without a step (the first as_n0 of the check order)
-    int as_begin() {
+    int as_begin() {  // the paths are in place: the checks start with a full one
         as_ready = true;
         as_full = true;
-        as_n0 = as_compact ? (ctx->h_as_total[1] & 0xffffffffull) : 0;
-        if (as_compact && nfcf) CK(hipMemsetAsync(ctx->d_walk, 0xFF, sizeof(int64_t) * 4 * nfcf, ctx->stream));
         const char* lg = std::getenv("DMTZ_LOG");
         if (lg && lg[0] == '1')
-            std::fprintf(stderr, "dmtz ascending paths: %llu branches, %llu without a step, %llu steps\n",
-                         (unsigned long long)(2 * nfcf), (unsigned long long)as_n0, (unsigned long long)as_total);
+            std::fprintf(stderr, "dmtz ascending paths: %llu faces, %llu steps, %s\n", (unsigned long long)nfcf,
+                         (unsigned long long)as_total, as_listed ? "listed" : "walked");
         return 0;
     }
 
@@ -2513,7 +2423,7 @@ struct Driver {
     int as_stage = 0;
 
     int as_start_async() {
-        if (!ctx->fix_concurrent || !as_precomputable() || as_ready || !nfcf) return 0;
+        if (!ctx->fix_concurrent || !as_listable() || as_ready || !nfcf) return 0;
         if (!ctx->as_stream) {
             CK(hipStreamCreateWithFlags(&ctx->as_stream, hipStreamNonBlocking));
             CK(hipEventCreateWithFlags(&ctx->as_ev_fork, hipEventDisableTiming));
@@ -2522,7 +2432,7 @@ struct Driver {
         }
         CK(hipEventRecord(ctx->as_ev_fork, ctx->stream));
         CK(hipStreamWaitEvent(ctx->as_stream, ctx->as_ev_fork, 0));
-        int rc = as_paths_count(fcrit_lists(ctx), 2 * nfcf, ctx->as_stream, ctx->h_as_total);
+        int rc = as_count(ctx->as_stream);
         if (rc) return rc;
         CK(hipEventRecord(ctx->as_ev_count, ctx->as_stream));
         as_stage = 1;
@@ -2539,10 +2449,7 @@ struct Driver {
         } else {
             CK(hipEventSynchronize(ctx->as_ev_count));
         }
-        Lists4 FL = fcrit_lists(ctx);
-        int rc = as_paths_fill(FL, 2 * nfcf, ctx->as_stream, *ctx->h_as_total);
-        if (rc) return rc;
-        rc = as_bitmaps_and_ds(FL, (size_t)(c.N >> 5) + 1, ctx->as_stream);
+        int rc = as_fill(ctx->as_stream);
         if (rc) return rc;
         CK(hipEventRecord(ctx->as_ev_done, ctx->as_stream));
         as_stage = 2;
@@ -2553,173 +2460,65 @@ struct Driver {
     int as_join() {
         int rc = as_advance(true);
         if (rc) return rc;
-        if (as_stage == 2) {
-            CK(hipEventSynchronize(ctx->as_ev_done));  // usually long done: the sweeps take longer
-            CK(hipStreamWaitEvent(ctx->stream, ctx->as_ev_done, 0));
-            as_stage = 0;
-            return as_begin();
-        }
-        return 0;
+        CK(hipStreamWaitEvent(ctx->stream, ctx->as_ev_done, 0));
+        as_stage = 0;
+        return as_begin();
     }
 
-    // The ascending-path precompute in two phases on stream st: the counting walk and the scan of
-    // the step counts (the total lands in *h_total when st gets there), then, with the total on
-    // the host, the ordering, the fill and the compact copies.
-    int as_paths(const Lists4& FL, ull nb) {
-        int rc = as_paths_count(FL, nb, ctx->stream, ctx->h_as_total);
+    // First half, on stream st: f's pair words, the counting walk and the scan of its counts; the
+    // number of steps lands in *h_as_total when st gets there.
+    int as_count(hipStream_t st) {
+        const size_t words = (size_t)(c.N + 31) / 32;
+        int rc = pairs_of(f, ctx->d_code_f, ctx->d_pairf, ctx->pairf_cap, st);
         if (rc) return rc;
-        CK(hipStreamSynchronize(ctx->stream));
-        return as_paths_fill(FL, nb, ctx->stream, *ctx->h_as_total);
-    }
-
-    int as_paths_count(const Lists4& FL, ull nb, hipStream_t st, ull* h_total) {
-        int rc = grow_buf(ctx, ctx->d_as_cnt, ctx->as_cnt_cap, nb + 1);
+        rc = grow_buf(ctx, ctx->d_mis, ctx->mis_cap, (size_t)c.N + DS_V);
         if (rc) return rc;
-        rc = grow_buf(ctx, ctx->d_as_off, ctx->as_off_cap, nb + 1);
+        rc = grow_buf(ctx, ctx->d_marks, ctx->marks_cap, words);
         if (rc) return rc;
-        const int keep = as_keep_steps(nb);
-        rc = grow_buf(ctx, ctx->d_as_first, ctx->as_first_cap, nb * (ull)keep);
+        *ctx->h_as_total = 0;
+        as_listed = as_listable();
+        if (!as_listed || !nfcf) return 0;
+        rc = grow_buf(ctx, ctx->d_as_cnt, ctx->as_cnt_cap, nfcf + 1);
         if (rc) return rc;
-        CK(hipMemsetAsync(ctx->d_as_cnt + nb, 0, sizeof(ull), st));
-        CK(hipMemsetAsync(ctx->d_ctr + K_ASNEXT, 0, sizeof(ull), st));
-        const unsigned cap_blocks = st == ctx->stream ? AS_WS_BLOCKS : AS_WS_BLOCKS_SIDE;
-        const unsigned wsb = nblocks(nb) < cap_blocks ? nblocks(nb) : cap_blocks;
-        k_as_count_ws<T><<<wsb, BLOCK, 0, st>>>(FL.l[2], nb, f, ctx->d_code_f, d, c, ctx->d_as_cnt,
-                                                          ctx->d_as_first, keep, ctx->d_ctr + K_ASNEXT,
-                                                          ctx->d_ctr + K_WALK);
-        CK(hipGetLastError());
+        rc = grow_buf(ctx, ctx->d_as_off, ctx->as_off_cap, nfcf + 1);
+        if (rc) return rc;
         size_t tmp = 0;
-        CK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, ctx->d_as_cnt, ctx->d_as_off, (int)(nb + 1), st));
+        CK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, ctx->d_as_cnt, ctx->d_as_off, (int)(nfcf + 1), st));
         uint8_t* tp = (uint8_t*)ctx->d_scan_tmp;
         rc = grow_buf(ctx, tp, ctx->scan_tmp_cap, tmp);
         ctx->d_scan_tmp = tp;
         if (rc) return rc;
-        CK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tmp, ctx->d_as_cnt, ctx->d_as_off, (int)(nb + 1),
-                                            st));
-        CK(hipMemcpyAsync(h_total, ctx->d_as_off + nb, sizeof(ull), hipMemcpyDeviceToHost, st));
-        return 0;
-    }
-
-    int as_paths_fill(const Lists4& FL, ull nb, hipStream_t st, ull total) {
-        const int keep = as_keep_steps(nb);
-        size_t tmp = 0;
-        CK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, ctx->d_as_cnt, ctx->d_as_off, (int)(nb + 1), st));
-        int rc = grow_buf(ctx, ctx->d_as_steps, ctx->as_steps_cap, total);
-        if (rc) return rc;
-        as_compact = total < ((ull)1 << 32) && nb < ((ull)1 << 31);
-        if (as_compact) {  // check order: by region, then path length (for the fill and the checks)
-            rc = grow_buf(ctx, ctx->d_as_order, ctx->as_order_cap, nb);
-            if (rc) return rc;
-            const ull nblk = (nb + CS_PER_BLOCK - 1) / CS_PER_BLOCK, m = nblk * LEN_BINS;
-            const size_t hist_bytes = (sizeof(uint32_t) * m + 255) / 256 * 256;
-            size_t tmp2 = 0;
-            CK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp2, (uint32_t*)nullptr, (uint32_t*)nullptr, (int)m, st));
-            uint8_t* tp2 = (uint8_t*)ctx->d_scan_tmp;
-            rc = grow_buf(ctx, tp2, ctx->scan_tmp_cap, 2 * hist_bytes + (tmp > tmp2 ? tmp : tmp2));
-            ctx->d_scan_tmp = tp2;
-            if (rc) return rc;
-            uint32_t* hist = reinterpret_cast<uint32_t*>(tp2);
-            uint32_t* first = reinterpret_cast<uint32_t*>(tp2 + hist_bytes);
-            k_len_hist<<<(unsigned)nblk, BLOCK, 0, st>>>(nb, ctx->d_as_cnt, nblk, hist);
-            CK(hipGetLastError());
-            CK(hipcub::DeviceScan::ExclusiveSum(tp2 + 2 * hist_bytes, tmp2, hist, first, (int)m, st));
-            k_len_scatter<<<(unsigned)nblk, BLOCK, 0, st>>>(nb, ctx->d_as_cnt, nblk, first, ctx->d_as_order);
-            CK(hipGetLastError());
-            // branches without a step: the first slot of length 1 (low half of h_as_total[1])
-            ctx->h_as_total[1] = 0;
-            CK(hipMemcpyAsync(ctx->h_as_total + 1, first + nblk, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-            // steps in check order: offsets from the counts taken in that order
-            k_as_gather_cnt<<<nblocks(nb + 1), BLOCK, 0, st>>>(nb, ctx->d_as_order, ctx->d_as_cnt,
-                                                                       ctx->d_as_off);
-            CK(hipGetLastError());
-            CK(hipcub::DeviceScan::ExclusiveSum(tp2 + 2 * hist_bytes, tmp, ctx->d_as_off, ctx->d_as_cnt,
-                                                (int)(nb + 1), st));
-            std::swap(ctx->d_as_cnt, ctx->d_as_off);
-            std::swap(ctx->as_cnt_cap, ctx->as_off_cap);
-        }
-        k_as_fill<T><<<nblocks(nb), BLOCK, 0, st>>>(FL.l[2], nb, as_compact ? ctx->d_as_order : nullptr, f,
-                                                              ctx->d_code_f, d, c, ctx->d_as_off, ctx->d_as_first,
-                                                              keep, ctx->d_as_steps);
+        CK(hipMemsetAsync(ctx->d_as_cnt + nfcf, 0, sizeof(uint32_t), st));
+        CK(hipMemsetAsync(ctx->d_ctr + K_ASNEXT, 0, sizeof(ull) * 2, st));
+        k_as_walk<false><<<as_walk_blocks(st), BLOCK, 0, st>>>(fcrit_lists(ctx).l[2], nfcf, ctx->d_pairf, d, c.N,
+                                                               ctx->d_as_cnt, nullptr, nullptr, ctx->d_ctr + K_ASNEXT,
+                                                               ctx->d_ctr + K_ASTOTAL, ctx->d_ctr + K_WALK);
         CK(hipGetLastError());
-        if (as_compact) {
-            rc = grow_buf(ctx, ctx->d_as_off32, ctx->as_off32_cap, nb + 1);
-            if (rc) return rc;
-            rc = grow_buf(ctx, ctx->d_as_cube, ctx->as_cube_cap, total + 1);
-            if (rc) return rc;
-            k_as_compact<<<nblocks(nb), BLOCK, 0, st>>>(nb, ctx->d_as_off, ctx->d_as_steps, ctx->d_as_off32,
-                                                                  ctx->d_as_cube);
-            CK(hipGetLastError());
-            rc = grow_buf(ctx, ctx->d_as_sd, ctx->as_sd_cap, (total + 63) / 64 + 1);
-            if (rc) return rc;
-            rc = grow_buf(ctx, ctx->d_as_fails, ctx->as_fails_cap, (nb + 31) / 32 + 1);
-            if (rc) return rc;
-            as_total = total;
-        }
+        CK(hipcub::DeviceScan::ExclusiveSum(ctx->d_scan_tmp, tmp, ctx->d_as_cnt, ctx->d_as_off, (int)(nfcf + 1), st));
+        CK(hipMemcpyAsync(ctx->h_as_total, ctx->d_ctr + K_ASTOTAL, sizeof(ull), hipMemcpyDeviceToHost, st));
         return 0;
     }
 
-    int as_bitmaps_and_ds(const Lists4& FL, size_t words, hipStream_t st) {
-        int rc = grow_buf(ctx, ctx->d_cubes, ctx->cubes_cap, words);
+    // Second half, with the number of steps on the host.
+    int as_fill(hipStream_t st) {
+        as_total = *ctx->h_as_total;
+        as_listed = as_listed && as_total < ((ull)1 << 32);
+        if (!as_listed || !nfcf || !as_total) return 0;
+        int rc = grow_buf(ctx, ctx->d_as_steps, ctx->as_steps_cap, as_total);
         if (rc) return rc;
-        rc = grow_buf(ctx, ctx->d_vbits, ctx->vbits_cap, words);
+        rc = grow_buf(ctx, ctx->d_as_bad, ctx->as_bad_cap, (as_total + 63) / 64);
         if (rc) return rc;
-        CK(hipMemsetAsync(ctx->d_cubes, 0, sizeof(uint32_t) * words, st));
-        CK(hipMemsetAsync(ctx->d_vbits, 0, sizeof(uint32_t) * words, st));
-        if (nfce) {
-            rc = grow_buf(ctx, ctx->d_dsv, ctx->dsv_cap, nfce);
-            if (rc) return rc;
-            rc = grow_buf(ctx, ctx->d_dse, ctx->dse_cap, nfce);
-            if (rc) return rc;
-            rc = grow_buf(ctx, ctx->d_ds_res, ctx->ds_res_cap, nfce);
-            if (rc) return rc;
-            k_ds_prepare<T><<<nblocks(nfce), BLOCK, 0, st>>>(FL.l[1], nfce, f, ctx->d_code_f, d, c,
-                                                                       ctx->d_dsv, ctx->d_dse);
-            CK(hipGetLastError());
-        }
-        return 0;
-    }
-
-    int as_check() {
-        if (!as_ready) {
-            int rc = as_prepare();
-            if (rc) return rc;
-        }
-        const ull nb = 2 * nfcf;
-        if (!nb) return 0;
-        if (as_compact) {
-            if (as_full) CK(hipMemsetAsync(ctx->d_as_fails, 0, sizeof(uint32_t) * ((nb + 31) / 32), ctx->stream));
-            if (!as_full && as_total) {
-                k_as_step_dirty<<<nblocks((as_total + SD_WORDS_PER_WAVE - 1) / SD_WORDS_PER_WAVE), BLOCK, 0,
-                                  ctx->stream>>>(as_total, ctx->d_as_cube, ctx->d_cubes, ctx->d_as_sd);
-                CK(hipGetLastError());
-            }
-            if (nb > as_n0)
-                k_as_check32<T><<<nblocks(nb - as_n0), BLOCK, 0, ctx->stream>>>(
-                    as_n0, nb, ctx->d_as_order, ctx->d_as_off32, ctx->d_as_sd, ctx->d_as_steps, g, ctx->d_code_g, d, c,
-                    as_full ? 1 : 0, ctx->d_walk, ctx->d_as_fails);
-        } else
-            k_as_check<T><<<nblocks(nb), BLOCK, 0, ctx->stream>>>(nb, ctx->d_as_off, ctx->d_as_steps, g,
-                                                                   ctx->d_code_g, d, c, ctx->d_cubes, as_full ? 1 : 0,
-                                                                   ctx->d_walk);
+        CK(hipMemsetAsync(ctx->d_ctr + K_ASNEXT, 0, sizeof(ull), st));
+        k_as_walk<true><<<as_walk_blocks(st), BLOCK, 0, st>>>(fcrit_lists(ctx).l[2], nfcf, ctx->d_pairf, d, c.N, nullptr,
+                                                              ctx->d_as_off, ctx->d_as_steps, ctx->d_ctr + K_ASNEXT,
+                                                              nullptr, ctx->d_ctr + K_WALK);
         CK(hipGetLastError());
         return 0;
     }
 
-    int ds_check() {
-        k_ds_check<T><<<nblocks(nfce), BLOCK, 0, ctx->stream>>>(nfce, ctx->d_dsv, ctx->d_dse, g, ctx->d_code_g, d, c,
-                                                                 ctx->d_vbits, as_full ? 1 : 0, ctx->d_ds_res,
-                                                                 path_list(0));
-        CK(hipGetLastError());
-        return 0;
-    }
-
-    // After a path check: both dirty bitmaps start empty and the next check is incremental.
-    int paths_checked() {
-        const size_t words = (size_t)(c.N >> 5) + 1;
-        CK(hipMemsetAsync(ctx->d_cubes, 0, sizeof(uint32_t) * words, ctx->stream));
-        CK(hipMemsetAsync(ctx->d_vbits, 0, sizeof(uint32_t) * words, ctx->stream));
-        as_full = false;
-        return 0;
+    unsigned as_walk_blocks(hipStream_t st) const {
+        const unsigned cap = st == ctx->stream ? AS_WS_BLOCKS : AS_WS_BLOCKS_SIDE, n = nblocks(nfcf);
+        return n < cap ? n : cap;
     }
 
     int fix_paths(ull nds, ull nas, ull nw) {
@@ -2736,7 +2535,7 @@ struct Driver {
     }
 
     int filtration() {
-        int rc = fcrit(15);
+        int rc = fcrit(nullptr, 15);
         if (rc) return rc;
         Lists4 FL = fcrit_lists(ctx);
         for (int ty = 0; ty < 4; ty++) {
@@ -2773,7 +2572,7 @@ struct Driver {
         CK(hipMemsetAsync(ctx->d_counter, 1, (size_t)c.N, ctx->stream));  // init_counter :6782
         bool paths = fl.preserve_vpath == 1;
         if (paths) {
-            rc = prepare_paths();
+            rc = prepare_paths(nullptr);
             if (rc) return rc;
         }
         rc = g_codes();  // gradient of g, main_3d.cu:6624-6638
@@ -3237,7 +3036,7 @@ int paths_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, co
     uint64_t* gfaces = nullptr;
     if (fl.preserve_geometry != 1) {
         // get_false_as_vpath_connectivity starts from g's critical faces (main_3d.cu:4766)
-        rc = drv.fcrit_of(ctx->d_code_g, 4);
+        rc = drv.fcrit(ctx->d_code_g, 4);
         if (rc) return rc;
         drv.n_gfaces = ctx->h_ctr[K_FC0 + 2];
         CK(hipMalloc(&gfaces, sizeof(uint64_t) * (drv.n_gfaces + 1)));
@@ -3250,7 +3049,7 @@ int paths_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, co
         }
         drv.as_gfaces = gfaces;
     }
-    rc = drv.prepare_paths();
+    rc = drv.prepare_paths(ctx->d_code_f);
     if (rc == 0) rc = drv.detect_paths();
     if (gfaces) {
         (void)hipStreamSynchronize(ctx->stream);
@@ -3322,7 +3121,7 @@ int walls_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, do
     if (rc) return rc;
     rc = drv.g_codes();
     if (rc) return rc;
-    rc = drv.prepare_paths();
+    rc = drv.prepare_paths(ctx->d_code_f);
     if (rc) return rc;
     rc = drv.walls();
     if (rc) return rc;
