@@ -43,11 +43,6 @@ void dmtz_ctx_destroy(dmtz_ctx* ctx) {
     free_fc(ctx);
     free_paths(ctx);
     (void)hipFree(ctx->d_ctr);
-    for (int k = 0; k < 3; k++) {
-        (void)hipFree(ctx->d_fk[k]);
-        (void)hipFree(ctx->d_fsorted[k]);
-        (void)hipFree(ctx->d_ftmp[k]);
-    }
     if (ctx->fix_stream) {
         (void)hipStreamSynchronize(ctx->fix_stream);
         (void)hipStreamDestroy(ctx->fix_stream);

@@ -8,7 +8,7 @@
 // Device work (one HIP stream per context):
 //   k_code        lower star of every vertex -> 32-byte star code (the gradient of
 //                 main_3d.cu:1930-2316 restricted to each vertex's lower star)
-//   k_critf       f-critical status of the 75 local cells of every vertex (once per run)
+//   k_critf_gather  f-critical status of the 75 local cells of every vertex (once per run)
 //   k_detect      mismatch records from the g star codes and the f-critical masks
 //                 (get_false_* main_3d.cu:2492-2550), 4 typed lists
 //   k_fix_cp      repair rules over a record list -> edit set (main_3d.cu:2554-4303)
@@ -16,8 +16,10 @@
 //   k_dirty, k_code_list
 //                 re-evaluation of the g star codes around the vertices whose value changed
 //   k_fcrit       f-critical cells (for separatrix checks and filtration)
-//   k_ds_geo, k_as_branch + k_as_combine, k_ds_branch + k_ds_combine, k_labels
-//                 separatrix checks (main_3d.cu:4437-5062)
+//   k_pairs, k_as_walk, k_mism_full / k_mism_marked, k_as_bad + k_as_list, k_ds_list
+//                 separatrix checks, geometry (main_3d.cu:4437-4497, 4837-4959)
+//   k_labels, k_as_branch + k_as_combine, k_ds_branch + k_ds_combine
+//                 separatrix checks, connectivity (main_3d.cu:4499-4835, 4961-5062)
 //   k_fix_paths   separatrix repairs (main_3d.cu:5135-5295)
 //   k_pin         filtration (main_3d.cu:2405-2490)
 //   k_zone_cells, k_zone, k_snap_boxes, k_tie_mark, k_tie_raise, k_freeze_all
@@ -47,6 +49,7 @@
 #include "mismatch.h"
 #include "pairs.h"
 #include "repair.h"
+#include "rules.h"
 
 using namespace dmtz;
 typedef unsigned long long ull;
@@ -541,199 +544,42 @@ struct HoldSink {
     }
 };
 
-// Branch classes of the repair rules: the first split of each rule, i.e. the cell's partner in f
-// (an edge with its vertex or a triangle; a triangle with an edge or a tet) or, when f leaves it
-// critical, its partner in g, and for the 2-saddle and maximum rules the next split (how the
-// partner's remaining vertex lies against the cell in f or g). The class only orders the records,
-// and the edit set does not depend on the order; but records of one class take the same
-// branches, so a wave of them runs one branch body instead of all of them. It is read from the
-// star codes: the record's vertex owns the cell in g, the f-critical masks tell whether f pairs
-// it, and the cell's owner in f (its highest vertex in f) holds f's partner.
-constexpr int FIX_CLASS_BITS = 4;  // classes 1..12
-
-template <class T, int TYPE>
-__global__ __launch_bounds__(BLOCK) void k_fix_class(const uint64_t* recs, ull n, const T* f, const StarCode* cf,
-                                                     const T* g, const StarCode* cg, const CritMask* critf, Dims d,
-                                                     Counts c, uint16_t* key) {
-    const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const uint64_t r = recs[i];
-    const i64 v = (i64)(r >> 7);
-    const int lc = (int)(r & 127u);
-    const CritMask cm = critf[v];
-    const bool fcrit = lc < 51 ? ((cm.lo >> lc) & 1ull) != 0 : ((cm.hi >> (lc - 51)) & 1u) != 0;
-    const FieldGrad<T> F(f, cf, d, c), G(g, cg, d, c);
-    auto nbv = [&](i64 u, int slot) {
-        i64 x, y, z;
-        vxyz(d, u, x, y, z);
-        return vidx(d, x + DIR[slot][0], y + DIR[slot][1], z + DIR[slot][2]);
-    };
-    // the cell's owner in f and its local index there
-    auto f_owner = [&](i64& m, int& lm) {
-        m = v;
-        lm = lc;
-        cell_at_other_vertices(d, v, lc, [&](i64 w, int lw) {
-            if (F.above(w, m)) {
-                m = w;
-                lm = lw;
-            }
-        });
-    };
-    int k = 0;
-    if (TYPE == 1) {  // fix_saddle main_3d.cu:2588-3037: partner in f, else in g
-        const i64 w = nbv(v, lc - LC_EDGE);
-        const i64 v1 = v > w ? v : w, v2 = v > w ? w : v;  // endpoints by index
-        if (fcrit) {
-            const int nib = code_edge(cg[v], lc - LC_EDGE);
-            if (nib < 14) {  // triangle with v3: are the endpoints ordered alike against v3 (:2886-2890)
-                const i64 v3 = nbv(v, nib);
-                k = G.above(v2, v3) == G.above(v1, v3) ? 6 : 7;
-            } else {
-                k = nib == 14 ? 5 : 8;
-            }
-        } else {
-            i64 m;
-            int lm;
-            f_owner(m, lm);
-            const int nib = code_edge(cf[m], lm - LC_EDGE);
-            if (nib < 14) {  // triangle with v3: is v3 below both endpoints in g or in f (:2643-2700)
-                const i64 v3 = nbv(m, nib);
-                const bool cheap = (G.above(v1, v3) && G.above(v2, v3)) || (F.above(v1, v3) && F.above(v2, v3));
-                k = cheap ? 2 : 3;
-            } else {
-                k = nib == 14 ? 1 : 4;
-            }
-        }
-    } else if (TYPE == 2) {  // fix_2saddle main_3d.cu:3039-3983
-        if (fcrit) {  // partner in g, from the g owner v
-            const int t = lc - LC_TRI;
-            const int cc = code_tri(cg[v], t);
-            if (cc < 2) {  // edge (v, n): its partner in f (:3488-3610)
-                const int sl = cc == 0 ? ST.tri_i[t] : ST.tri_j[t];
-                const i64 w = nbv(v, sl);
-                const int nib = F.above(w, v) ? code_edge(cf[w], sl ^ 1) : code_edge(cf[v], sl);
-                k = nib < 14 ? 7 : (nib == 14 ? 8 : 9);
-            } else if (cc < 4) {  // tet through n4: is n4 below the face in g (:3613-3980)
-                const i64 a = nbv(v, ST.tri_i[t]), b = nbv(v, ST.tri_j[t]), v4 = nbv(v, ST.tri_k[t][cc - 2]);
-                k = (G.above(a, v4) && G.above(b, v4)) ? 10 : 11;
-            } else {
-                k = 12;
-            }
-        } else {  // partner in f, from the f owner m
-            i64 m;
-            int lm;
-            f_owner(m, lm);
-            const int t = lm - LC_TRI;
-            const int cc = code_tri(cf[m], t);
-            const i64 a = nbv(m, ST.tri_i[t]), b = nbv(m, ST.tri_j[t]);
-            if (cc < 2) {  // edge (m, e) and the third vertex u (:3057-3223)
-                const i64 e = cc == 0 ? a : b, u = cc == 0 ? b : a;
-                const i64 v1 = m > e ? m : e, v2 = m > e ? e : m;
-                const bool v1e = G.above(v2, u), v2e = G.above(v1, u);
-                const bool o1 = F.above(v2, u), o2 = F.above(v1, u);
-                k = (v1e && v2e) ? 1 : ((o1 != o2 && v1e != v2e) ? 2 : 3);
-            } else if (cc < 4) {  // tet through n4: is n4 below the face in f (:3226-3477)
-                const i64 v4 = nbv(m, ST.tri_k[t][cc - 2]);
-                k = (F.above(a, v4) && F.above(b, v4)) ? 4 : 5;
-            } else {
-                k = 6;
-            }
-        }
-    } else if (TYPE == 3) {  // fix_maximum main_3d.cu:3985-4303: is the left-out vertex below the face
-        i64 m = v;
-        int lm = lc;
-        if (!fcrit) f_owner(m, lm);
-        const int q = lm - LC_TET;
-        const int cc = code_tet(fcrit ? cg[m] : cf[m], q);
-        if (cc < 3) {
-            const int s0 = ST.tet_s[q][0], s1 = ST.tet_s[q][1], s2 = ST.tet_s[q][2];
-            const int out = cc == 0 ? s0 : (cc == 1 ? s1 : s2);
-            const i64 w = nbv(m, out);
-            const i64 x = nbv(m, cc == 0 ? s1 : s0), y = nbv(m, cc == 2 ? s1 : s2);
-            const FieldGrad<T>& X = fcrit ? G : F;
-            k = (fcrit ? 3 : 1) + ((X.above(x, w) && X.above(y, w)) ? 0 : 1);
-        } else {
-            k = fcrit ? 5 : 6;
-        }
-    }
-    key[i] = (uint16_t)k;
-}
-
-// Grouping of one kind's records by branch class: a counting sort over the 2^FIX_CLASS_BITS
-// classes. Each block of CS_PER_BLOCK records counts its classes (k_class_hist, class-major
-// counts, so that their exclusive scan is every (class, block)'s first output slot), then
-// scatters its records there (k_class_scatter). Lanes of a wave that share a class claim their
-// slots with one LDS atomic. No pass waits on another block's progress, so the sort runs beside
-// other kernels without stalling.
-constexpr int CS_BINS = 1 << FIX_CLASS_BITS;
-constexpr int CS_V = 8;
-constexpr ull CS_PER_BLOCK = (ull)BLOCK * CS_V;
-
-// Slot of this lane among the lanes of its wave with the same bin, from a per-bin LDS counter:
-// one LDS atomic per distinct bin in the wave. Lanes with bin < 0 take no slot.
-__device__ __forceinline__ uint32_t wave_bin_claim(int bin, uint32_t* h) {
-    uint32_t slot = 0;
-    ull todo = __ballot(bin >= 0);
-    while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const int b = __shfl(bin, leader, 64);
-        const ull same = __ballot(bin == b);
-        uint32_t base = 0;
-        if (__lane_id() == leader) base = atomicAdd(h + b, (uint32_t)__popcll(same));
-        base = __shfl(base, leader, 64);
-        if (bin == b) slot = base + (uint32_t)__popcll(same & ((1ull << __lane_id()) - 1ull));
-        todo &= ~same;
-    }
-    return slot;
-}
-
-__global__ __launch_bounds__(BLOCK) void k_class_hist(const uint16_t* key, ull n, ull nblk, uint32_t* hist) {
-    __shared__ uint32_t h[CS_BINS];
-    if (threadIdx.x < CS_BINS) h[threadIdx.x] = 0;
-    __syncthreads();
-    const ull base = (ull)blockIdx.x * CS_PER_BLOCK;
-    for (int k = 0; k < CS_V; k++) {
-        const ull i = base + (ull)k * BLOCK + threadIdx.x;
-        (void)wave_bin_claim(i < n ? (int)(key[i] & (CS_BINS - 1)) : -1, h);
-    }
-    __syncthreads();
-    if (threadIdx.x < CS_BINS) hist[(ull)threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
-}
-
-__global__ __launch_bounds__(BLOCK) void k_class_scatter(const uint16_t* key, const uint64_t* recs, ull n, ull nblk,
-                                                         const uint32_t* first, uint64_t* out) {
-    __shared__ uint32_t h[CS_BINS];
-    if (threadIdx.x < CS_BINS) h[threadIdx.x] = first[(ull)threadIdx.x * nblk + blockIdx.x];
-    __syncthreads();
-    const ull base = (ull)blockIdx.x * CS_PER_BLOCK;
-    for (int k = 0; k < CS_V; k++) {
-        const ull i = base + (ull)k * BLOCK + threadIdx.x;
-        const int bin = i < n ? (int)(key[i] & (CS_BINS - 1)) : -1;
-        const uint32_t slot = wave_bin_claim(bin, h);
-        if (bin >= 0) out[slot] = recs[i];
-    }
-}
-
-// One kernel per cell type, so each holds only its own repair rule (one kernel over all types
-// needs twice the registers of the largest rule, and half the waves).
+// One kernel per cell type, so each holds only its own repair rule. The rule runs in vertex frames
+// (rules.h); a record whose numbers collide takes the rule over global ids, a wave-rare branch.
+// Bound by its two to five dependent reads (values, then a star code, then the partner's values and
+// code): a list of a few records takes 12 us (2-saddles; 80 over global ids). The records are taken in
+// the order of their lists: neighbouring records share the lines
+// they read, which is worth more than waves of one branch. (Over global ids, where a wave paid for
+// every branch body with thousands of instructions, the records were grouped by branch first; with
+// these rules the grouping costs 512^3 fBm 19 ms of 195 and 256^3 mixtures 13 of 122.)
 template <class T, int TYPE>
 __global__ __launch_bounds__(BLOCK) void k_fix_cp(const uint64_t* recs, ull n, const T* f, const StarCode* cf,
                                                   const T* g, const StarCode* cg, Dims d, Counts c,
                                                   const uint8_t* counter, double eps, double range, int edit_type,
                                                   TargetSink sink) {
+    __shared__ RuleTables tb;
+    __shared__ int32_t off[15];
+    if (threadIdx.x < sizeof(RuleTables) / 4)
+        reinterpret_cast<uint32_t*>(&tb)[threadIdx.x] = reinterpret_cast<const uint32_t*>(&RT)[threadIdx.x];
+    if (threadIdx.x < 15) off[threadIdx.x] = threadIdx.x == 14 ? 0 : (int32_t)slot_step(d, threadIdx.x);
+    __syncthreads();
     const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    Repair<T, HoldSink> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, HoldSink{sink, 0u, 0u, 0u, 0u, 0});
+    HoldSink hold{sink, 0u, 0u, 0u, 0u, 0};
     if (i < n) {
         const uint64_t r = recs[i];
-        const i64 v = (i64)(r >> 7);
+        const uint32_t v = (uint32_t)(r >> 7);
         const int lc = (int)(r & 127u);
-        const i64 id = local_cell_id(d, c, v, lc);
-        if (TYPE == 0) R.fix_minimum(id);
-        else if (TYPE == 1) R.fix_saddle(id);
-        else if (TYPE == 2) R.fix_2saddle(id);
-        else R.fix_maximum(id);
+        LocalRules<T, HoldSink> L{f, cf, g, cg, counter, &tb, off, d, c, eps, edit_type, hold};
+        if (__builtin_expect(!L.template run<TYPE>(v, lc), 0)) {
+            Repair<T, HoldSink> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, hold);
+            const i64 id = local_cell_id(d, c, (i64)v, lc);
+            if (TYPE == 1) R.fix_saddle(id);
+            else if (TYPE == 2) R.fix_2saddle(id);
+            else if (TYPE == 3) R.fix_maximum(id);
+            hold = R.sink;
+        }
     }
-    R.sink.flush();
+    hold.flush();
 }
 
 // Zero the counters whose bit is set in mask: one launch where a memset per run of counters
@@ -1139,7 +985,7 @@ __device__ __forceinline__ void load_slot_steps(const Dims& d, i64* step) {
 // v2 if they do there. Taken from the vertices: each vertex that differs records its f-critical
 // edges (bits of its f-critical mask) except those whose larger end differs too and records them.
 // A thread tests 16 vertices with one load, so an edge costs nothing unless an end differs (the
-// pass reads N bytes; 512^3, 11 checks: 5.8 ms with a thread and 36 bytes per edge -> 0.4 ms).
+// pass reads N bytes; 512^3 fBm, 11 checks: 5.8 ms with a thread and 36 bytes per edge -> 1.4 ms).
 constexpr int DS_V = 16;
 __global__ __launch_bounds__(BLOCK) void k_ds_list(const uint8_t* mis, const CritMask* critf, Dims d, Counts c, i64 n,
                                                    PathList out) {
@@ -1187,9 +1033,9 @@ __global__ __launch_bounds__(BLOCK) void k_ds_list(const uint8_t* mis, const Cri
 // step. A check then asks for every step, independently of all others, whether f and g pair its tet
 // alike (k_as_bad: a coalesced 4-byte read and a byte of mis per step, one bit out), and the first
 // differing step of a face is its first set bit (k_as_list). No check walks a path, and a check
-// costs the same whatever changed: 512^3 fBm, 320 M steps, 11 checks: 42 ms when each branch was
-// walked by a thread over star codes -> 7 ms; a 33 x 32 x 34 mixture, whose longest path has some
-// hundred steps, 227 -> 9 us per check.
+// costs the same whatever changed: 512^3 fBm, 320 M steps, 11 checks: 41 ms when each branch was
+// walked by a thread over star codes -> 15 ms with the refresh of mis; a 33 x 32 x 34 mixture, whose
+// longest path has some hundred steps, 230 -> 33 us per check.
 // A step word is 12 v + 2 type + 1 for the first step of a path (12 N < 2^32).
 __device__ __forceinline__ uint32_t step_word(const TetAt& a, bool first) {
     return (uint32_t)a.v * 12u + 2u * (uint32_t)a.type + (first ? 1u : 0u);
@@ -1201,7 +1047,7 @@ __device__ __forceinline__ uint32_t step_word(const TetAt& a, bool first) {
 // A wave claims AS_WS_CHUNK faces at a time from the shared counter (*next) and hands them to its
 // idle lanes. Bound by the latency of the pair-word reads, which lie near one another (faces are
 // listed in about vertex order). Walking twice is cheaper than keeping the counted steps.
-// (512^3 fBm: the count 54 ms and the fill with its copies 19 ms over star codes.)
+// (512^3 fBm: the count 54 -> 5 ms, the fill 19 -> 7 ms against walks over star codes.)
 constexpr unsigned AS_WS_BLOCKS = 2048;  // eight blocks per CU
 // Beside the repair sweeps (on a second stream) the walk takes half the wave slots: its waves
 // run until every face is walked, so with all slots the sweeps' kernels would wait for it.
@@ -1388,8 +1234,8 @@ __global__ __launch_bounds__(BLOCK) void k_as_list(ull nf, const uint32_t* off, 
 // lab_from_f the start faces are g's critical faces and f's label is found here (the maximum f
 // reaches from the tet when f leaves the face critical, -1 otherwise: labels exist only for f's
 // critical faces, main_3d.cu:4689-4759). res[2*j] = start tet if the branch fails else -1,
-// res[2*j+1] = the divergent tet. A chain of dependent 4-byte reads; over star codes and ids the
-// 129 x 96 x 111 mixture's checks took 3.1 ms each, now 0.5.
+// res[2*j+1] = the divergent tet. A chain of dependent 4-byte reads (129 x 96 x 111 mixture in
+// float64: 3.1 ms per check over star codes and ids, now 0.06).
 __global__ __launch_bounds__(BLOCK) void k_as_branch(const uint64_t* fcf, ull n, const int64_t* maxlab, int lab_from_f,
                                                      const CritMask* critf, const uint32_t* pf, const uint32_t* pg,
                                                      Dims d, i64 cap, int64_t* res, ull* walk_ctr) {
@@ -1606,15 +1452,10 @@ struct dmtz_ctx {
     uint64_t* d_rec = nullptr;    // 4 mismatch record lists of rec_cap entries
     uint64_t* d_fc = nullptr;     // 4 f-critical lists of fc_cap entries
     int64_t* d_path = nullptr;    // ds id/rec, as id/rec, wall id/rec (fc_cap each)
-    // Repairs of record types 1..3: class keys, grouped records and counting-sort scratch per type,
-    // and the second stream of the repair phase.
+    // The second stream of the repair phase.
     bool fix_concurrent = true;  // off in batch lanes: no second stream (repairs, path precompute)
     hipStream_t fix_stream = nullptr;
     hipEvent_t fix_fork = nullptr, fix_join = nullptr;
-    uint16_t* d_fk[3] = {nullptr, nullptr, nullptr};
-    uint64_t* d_fsorted[3] = {nullptr, nullptr, nullptr};
-    uint8_t* d_ftmp[3] = {nullptr, nullptr, nullptr};
-    size_t fk_cap[3] = {0, 0, 0}, fsorted_cap[3] = {0, 0, 0}, ftmp_cap[3] = {0, 0, 0};
     uint32_t* d_pairf = nullptr;     // pair words of f and, where branches are walked, of g
     uint32_t* d_pairg = nullptr;
     uint8_t* d_mis = nullptr;        // per vertex: where the pairings of f and g differ
@@ -1932,46 +1773,12 @@ struct Driver {
         return 0;
     }
 
-    // Repair phase of one critical-point sweep (main_3d.cu:6801-6833) + apply (:6837). The
-    // records of each kind are grouped by branch class, then the kinds are repaired concurrently
+    // Repair phase of one critical-point sweep (main_3d.cu:6801-6833) + apply (:6837). The kinds are
+    // repaired concurrently
     // (the edits form a set: their order does not matter): minima and 2-saddles on the context's
     // stream, saddles then maxima on a second one, so that one kind's longest chains of dependent
     // reads overlap another's work. Two streams rather than one per kind: the process's streams
     // share four hardware queues, and two streams on one queue run one after the other.
-
-    // Group the n records of kind ty (1..3) by branch class; recs then points at the grouped copy.
-    // Grouping only orders the records, so lists beyond 32-bit slots are left as they are, and
-    // so are short lists: a few blocks of records take as long as their slowest chain whatever
-    // their order, and the grouping's five launches would cost more than it saves.
-    static constexpr ull FIX_GROUP_MIN = 8192;
-    int sort_class(int ty, const uint64_t*& recs, ull n) {
-        if (n < FIX_GROUP_MIN || n >= (1ull << 32)) return 0;
-        const int k = ty - 1;
-        hipStream_t st = ctx->stream;
-        int rc = grow_buf(ctx, ctx->d_fk[k], ctx->fk_cap[k], n);
-        if (rc) return rc;
-        rc = grow_buf(ctx, ctx->d_fsorted[k], ctx->fsorted_cap[k], n);
-        if (rc) return rc;
-        auto cls = ty == 1 ? k_fix_class<T, 1> : ty == 2 ? k_fix_class<T, 2> : k_fix_class<T, 3>;
-        cls<<<nblocks(n), BLOCK, 0, st>>>(recs, n, f, ctx->d_code_f, g, ctx->d_code_g, ctx->d_critf, d, c,
-                                          ctx->d_fk[k]);
-        CK(hipGetLastError());
-        const ull nblk = (n + CS_PER_BLOCK - 1) / CS_PER_BLOCK, m = nblk * CS_BINS;
-        const size_t hist_bytes = (sizeof(uint32_t) * m + 255) / 256 * 256;
-        size_t tmp = 0;
-        CK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, (uint32_t*)nullptr, (uint32_t*)nullptr, (int)m, st));
-        rc = grow_buf(ctx, ctx->d_ftmp[k], ctx->ftmp_cap[k], 2 * hist_bytes + tmp);
-        if (rc) return rc;
-        uint32_t* hist = reinterpret_cast<uint32_t*>(ctx->d_ftmp[k]);
-        uint32_t* first = reinterpret_cast<uint32_t*>(ctx->d_ftmp[k] + hist_bytes);
-        k_class_hist<<<(unsigned)nblk, BLOCK, 0, st>>>(ctx->d_fk[k], n, nblk, hist);
-        CK(hipGetLastError());
-        CK(hipcub::DeviceScan::ExclusiveSum(ctx->d_ftmp[k] + 2 * hist_bytes, tmp, hist, first, (int)m, st));
-        k_class_scatter<<<(unsigned)nblk, BLOCK, 0, st>>>(ctx->d_fk[k], recs, n, nblk, first, ctx->d_fsorted[k]);
-        CK(hipGetLastError());
-        recs = ctx->d_fsorted[k];
-        return 0;
-    }
 
     int fix_cp(const ull counts[4]) {
         int rc = begin_edits(true);
@@ -1987,18 +1794,10 @@ struct Driver {
     int repair_records(const ull counts[4], ull& nrec) {
         Lists4 L = rec_lists(ctx);
         bool active[4];
-        const uint64_t* recs[4];
         nrec = 0;
-        int rc = 0;
         for (int ty = 0; ty < 4; ty++) {
             active[ty] = counts[ty] != 0 && !((ty == 1 || ty == 2) && fl.preserve_saddles != 1);
-            recs[ty] = L.l[ty];
-            if (!active[ty]) continue;
-            nrec += counts[ty];
-            if (ty != 0) {
-                rc = sort_class(ty, recs[ty], counts[ty]);
-                if (rc) return rc;
-            }
+            if (active[ty]) nrec += counts[ty];
         }
         const bool side = ctx->fix_concurrent && (active[1] || active[3]) && (active[0] || active[2]);
         if (side && !ctx->fix_stream) {
@@ -2015,7 +1814,7 @@ struct Driver {
             if (!active[ty]) continue;
             hipStream_t st = side && (ty == 1 || ty == 3) ? ctx->fix_stream : ctx->stream;
             auto kern = ty == 0 ? k_fix_cp<T, 0> : ty == 1 ? k_fix_cp<T, 1> : ty == 2 ? k_fix_cp<T, 2> : k_fix_cp<T, 3>;
-            kern<<<nblocks(counts[ty]), BLOCK, 0, st>>>(recs[ty], counts[ty], f, ctx->d_code_f, g, ctx->d_code_g, d,
+            kern<<<nblocks(counts[ty]), BLOCK, 0, st>>>(L.l[ty], counts[ty], f, ctx->d_code_f, g, ctx->d_code_g, d,
                                                         c, ctx->d_counter, eps, range, fl.edit_type, sink());
             CK(hipGetLastError());
         }
