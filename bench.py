@@ -269,7 +269,7 @@ def main():
                            traffic=int(det_prof["traffic_bytes_per_launch"]) if det_prof else None,
                            bytes_per_launch=int(bytes_per_launch), avg_launch_ms=round(avg_ms, 4),
                            launches=int(ks["launches"]),
-                           basis="4 B count per 2048-voxel tile + the 16-byte mismatch masks of the tiles with a mismatch read + 8 B per record written")
+                           basis="4 B count per 2048-voxel tile + the 12-byte mismatch masks of the tiles with a mismatch read + 8 B per record written")
 
     other = {}
     for r in [x for x in args.other_rel.split(",") if x.strip()]:

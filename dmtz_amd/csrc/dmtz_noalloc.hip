@@ -29,13 +29,13 @@ __global__ __launch_bounds__(64) void k_clear_counters(ull* ctr) {
 }
 
 // Critical cells each vertex owns, split into the two output masks of dmtz_classify_f32.
-__global__ __launch_bounds__(BLOCK) void k_crit_split(const StarCode* code, i64 n, uint64_t* lo_out,
+__global__ __launch_bounds__(BLOCK) void k_crit_split(CodeArray code, i64 n, uint64_t* lo_out,
                                                       uint32_t* hi_out) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= n) return;
     uint64_t lo, ilo;
     uint32_t hi, ihi;
-    code_masks(code[v], lo, hi, ilo, ihi);
+    code_masks(code_at(code, v), lo, hi, ilo, ihi);
     if (lo_out) lo_out[v] = lo & ilo;
     if (hi_out) hi_out[v] = hi & ihi;
 }
@@ -81,14 +81,14 @@ int dmtz_classify_noalloc_f32(dmtz_ctx* ctx, const float* d_field, int64_t nx, i
         ctx->err = "scratch of dmtz_classify_noalloc_f32 is not set up on this device";
         return DMTZ_E_HIP;
     }
-    StarCode* code = (StarCode*)base;
+    const CodeArray code{(uint64_t*)base, N};
     ull* ctr = (ull*)((unsigned char*)base + NOALLOC_CODE_BYTES);
     Dims d{nx, ny, nz};
     Counts c = make_counts(d);
     hipStream_t s = ctx->stream;
     k_clear_counters<<<1, 64, 0, s>>>(ctr);
     CK(hipGetLastError());
-    k_code<float><<<nblocks(N), BLOCK, 0, s>>>(d_field, d, c, code, nullptr);
+    k_code<float><<<nblocks(N), BLOCK, 0, s>>>(d_field, d, c, code, MaskArray{nullptr, nullptr});
     CK(hipGetLastError());
     k_crit_count<<<nblocks(N), BLOCK, 0, s>>>(code, N, ctr);
     CK(hipGetLastError());

@@ -50,6 +50,7 @@
 #include "pairs.h"
 #include "repair.h"
 #include "rules.h"
+#include "star_planes.h"
 
 using namespace dmtz;
 typedef unsigned long long ull;
@@ -232,31 +233,43 @@ __device__ __forceinline__ void block_emit(i64 base, const uint64_t (&lo)[EMIT_V
 // Star codes of every vertex (dense) or of the listed vertices.
 // 75-bit mask over the local cells of a vertex: the f-critical status of every local cell
 // (mismatch.h: local_crit), or the mismatched cells a vertex owns in g.
-struct __align__(16) CritMask {
+struct CritMask {
     uint64_t lo;
-    uint32_t hi, pad;
+    uint32_t hi;
 };
+// Masks of all vertices, the two parts apart so that dense passes write full lines.
+struct MaskArray {
+    uint64_t* lo;
+    uint32_t* hi;
+    __device__ __forceinline__ CritMask get(i64 v) const { return CritMask{lo[v], hi[v]}; }
+    __device__ __forceinline__ void put(i64 v, const CritMask& m) const {
+        lo[v] = m.lo;
+        hi[v] = m.hi;
+    }
+};
+constexpr double MASK_BYTES = sizeof(uint64_t) + sizeof(uint32_t);
 
 // The lower-star classification is fully unrolled straight-line code of about 5k instructions
 // needing about 100 VGPRs (lower_star.h keeps its live state small). CODE_BLOCKS_PER_CU = 4 caps
 // the code kernels at 128 VGPRs: four waves per SIMD to hide the loads of the star values.
 constexpr int CODE_BLOCKS_PER_CU = 4;
 
-// own (nullable) receives the critical cells each vertex owns, from the lower star itself (the
+// own (lo nullable) receives the critical cells each vertex owns, from the lower star itself (the
 // first pass of the f-critical masks, without reading the codes back).
 template <class T>
-__global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code(const T* fld, Dims d, Counts c, StarCode* code,
-                                                                    CritMask* own) {
+__global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code(const T* fld, Dims d, Counts c, CodeArray code,
+                                                                    MaskArray own) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= c.N) return;
     LowerStar ls;
     star_of(fld, d, v, ls);
-    encode_star(ls, code[v]);
-    if (own) {
+    StarCode sc;
+    encode_star(ls, sc);
+    code_put(code, v, sc);
+    if (own.lo) {
         CritMask m;
         crit_mask(ls, m.lo, m.hi);
-        m.pad = 0;
-        own[v] = m;
+        own.put(v, m);
     }
 }
 
@@ -264,15 +277,15 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code(const T* fld
 // g differs from f's (owner_mismatch, main_3d.cu:2492-2550). Returns whether the code changed.
 // nz_old / nz_new (nullable) receive whether the mask was nonzero before and after.
 template <class T>
-__device__ __forceinline__ bool code_g_at(const T* g, Dims d, i64 v, StarCode* code, const CritMask* crit_f,
-                                          CritMask* mm, bool* nz_old = nullptr, bool* nz_new = nullptr) {
+__device__ __forceinline__ bool code_g_at(const T* g, Dims d, i64 v, CodeArray code, MaskArray crit_f,
+                                          MaskArray mm, bool* nz_old = nullptr, bool* nz_new = nullptr) {
     LowerStar ls;
     star_of(g, d, v, ls);
     StarCode sc;
     encode_star(ls, sc);
-    const StarCode old = code[v];
-    code[v] = sc;
-    const CritMask cf = crit_f[v];
+    const StarCode old = code_at(code, v);
+    code_put(code, v, sc);
+    const CritMask cf = crit_f.get(v);
     uint64_t c_lo, i_lo;  // owner_mismatch of sc, from the lower star's own masks
     uint32_t c_hi, i_hi;
     crit_mask(ls, c_lo, c_hi);
@@ -280,13 +293,12 @@ __device__ __forceinline__ bool code_g_at(const T* g, Dims d, i64 v, StarCode* c
     CritMask m;
     m.lo = (c_lo ^ cf.lo) & i_lo;
     m.hi = (c_hi ^ cf.hi) & i_hi;
-    m.pad = 0;
     if (nz_old) {
-        const CritMask o = mm[v];
+        const CritMask o = mm.get(v);
         *nz_old = (o.lo | (uint64_t)o.hi) != 0;
     }
     if (nz_new) *nz_new = (m.lo | (uint64_t)m.hi) != 0;
-    mm[v] = m;
+    mm.put(v, m);
     return ((old.w[0] ^ sc.w[0]) | (old.w[1] ^ sc.w[1]) | (old.w[2] ^ sc.w[2]) | (old.w[3] ^ sc.w[3])) != 0;
 }
 
@@ -310,8 +322,8 @@ __device__ __forceinline__ void mark_vertex(Dims d, uint32_t v, uint32_t* marks)
 // Dense re-evaluation; tile_nz (zeroed before) receives, per EMIT_TILE vertices, the number with
 // a nonzero mismatch mask (a wave's 64 vertices lie in one tile).
 template <class T>
-__global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_g(const T* g, Dims d, Counts c, StarCode* code,
-                                                  const CritMask* crit_f, CritMask* mm, uint32_t* tile_nz) {
+__global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_g(const T* g, Dims d, Counts c, CodeArray code,
+                                                  MaskArray crit_f, MaskArray mm, uint32_t* tile_nz) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     bool nz = false;
     if (v < c.N) code_g_at(g, d, v, code, crit_f, mm, nullptr, &nz);
@@ -325,8 +337,8 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_g(const T* g
 // whose code changed is marked for the path checks (their results read nothing but star codes).
 // tile_nz follows the masks whose nonzero-ness changes.
 template <class T>
-__global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const T* g, Dims d, StarCode* code,
-                                                                         const CritMask* crit_f, CritMask* mm,
+__global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const T* g, Dims d, CodeArray code,
+                                                                         MaskArray crit_f, MaskArray mm,
                                                                          const uint32_t* list, const ull* n_ptr,
                                                                          ull* stars, uint32_t* marks,
                                                                          uint32_t* tile_nz) {
@@ -341,32 +353,180 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const
     }
 }
 
+// The dense classifications over bit planes (star_planes.h): a wave takes PLANE_TILE consecutive
+// vertices, lane l and bit 31 - b the vertex base + 64 b + l, so that a row of a tile is 64
+// consecutive vertices, read and written coalesced. About 23 thousand instructions per tile, a third of
+// them comparisons; the words of the passes take all 512 registers, so one wave runs per SIMD and
+// the instruction issue of that wave is the bound. 512^3 float32: 15.2 ms with a thread per vertex,
+// now 4.6 (the bytes alone take about 1.5 ms); 256^3: 1.99 -> 0.61 ms. With 256 registers and two waves
+// the spills cost more than the second wave gives (15 ms). Codes and masks are stored word by word
+// (CodeArray, MaskArray): as 32-byte structs, whose words leave a tile at different times, the lines
+// were written to memory several times over (23.5 GB instead of 6.4 at 512^3, 10.7 ms).
+constexpr int PLANE_ROWS = 32;
+constexpr i64 PLANE_TILE = 64 * PLANE_ROWS;
+static_assert(PLANE_TILE == EMIT_TILE, "a wave's count of nonzero masks is its tile's");
+
+// 64 vertices further in coordinates: at most one carry per axis.
+struct Step64 {
+    int x, y, z;
+    explicit Step64(const Dims& d)
+        : x((int)(64 % d.W)), y((int)(64 / d.W % d.H)), z((int)(64 / (d.W * d.H))) {}
+};
+
+// The comparison words of a wave's tile. The next row's values are loaded while a row is compared;
+// a neighbour's index is only kept inside the field, since finish() drops the slots outside the grid.
+template <class T>
+__device__ __forceinline__ void tile_words(const T* fld, const Dims& d, const Step64& st, i64 n, i64 v0, StarWords& w) {
+    const int W = (int)d.W, H = (int)d.H, D = (int)d.D, last = (int)(n - 1);
+    i64 x64, y64, z64;
+    vxyz(d, v0 <= last ? v0 : last, x64, y64, z64);
+    int x = (int)x64, y = (int)y64, z = (int)z64;
+    uint32_t v = (uint32_t)v0;  // v0 < n + PLANE_TILE < 2^32
+    int32_t off[14];
+#pragma unroll
+    for (int k = 0; k < 14; k++) off[k] = (int32_t)slot_step(d, k);
+    uint32_t side[6] = {0, 0, 0, 0, 0, 0};
+    auto load = [&](T* val) {
+        const uint32_t u = v < (uint32_t)last ? v : (uint32_t)last;
+#pragma unroll
+        for (int k = 0; k < 14; k++) {
+            uint32_t q;
+            if (k & 1) {  // odd slots lead down
+                const int t = (int)u + off[k];
+                q = t < 0 ? 0u : (uint32_t)t;
+            } else {
+                const uint32_t t = u + (uint32_t)off[k];
+                q = t < (uint32_t)last ? t : (uint32_t)last;
+            }
+            val[k] = fld[q];
+        }
+        val[14] = fld[u];
+        v += 64;
+    };
+    auto sides = [&]() {
+        side[0] = (side[0] << 1) | (uint32_t)(x > 0);
+        side[1] = (side[1] << 1) | (uint32_t)(x < W - 1);
+        side[2] = (side[2] << 1) | (uint32_t)(y > 0);
+        side[3] = (side[3] << 1) | (uint32_t)(y < H - 1);
+        side[4] = (side[4] << 1) | (uint32_t)(z > 0);
+        side[5] = (side[5] << 1) | (uint32_t)(z < D - 1);
+        x += st.x;
+        const int cx = x >= W;
+        x -= cx ? W : 0;
+        y += st.y + cx;
+        const int cy = y >= H;
+        y -= cy ? H : 0;
+        z += st.z + cy;
+    };
+#pragma unroll
+    for (int k = 0; k < N_PAIRS; k++) w.p[k] = 0;
+#pragma unroll
+    for (int k = 0; k < 14; k++) w.l[k] = 0;
+    T cur[15], nxt[15];
+    load(cur);
+#pragma unroll 1
+    for (int b = 0; b < PLANE_ROWS; b++) {
+        load(nxt);  // past the last row: not used
+        sides();
+        add_vertex(cur, w);
+#pragma unroll
+        for (int k = 0; k < 15; k++) cur[k] = nxt[k];
+    }
+    finish(w, side);
+}
+
+// Stores of a tile: codes, and per vertex its owned critical cells (crit_f null) or the mismatch
+// with f's critical cells.
+struct TileOut {
+    i64 v0, n;
+    CodeArray codes;
+    MaskArray mask;    // lo nullable
+    MaskArray crit_f;  // lo null: mask receives the owned critical cells
+    bool full;         // the whole tile lies in the field (wave-uniform)
+    uint32_t nz;       // bit r: the vertex of bit r has a nonzero mismatch mask
+
+    __device__ __forceinline__ i64 vertex(int r) const { return v0 + 64 * (PLANE_ROWS - 1 - r); }
+    template <class Fn>
+    __device__ __forceinline__ void rows(Fn fn) const {
+        if (full) {
+#pragma unroll
+            for (int r = 0; r < 32; r++) fn(r, vertex(r));
+        } else {
+#pragma unroll
+            for (int r = 0; r < 32; r++)
+                if (vertex(r) < n) fn(r, vertex(r));
+        }
+    }
+    __device__ __forceinline__ void code(int k, const uint32_t* lo, const uint32_t* hi) const {
+        uint64_t* const w = codes.w + k * codes.n;
+        rows([&](int r, i64 v) { *reinterpret_cast<uint2*>(w + v) = make_uint2(lo[r], hi[r]); });
+    }
+    __device__ __forceinline__ void masks_lo(uint32_t* c0, uint32_t* c1, const uint32_t* i0, const uint32_t* i1) {
+        if (!mask.lo) return;
+        if (crit_f.lo) {
+            uint32_t x = 0;
+            rows([&](int r, i64 v) {
+                const uint2 cf = *reinterpret_cast<const uint2*>(crit_f.lo + v);
+                c0[r] ^= cf.x & i0[r];
+                c1[r] ^= cf.y & i1[r];
+                x |= (uint32_t)((c0[r] | c1[r]) != 0u) << r;
+            });
+            nz |= x;
+        }
+        rows([&](int r, i64 v) { *reinterpret_cast<uint2*>(mask.lo + v) = make_uint2(c0[r], c1[r]); });
+    }
+    __device__ __forceinline__ void masks_hi(uint32_t* c2, const uint32_t* i2) {
+        if (!mask.lo) return;
+        if (crit_f.lo) {
+            uint32_t x = 0;
+            rows([&](int r, i64 v) {
+                c2[r] ^= crit_f.hi[v] & i2[r];
+                x |= (uint32_t)(c2[r] != 0u) << r;
+            });
+            nz |= x;
+        }
+        rows([&](int r, i64 v) { mask.hi[v] = c2[r]; });
+    }
+};
+
+// k_code and k_code_g (crit_f.lo and tile_nz not null) over bit planes.
+template <class T>
+__global__ __launch_bounds__(64, 1) void k_code_planes(const T* fld, Dims d, Step64 st, i64 n, CodeArray code,
+                                                       MaskArray mask, MaskArray crit_f, uint32_t* tile_nz) {
+    const i64 v0 = (i64)blockIdx.x * PLANE_TILE + threadIdx.x;
+    StarWords w;
+    tile_words(fld, d, st, n, v0, w);
+    TileOut out{v0, n, code, mask, crit_f, ((i64)blockIdx.x + 1) * PLANE_TILE <= n, 0u};
+    classify_words(w, out);
+    if (tile_nz) {
+        int cnt = __popc(out.nz);
+        for (int o = 32; o > 0; o >>= 1) cnt += __shfl_down(cnt, o, 64);
+        if (threadIdx.x == 0) tile_nz[blockIdx.x] = (uint32_t)cnt;
+    }
+}
+
 // f-critical status of the local cells of every vertex (once per run), in two passes: each
 // vertex writes the critical cells it owns (k_code's own output, or k_critf_own from the codes),
 // then gathers the ones its 14 neighbours own that contain it (k_critf_gather: 15 coalesced
 // 16-byte reads and one store per vertex; the reverse, each owner spreading its cells with
 // atomics, wrote five times the masks' size to memory and took twice as long).
-__global__ __launch_bounds__(BLOCK) void k_critf_own(const StarCode* cf, i64 n, CritMask* out) {
+__global__ __launch_bounds__(BLOCK) void k_critf_own(CodeArray cf, i64 n, MaskArray out) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= n) return;
     uint64_t lo, ilo;
     uint32_t hi, ihi;
-    code_masks(cf[v], lo, hi, ilo, ihi);
-    CritMask m;
-    m.lo = lo & ilo;
-    m.hi = hi & ihi;
-    m.pad = 0;
-    out[v] = m;
+    code_masks(code_at(cf, v), lo, hi, ilo, ihi);
+    out.put(v, CritMask{lo & ilo, hi & ihi});
 }
 
 // Critical cells per type (vertex, edge, triangle, tet) over all owners: one atomic per wave and type.
-__global__ __launch_bounds__(BLOCK) void k_crit_count(const StarCode* code, i64 n, ull* ctr) {
+__global__ __launch_bounds__(BLOCK) void k_crit_count(CodeArray code, i64 n, ull* ctr) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     int cnt[4] = {0, 0, 0, 0};
     if (v < n) {
         uint64_t lo, ilo;
         uint32_t hi, ihi;
-        code_masks(code[v], lo, hi, ilo, ihi);
+        code_masks(code_at(code, v), lo, hi, ilo, ihi);
         lo &= ilo;
         hi &= ihi;
         cnt[0] = (int)(lo & 1ull);
@@ -382,7 +542,7 @@ __global__ __launch_bounds__(BLOCK) void k_crit_count(const StarCode* code, i64 
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_critf_gather(const CritMask* own, Dims d, i64 n, CritMask* out) {
+__global__ __launch_bounds__(BLOCK) void k_critf_gather(MaskArray own, Dims d, i64 n, MaskArray out) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= n) return;
     uint64_t lo;
@@ -390,16 +550,12 @@ __global__ __launch_bounds__(BLOCK) void k_critf_gather(const CritMask* own, Dim
     crit_gather(
         d, v,
         [&](i64 u, uint64_t& a, uint32_t& b) {
-            const CritMask m = own[u];
+            const CritMask m = own.get(u);
             a = m.lo;
             b = m.hi;
         },
         lo, hi);
-    CritMask m;
-    m.lo = lo;
-    m.hi = hi;
-    m.pad = 0;
-    out[v] = m;
+    out.put(v, CritMask{lo, hi});
 }
 
 // Dense mismatch detection: every vertex lists the mismatched cells it owns in g, from the
@@ -412,7 +568,7 @@ __global__ __launch_bounds__(BLOCK) void k_critf_gather(const CritMask* own, Dim
 // per tile of the grid.
 constexpr unsigned DETECT_BLOCKS = 2048;
 
-__global__ __launch_bounds__(BLOCK) void k_detect(const CritMask* mm, i64 n, const uint32_t* tile_nz, Lists4 out,
+__global__ __launch_bounds__(BLOCK) void k_detect(MaskArray mm, i64 n, const uint32_t* tile_nz, Lists4 out,
                                                   ull* ctr, ull* tiles_read) {
     __shared__ uint64_t nz_mask;
     const i64 ntiles = (n + EMIT_TILE - 1) / EMIT_TILE, stride = (i64)gridDim.x;
@@ -439,7 +595,7 @@ __global__ __launch_bounds__(BLOCK) void k_detect(const CritMask* mm, i64 n, con
                 lo[k] = 0;
                 hi[k] = 0;
                 if (v < n) {
-                    const CritMask m = mm[v];
+                    const CritMask m = mm.get(v);
                     lo[k] = m.lo;
                     hi[k] = m.hi;
                 }
@@ -450,9 +606,9 @@ __global__ __launch_bounds__(BLOCK) void k_detect(const CritMask* mm, i64 n, con
 }
 
 // Critical cells owned by each vertex, from the masks of owned critical cells (own, as k_code leaves
-// them) or, when own is null, from the star codes; type_mask selects which types count, and a
+// them) or, when own.lo is null, from the star codes; type_mask selects which types count, and a
 // type whose list is null is counted but not listed.
-__global__ __launch_bounds__(BLOCK) void k_fcrit(const CritMask* own, const StarCode* cf, Counts c, Lists4 out,
+__global__ __launch_bounds__(BLOCK) void k_fcrit(MaskArray own, CodeArray cf, Counts c, Lists4 out,
                                                  ull* ctr, int type_mask) {
     const i64 base = (i64)blockIdx.x * EMIT_TILE;
     uint64_t keep = 0;
@@ -467,14 +623,14 @@ __global__ __launch_bounds__(BLOCK) void k_fcrit(const CritMask* own, const Star
         lo[k] = 0;
         hi[k] = 0;
         if (v < c.N) {
-            if (own) {
-                const CritMask m = own[v];
+            if (own.lo) {
+                const CritMask m = own.get(v);
                 lo[k] = m.lo;
                 hi[k] = m.hi;
             } else {
                 uint64_t ilo;
                 uint32_t ihi;
-                code_masks(cf[v], lo[k], hi[k], ilo, ihi);
+                code_masks(code_at(cf, v), lo[k], hi[k], ilo, ihi);
             }
             lo[k] &= keep;
             if (!(type_mask & 8)) hi[k] = 0;
@@ -553,8 +709,8 @@ struct HoldSink {
 // every branch body with thousands of instructions, the records were grouped by branch first; with
 // these rules the grouping costs 512^3 fBm 19 ms of 195 and 256^3 mixtures 13 of 122.)
 template <class T, int TYPE>
-__global__ __launch_bounds__(BLOCK) void k_fix_cp(const uint64_t* recs, ull n, const T* f, const StarCode* cf,
-                                                  const T* g, const StarCode* cg, Dims d, Counts c,
+__global__ __launch_bounds__(BLOCK) void k_fix_cp(const uint64_t* recs, ull n, const T* f, CodeArray cf,
+                                                  const T* g, CodeArray cg, Dims d, Counts c,
                                                   const uint8_t* counter, double eps, double range, int edit_type,
                                                   TargetSink sink) {
     __shared__ RuleTables tb;
@@ -569,9 +725,9 @@ __global__ __launch_bounds__(BLOCK) void k_fix_cp(const uint64_t* recs, ull n, c
         const uint64_t r = recs[i];
         const uint32_t v = (uint32_t)(r >> 7);
         const int lc = (int)(r & 127u);
-        LocalRules<T, HoldSink> L{f, cf, g, cg, counter, &tb, off, d, c, eps, edit_type, hold};
+        LocalRules<T, HoldSink, CodeArray> L{f, cf, g, cg, counter, &tb, off, d, c, eps, edit_type, hold};
         if (__builtin_expect(!L.template run<TYPE>(v, lc), 0)) {
-            Repair<T, HoldSink> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, hold);
+            Repair<T, HoldSink, CodeArray> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, hold);
             const i64 id = local_cell_id(d, c, (i64)v, lc);
             if (TYPE == 1) R.fix_saddle(id);
             else if (TYPE == 2) R.fix_2saddle(id);
@@ -912,7 +1068,7 @@ struct NoSink {
 // Pair words (pairs.h) of every vertex of a field. Bound by the reads of the values and of the
 // codes' first two words (the whole 32-byte codes, as lines go).
 template <class T>
-__global__ __launch_bounds__(BLOCK) void k_pairs(const T* fld, const StarCode* code, Dims d, i64 n, uint32_t* out) {
+__global__ __launch_bounds__(BLOCK) void k_pairs(const T* fld, CodeArray code, Dims d, i64 n, uint32_t* out) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= n) return;
     i64 x, y, z;
@@ -923,7 +1079,7 @@ __global__ __launch_bounds__(BLOCK) void k_pairs(const T* fld, const StarCode* c
 // Where the pairings of f and g differ (pairs.h pair_mismatch), one byte per vertex, for every
 // vertex. pg (nullable) receives g's pair words.
 template <class T>
-__global__ __launch_bounds__(BLOCK) void k_mism_full(const T* g, const StarCode* code, const uint32_t* pf, Dims d,
+__global__ __launch_bounds__(BLOCK) void k_mism_full(const T* g, CodeArray code, const uint32_t* pf, Dims d,
                                                      i64 n, uint8_t* mis, uint32_t* pg) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v >= n) return;
@@ -940,7 +1096,7 @@ __global__ __launch_bounds__(BLOCK) void k_mism_full(const T* g, const StarCode*
 // 32 * BLOCK vertices, clears them, lists the marked vertices in LDS and spreads them over its
 // threads, so that a few marks cost a pass over the bitmap (N / 8 bytes).
 template <class T>
-__global__ __launch_bounds__(BLOCK) void k_mism_marked(const T* g, const StarCode* code, const uint32_t* pf, Dims d,
+__global__ __launch_bounds__(BLOCK) void k_mism_marked(const T* g, CodeArray code, const uint32_t* pf, Dims d,
                                                        i64 n, uint32_t* marks, uint8_t* mis) {
     __shared__ uint16_t list[32 * BLOCK];
     __shared__ int wsum[BLOCK / 64];
@@ -987,7 +1143,7 @@ __device__ __forceinline__ void load_slot_steps(const Dims& d, i64* step) {
 // A thread tests 16 vertices with one load, so an edge costs nothing unless an end differs (the
 // pass reads N bytes; 512^3 fBm, 11 checks: 5.8 ms with a thread and 36 bytes per edge -> 1.4 ms).
 constexpr int DS_V = 16;
-__global__ __launch_bounds__(BLOCK) void k_ds_list(const uint8_t* mis, const CritMask* critf, Dims d, Counts c, i64 n,
+__global__ __launch_bounds__(BLOCK) void k_ds_list(const uint8_t* mis, const uint64_t* critf, Dims d, Counts c, i64 n,
                                                    PathList out) {
     __shared__ i64 step[16];
     load_slot_steps(d, step);
@@ -1002,7 +1158,7 @@ __global__ __launch_bounds__(BLOCK) void k_ds_list(const uint8_t* mis, const Cri
     }
     // f-critical edges of vertex v that v records
     auto edges = [&](i64 v) {
-        uint32_t e = (uint32_t)(critf[v].lo >> LC_EDGE) & 0x3FFFu;
+        uint32_t e = (uint32_t)(critf[v] >> LC_EDGE) & 0x3FFFu;
         for (uint32_t up = e & 0x1555u; up; up &= up - 1) {  // even slots lead to larger indices
             const int s = __builtin_ctz(up);
             if (mis[v + step[s]] & MIS_SLOT) e &= ~(1u << s);
@@ -1237,7 +1393,7 @@ __global__ __launch_bounds__(BLOCK) void k_as_list(ull nf, const uint32_t* off, 
 // res[2*j+1] = the divergent tet. A chain of dependent 4-byte reads (129 x 96 x 111 mixture in
 // float64: 3.1 ms per check over star codes and ids, now 0.06).
 __global__ __launch_bounds__(BLOCK) void k_as_branch(const uint64_t* fcf, ull n, const int64_t* maxlab, int lab_from_f,
-                                                     const CritMask* critf, const uint32_t* pf, const uint32_t* pg,
+                                                     const uint64_t* critf, const uint32_t* pf, const uint32_t* pg,
                                                      Dims d, i64 cap, int64_t* res, ull* walk_ctr) {
     __shared__ uint8_t across[24];
     load_across(across);
@@ -1254,7 +1410,7 @@ __global__ __launch_bounds__(BLOCK) void k_as_branch(const uint64_t* fcf, ull n,
     bool check = a.v >= 0;
     if (check && maxlab) check = paired_max(d, pg, across, a, cap, ovf) != maxlab[j];
     if (check && lab_from_f) {
-        const bool fcrit = ((critf[v].lo >> lc) & 1ull) != 0;
+        const bool fcrit = ((critf[v] >> lc) & 1ull) != 0;
         const i64 lab = fcrit ? paired_max(d, pf, across, a, cap, ovf) : -1;
         check = paired_max(d, pg, across, a, cap, ovf) != lab;
     }
@@ -1356,7 +1512,7 @@ __global__ __launch_bounds__(BLOCK) void k_ds_combine(const uint64_t* fce, ull n
 // outgrows its set is listed in ovf, to be walked again with more slots.
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_ds_wall(const uint64_t* starts, const uint32_t* sel, ull first, ull n,
-                                                   const T* f, const StarCode* cf, const T* g, const StarCode* cg,
+                                                   const T* f, CodeArray cf, const T* g, CodeArray cg,
                                                    Dims d, Counts c, uint32_t* scratch, uint32_t slots, PathList out,
                                                    uint32_t* ovf, ull* ovf_ctr) {
     const ull t = (ull)blockIdx.x * BLOCK + threadIdx.x;
@@ -1364,7 +1520,7 @@ __global__ __launch_bounds__(BLOCK) void k_ds_wall(const uint64_t* starts, const
     const ull s = sel ? (ull)sel[first + t] : first + t;
     const uint64_t r = starts[s];
     const i64 face = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-    Repair<T, NoSink> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NoSink{});
+    Repair<T, NoSink, CodeArray> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NoSink{});
     uint32_t* set = scratch + (size_t)t * (2 * (size_t)slots + 2);
     i64 found = -1;
     const bool overflow = R.wall_walk(face, set, set + slots, slots, found);
@@ -1383,11 +1539,11 @@ __global__ __launch_bounds__(BLOCK) void k_ds_wall(const uint64_t* starts, const
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_fix_paths(const int64_t* as_rec, ull n_as, const int64_t* ds_rec, ull n_ds,
                                                      const int64_t* wall_rec, ull n_wall, const T* f,
-                                                     const StarCode* cf, const T* g, const StarCode* cg, Dims d,
+                                                     CodeArray cf, const T* g, CodeArray cg, Dims d,
                                                      Counts c, const uint8_t* counter, double eps, double range,
                                                      int edit_type, TargetSink sink) {
     const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
-    Repair<T, HoldSink> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, HoldSink{sink, 0u, 0u, 0u, 0u, 0});
+    Repair<T, HoldSink, CodeArray> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, HoldSink{sink, 0u, 0u, 0u, 0u, 0});
     if (i < n_as) R.fix_as_vpath(as_rec[i]);
     else if (i < n_as + n_ds) R.fix_ds_vpath(ds_rec[i - n_as]);
     else if (i < n_as + n_ds + n_wall) R.fix_ds_wall(wall_rec[i - n_as - n_ds]);
@@ -1396,11 +1552,11 @@ __global__ __launch_bounds__(BLOCK) void k_fix_paths(const int64_t* as_rec, ull 
 
 // Dense pairing arrays for tests (dmtz_gradient_*): one thread per cell of each dimension.
 template <class T>
-__global__ __launch_bounds__(BLOCK) void k_pairing(const T* fld, const StarCode* code, Dims d, Counts c, int dim, ull n,
+__global__ __launch_bounds__(BLOCK) void k_pairing(const T* fld, CodeArray code, Dims d, Counts c, int dim, ull n,
                                                    int64_t* out) {
     const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
-    FieldGrad<T> X(fld, code, d, c);
+    FieldGrad<T, CodeArray> X(fld, code, d, c);
     switch (dim) {
         case 0: out[i] = X.pv((i64)i); break;
         case 1: out[i] = X.pe((i64)i); break;
@@ -1444,10 +1600,10 @@ struct dmtz_ctx {
     uint32_t* d_targets = nullptr;  // edit set
     uint32_t* d_changed = nullptr;  // edited vertices whose value changed
     uint32_t* d_dirty = nullptr;    // vertices whose g star code must be re-evaluated
-    StarCode* d_code_f = nullptr;   // star codes of f and g
-    StarCode* d_code_g = nullptr;
-    CritMask* d_critf = nullptr;    // f-critical status of every vertex's local cells
-    CritMask* d_mm = nullptr;       // mismatched cells each vertex owns in g
+    uint64_t* d_code_f = nullptr;   // star codes of f and g, word by word (CodeArray)
+    uint64_t* d_code_g = nullptr;
+    MaskArray d_critf = {nullptr, nullptr};  // f-critical status of every vertex's local cells
+    MaskArray d_mm = {nullptr, nullptr};     // mismatched cells each vertex owns in g
     uint32_t* d_tile_nz = nullptr;  // per EMIT_TILE vertices: how many have a nonzero d_mm
     uint64_t* d_rec = nullptr;    // 4 mismatch record lists of rec_cap entries
     uint64_t* d_fc = nullptr;     // 4 f-critical lists of fc_cap entries
@@ -1506,15 +1662,17 @@ void free_bufs(dmtz_ctx* ctx) {
     (void)hipFree(ctx->d_dirty);
     (void)hipFree(ctx->d_code_f);
     (void)hipFree(ctx->d_code_g);
-    (void)hipFree(ctx->d_critf);
-    (void)hipFree(ctx->d_mm);
+    for (MaskArray* m : {&ctx->d_critf, &ctx->d_mm}) {
+        (void)hipFree(m->lo);
+        (void)hipFree(m->hi);
+        *m = MaskArray{nullptr, nullptr};
+    }
     (void)hipFree(ctx->d_tile_nz);
     ctx->d_tile_nz = nullptr;
     ctx->d_f = ctx->d_g = nullptr;
     ctx->d_counter = nullptr;
     ctx->d_stamp = ctx->d_dstamp = ctx->d_targets = ctx->d_changed = ctx->d_dirty = nullptr;
     ctx->d_code_f = ctx->d_code_g = nullptr;
-    ctx->d_critf = ctx->d_mm = nullptr;
     ctx->field_bytes = 0;
     ctx->cap_n = 0;
 }
@@ -1582,8 +1740,10 @@ int ensure(dmtz_ctx* ctx, i64 N, size_t elem, bool want_fields) {
         CK(hipMalloc(&ctx->d_dirty, sizeof(uint32_t) * n));
         CK(hipMalloc(&ctx->d_code_f, sizeof(StarCode) * n));
         CK(hipMalloc(&ctx->d_code_g, sizeof(StarCode) * n));
-        CK(hipMalloc(&ctx->d_critf, sizeof(CritMask) * n));
-        CK(hipMalloc(&ctx->d_mm, sizeof(CritMask) * n));
+        for (MaskArray* m : {&ctx->d_critf, &ctx->d_mm}) {
+            CK(hipMalloc(&m->lo, sizeof(uint64_t) * n));
+            CK(hipMalloc(&m->hi, sizeof(uint32_t) * n));
+        }
         CK(hipMalloc(&ctx->d_tile_nz, sizeof(uint32_t) * (n / EMIT_TILE + 2)));
         ctx->cap_n = N;
         ctx->epoch = 0;
@@ -1701,6 +1861,9 @@ struct Driver {
     double eps, range;
     dmtz_flags fl;
 
+    CodeArray cf() const { return CodeArray{ctx->d_code_f, c.N}; }
+    CodeArray cg() const { return CodeArray{ctx->d_code_g, c.N}; }
+
     // Detection of the four critical-cell mismatch kinds into the record lists.
     int detect() {
         if (ctx->rec_cap == 0) {
@@ -1737,7 +1900,7 @@ struct Driver {
         ull m = ctx->h_ctr[0] + ctx->h_ctr[1] + ctx->h_ctr[2] + ctx->h_ctr[3];
         ctx->det_launches += 1;
         ctx->det_ms += ms;
-        ctx->det_bytes += 4.0 * (double)ntiles + (double)ctx->h_ctr[K_DTILES] * (double)EMIT_TILE * sizeof(CritMask) +
+        ctx->det_bytes += 4.0 * (double)ntiles + (double)ctx->h_ctr[K_DTILES] * (double)EMIT_TILE * MASK_BYTES +
                           8.0 * (double)m;
         ctx->det_voxels += (double)c.N;
         return 0;
@@ -1814,7 +1977,7 @@ struct Driver {
             if (!active[ty]) continue;
             hipStream_t st = side && (ty == 1 || ty == 3) ? ctx->fix_stream : ctx->stream;
             auto kern = ty == 0 ? k_fix_cp<T, 0> : ty == 1 ? k_fix_cp<T, 1> : ty == 2 ? k_fix_cp<T, 2> : k_fix_cp<T, 3>;
-            kern<<<nblocks(counts[ty]), BLOCK, 0, st>>>(L.l[ty], counts[ty], f, ctx->d_code_f, g, ctx->d_code_g, d,
+            kern<<<nblocks(counts[ty]), BLOCK, 0, st>>>(L.l[ty], counts[ty], f, cf(), g, cg(), d,
                                                         c, ctx->d_counter, eps, range, fl.edit_type, sink());
             CK(hipGetLastError());
         }
@@ -1876,7 +2039,7 @@ struct Driver {
         }
         CK(hipGetLastError());
         k_code_list_g<T><<<stride_blocks(15 * est), BLOCK, 0, ctx->stream>>>(
-            g, d, ctx->d_code_g, ctx->d_critf, ctx->d_mm, ctx->d_dirty, ctx->d_ctr + K_DIRTY, ctx->d_ctr + K_STARS,
+            g, d, cg(), ctx->d_critf, ctx->d_mm, ctx->d_dirty, ctx->d_ctr + K_DIRTY, ctx->d_ctr + K_STARS,
             as_ready ? ctx->d_marks : nullptr, ctx->d_tile_nz);
         CK(hipGetLastError());
         return 0;
@@ -1958,7 +2121,7 @@ struct Driver {
     // f, main_3d.cu:6539-6564, done once per run).
     int f_codes() {
         // the owned critical cells go to the mismatch masks first, which the g codes overwrite next
-        int rc = codes(f, ctx->d_code_f, ctx->d_mm);
+        int rc = codes(f, cf(), ctx->d_mm);
         if (rc) return rc;
         k_critf_gather<<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(ctx->d_mm, d, c.N, ctx->d_critf);
         CK(hipGetLastError());
@@ -1968,16 +2131,33 @@ struct Driver {
     // g star codes and mismatch masks of every vertex (the g gradient, main_3d.cu:6624-6638);
     // needs the f-critical masks.
     int g_codes() {
+        if (c.N >= PLANE_MIN) {
+            k_code_planes<T><<<plane_blocks(), 64, 0, ctx->stream>>>(g, d, Step64(d), c.N, cg(), ctx->d_mm, ctx->d_critf,
+                                                                     ctx->d_tile_nz);
+            CK(hipGetLastError());
+            return 0;
+        }
         CK(hipMemsetAsync(ctx->d_tile_nz, 0, sizeof(uint32_t) * (size_t)((c.N + EMIT_TILE - 1) / EMIT_TILE),
                           ctx->stream));
-        k_code_g<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(g, d, c, ctx->d_code_g, ctx->d_critf, ctx->d_mm,
+        k_code_g<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(g, d, c, cg(), ctx->d_critf, ctx->d_mm,
                                                              ctx->d_tile_nz);
         CK(hipGetLastError());
         return 0;
     }
 
+    // Grids from here on classify over bit planes: below, a wave per 2048 vertices leaves most of the chip
+    // idle and its 55 us of work (float32; 80 in float64) is the time of the pass, against 0.12 us per
+    // thousand vertices with a thread per vertex (64^3: 47 us, 129 x 96 x 111 float64: 172).
+    static constexpr i64 PLANE_MIN = (i64)1 << 19;
+    unsigned plane_blocks() const { return (unsigned)((c.N + PLANE_TILE - 1) / PLANE_TILE); }
+
     // Star codes of every vertex of a field.
-    int codes(const T* fld, StarCode* out, CritMask* own = nullptr) {
+    int codes(const T* fld, CodeArray out, MaskArray own) {
+        if (c.N >= PLANE_MIN) {
+            k_code_planes<T><<<plane_blocks(), 64, 0, ctx->stream>>>(fld, d, Step64(d), c.N, out, own, MaskArray{nullptr, nullptr}, nullptr);
+            CK(hipGetLastError());
+            return 0;
+        }
         k_code<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(fld, d, c, out, own);
         CK(hipGetLastError());
         return 0;
@@ -2002,7 +2182,7 @@ struct Driver {
     // Critical cells of the types in type_mask into the f-critical lists (grown on demand), from the
     // star codes given or, with codes null, from f's owned critical cells, which lie in d_mm between
     // f_codes() and g_codes(). Types outside list_mask are counted but not listed.
-    int fcrit(const StarCode* codes, int type_mask, int list_mask = 15) {
+    int fcrit(const CodeArray* codes, int type_mask, int list_mask = 15) {
         if (ctx->fc_cap == 0) {
             int rc0 = grow_fc(ctx, (ull)(c.N / 16));
             if (rc0) return rc0;
@@ -2013,7 +2193,7 @@ struct Driver {
                 if (!((list_mask >> k) & 1)) FL.l[k] = nullptr;
             CK(hipMemsetAsync(ctx->d_ctr + K_FC0, 0, sizeof(ull) * 4, ctx->stream));
             k_fcrit<<<(unsigned)((c.N + EMIT_TILE - 1) / EMIT_TILE), BLOCK, 0, ctx->stream>>>(
-                codes ? nullptr : ctx->d_mm, codes, c, FL, ctx->d_ctr + K_FC0, type_mask);
+                codes ? MaskArray{nullptr, nullptr} : ctx->d_mm, codes ? *codes : cf(), c, FL, ctx->d_ctr + K_FC0, type_mask);
             CK(hipGetLastError());
             int rc = sync_ctr(ctx);
             if (rc) return rc;
@@ -2027,7 +2207,7 @@ struct Driver {
 
     // The start cells of the separatrix checks: f-critical faces, and edges (listed in connectivity
     // mode only: the geometry checks find them from the vertices). codes as for fcrit().
-    int prepare_paths(const StarCode* codes) {
+    int prepare_paths(const CodeArray* codes) {
         const bool conn = fl.preserve_geometry != 1;
         int rc = fcrit(codes, 2 | 4, conn ? 15 : 4);
         if (rc) return rc;
@@ -2035,7 +2215,7 @@ struct Driver {
         nfce = ctx->h_ctr[K_FC0 + 1];
         nfcf = ctx->h_ctr[K_FC0 + 2];
         if (conn) {
-            rc = pairs_of(f, ctx->d_code_f, ctx->d_pairf, ctx->pairf_cap, ctx->stream);
+            rc = pairs_of(f, cf(), ctx->d_pairf, ctx->pairf_cap, ctx->stream);
             if (rc) return rc;
         }
         if (conn && nfce + nfcf) {
@@ -2049,7 +2229,7 @@ struct Driver {
         return 0;
     }
 
-    int pairs_of(const T* fld, const StarCode* codes, uint32_t*& out, size_t& cap, hipStream_t st) {
+    int pairs_of(const T* fld, CodeArray codes, uint32_t*& out, size_t& cap, hipStream_t st) {
         int rc = grow_buf(ctx, out, cap, (size_t)c.N);
         if (rc) return rc;
         k_pairs<T><<<nblocks(c.N), BLOCK, 0, st>>>(fld, codes, d, c.N, out);
@@ -2076,7 +2256,7 @@ struct Driver {
         if (!n) return 0;
         int rc = grow_buf(ctx, ctx->d_walk, ctx->walk_cap, 4 * n);
         if (rc) return rc;
-        k_as_branch<<<nblocks(2 * n), BLOCK, 0, ctx->stream>>>(faces, n, lab, lab_from_f, ctx->d_critf, ctx->d_pairf,
+        k_as_branch<<<nblocks(2 * n), BLOCK, 0, ctx->stream>>>(faces, n, lab, lab_from_f, ctx->d_critf.lo, ctx->d_pairf,
                                                                ctx->d_pairg, d, c.N, ctx->d_walk, ctx->d_ctr + K_WALK);
         CK(hipGetLastError());
         k_as_combine<<<nblocks(n), BLOCK, 0, ctx->stream>>>(ctx->d_walk, n, path_list(1));
@@ -2085,7 +2265,7 @@ struct Driver {
     }
 
     int check_connectivity() {
-        int rc = pairs_of(g, ctx->d_code_g, ctx->d_pairg, ctx->pairg_cap, ctx->stream);
+        int rc = pairs_of(g, cg(), ctx->d_pairg, ctx->pairg_cap, ctx->stream);
         if (rc) return rc;
         Lists4 FL = fcrit_lists(ctx);
         rc = as_gfaces ? as_branches(as_gfaces, n_gfaces, nullptr, 1)
@@ -2112,10 +2292,10 @@ struct Driver {
                 if (rc) return rc;
             }
             CK(hipMemsetAsync(ctx->d_marks, 0, sizeof(uint32_t) * words, ctx->stream));
-            k_mism_full<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(g, ctx->d_code_g, ctx->d_pairf, d, c.N, ctx->d_mis,
+            k_mism_full<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(g, cg(), ctx->d_pairf, d, c.N, ctx->d_mis,
                                                                      as_listed ? nullptr : ctx->d_pairg);
         } else {
-            k_mism_marked<T><<<nblocks(words), BLOCK, 0, ctx->stream>>>(g, ctx->d_code_g, ctx->d_pairf, d, c.N,
+            k_mism_marked<T><<<nblocks(words), BLOCK, 0, ctx->stream>>>(g, cg(), ctx->d_pairf, d, c.N,
                                                                          ctx->d_marks, ctx->d_mis);
         }
         CK(hipGetLastError());
@@ -2134,7 +2314,7 @@ struct Driver {
             if (rc) return rc;
         }
         if (nfce) {
-            k_ds_list<<<nblocks((c.N + DS_V - 1) / DS_V), BLOCK, 0, ctx->stream>>>(ctx->d_mis, ctx->d_critf, d, c, c.N,
+            k_ds_list<<<nblocks((c.N + DS_V - 1) / DS_V), BLOCK, 0, ctx->stream>>>(ctx->d_mis, ctx->d_critf.lo, d, c, c.N,
                                                                                    path_list(0));
             CK(hipGetLastError());
         }
@@ -2170,7 +2350,7 @@ struct Driver {
             for (ull first = 0; first < n; first += chunk) {
                 const ull last = first + chunk < n ? first + chunk : n;
                 k_ds_wall<T><<<nblocks(last - first), BLOCK, 0, ctx->stream>>>(
-                    FL.l[2], sel, first, last, f, ctx->d_code_f, g, ctx->d_code_g, d, c, ctx->d_wall_scr, slots,
+                    FL.l[2], sel, first, last, f, cf(), g, cg(), d, c, ctx->d_wall_scr, slots,
                     path_list(2), ovf, ctx->d_ctr + K_WOVF);
                 CK(hipGetLastError());
             }
@@ -2268,7 +2448,7 @@ struct Driver {
     // number of steps lands in *h_as_total when st gets there.
     int as_count(hipStream_t st) {
         const size_t words = (size_t)(c.N + 31) / 32;
-        int rc = pairs_of(f, ctx->d_code_f, ctx->d_pairf, ctx->pairf_cap, st);
+        int rc = pairs_of(f, cf(), ctx->d_pairf, ctx->pairf_cap, st);
         if (rc) return rc;
         rc = grow_buf(ctx, ctx->d_mis, ctx->mis_cap, (size_t)c.N + DS_V);
         if (rc) return rc;
@@ -2326,8 +2506,8 @@ struct Driver {
         if (fl.preserve_connectors != 1) nw = 0;
         if (nds + nas + nw) {
             k_fix_paths<T><<<nblocks(nds + nas + nw), BLOCK, 0, ctx->stream>>>(
-                path_list(1).rec, nas, path_list(0).rec, nds, path_list(2).rec, nw, f, ctx->d_code_f, g,
-                ctx->d_code_g, d, c, ctx->d_counter, eps, range, fl.edit_type, sink());
+                path_list(1).rec, nas, path_list(0).rec, nds, path_list(2).rec, nw, f, cf(), g,
+                cg(), d, c, ctx->d_counter, eps, range, fl.edit_type, sink());
             CK(hipGetLastError());
         }
         return apply(nds + nas + nw);
@@ -2622,25 +2802,23 @@ int classify_host(dmtz_ctx* ctx, const T* fld, i64 nx, i64 ny, i64 nz, int64_t* 
     Dims d{nx, ny, nz};
     Counts c = make_counts(d);
     CK(hipMemcpyAsync(ctx->d_f, fld, sizeof(T) * (size_t)N, hipMemcpyHostToDevice, ctx->stream));
-    k_code<T><<<nblocks(N), BLOCK, 0, ctx->stream>>>((const T*)ctx->d_f, d, c, ctx->d_code_f, nullptr);
+    k_code<T><<<nblocks(N), BLOCK, 0, ctx->stream>>>((const T*)ctx->d_f, d, c, CodeArray{ctx->d_code_f, c.N},
+                                                   MaskArray{nullptr, nullptr});
     CK(hipGetLastError());
     CK(hipMemsetAsync(ctx->d_ctr, 0, sizeof(ull) * 4, ctx->stream));
-    k_crit_count<<<nblocks(N), BLOCK, 0, ctx->stream>>>(ctx->d_code_f, N, ctx->d_ctr);
+    k_crit_count<<<nblocks(N), BLOCK, 0, ctx->stream>>>(CodeArray{ctx->d_code_f, N}, N, ctx->d_ctr);
     CK(hipGetLastError());
     rc = sync_ctr(ctx);
     if (rc) return rc;
     for (int k = 0; k < 4; k++) counts4[k] = (int64_t)ctx->h_ctr[k];
     if (crit_lo || crit_hi) {
-        k_critf_own<<<nblocks(N), BLOCK, 0, ctx->stream>>>(ctx->d_code_f, N, ctx->d_critf);
+        k_critf_own<<<nblocks(N), BLOCK, 0, ctx->stream>>>(CodeArray{ctx->d_code_f, N}, N, ctx->d_critf);
         CK(hipGetLastError());
-        std::vector<CritMask> hm((size_t)N);
-        CK(hipMemcpyAsync(hm.data(), ctx->d_critf, sizeof(CritMask) * (size_t)N, hipMemcpyDeviceToHost,
-                          ctx->stream));
+        if (crit_lo)
+            CK(hipMemcpyAsync(crit_lo, ctx->d_critf.lo, sizeof(uint64_t) * (size_t)N, hipMemcpyDeviceToHost, ctx->stream));
+        if (crit_hi)
+            CK(hipMemcpyAsync(crit_hi, ctx->d_critf.hi, sizeof(uint32_t) * (size_t)N, hipMemcpyDeviceToHost, ctx->stream));
         CK(hipStreamSynchronize(ctx->stream));
-        for (i64 v = 0; v < N; v++) {
-            if (crit_lo) crit_lo[v] = hm[(size_t)v].lo;
-            if (crit_hi) crit_hi[v] = hm[(size_t)v].hi;
-        }
     }
     return 0;
 }
@@ -2742,7 +2920,8 @@ int gradient_host(dmtz_ctx* ctx, const T* fld, i64 nx, i64 ny, i64 nz, int64_t* 
     rc = ensure(ctx, c.N, sizeof(T), true);
     if (rc) return rc;
     CK(hipMemcpyAsync(ctx->d_f, fld, sizeof(T) * (size_t)c.N, hipMemcpyHostToDevice, ctx->stream));
-    k_code<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>((const T*)ctx->d_f, d, c, ctx->d_code_f, nullptr);
+    k_code<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>((const T*)ctx->d_f, d, c, CodeArray{ctx->d_code_f, c.N},
+                                                   MaskArray{nullptr, nullptr});
     CK(hipGetLastError());
     int64_t* outs[4] = {pv, pe, pf, pt};
     i64 sizes[4] = {c.N, c.E, c.F, c.T};
@@ -2750,7 +2929,7 @@ int gradient_host(dmtz_ctx* ctx, const T* fld, i64 nx, i64 ny, i64 nz, int64_t* 
         int64_t* dbuf = nullptr;
         CK(hipMalloc(&dbuf, sizeof(int64_t) * (size_t)(sizes[k] > 0 ? sizes[k] : 1)));
         if (sizes[k] > 0) {
-            k_pairing<T><<<nblocks(sizes[k]), BLOCK, 0, ctx->stream>>>((const T*)ctx->d_f, ctx->d_code_f, d, c, k,
+            k_pairing<T><<<nblocks(sizes[k]), BLOCK, 0, ctx->stream>>>((const T*)ctx->d_f, CodeArray{ctx->d_code_f, c.N}, d, c, k,
                                                                         (ull)sizes[k], dbuf);
             hipError_t e = hipGetLastError();
             if (e == hipSuccess)
@@ -2835,7 +3014,8 @@ int paths_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, co
     uint64_t* gfaces = nullptr;
     if (fl.preserve_geometry != 1) {
         // get_false_as_vpath_connectivity starts from g's critical faces (main_3d.cu:4766)
-        rc = drv.fcrit(ctx->d_code_g, 4);
+        const CodeArray gc = drv.cg();
+        rc = drv.fcrit(&gc, 4);
         if (rc) return rc;
         drv.n_gfaces = ctx->h_ctr[K_FC0 + 2];
         CK(hipMalloc(&gfaces, sizeof(uint64_t) * (drv.n_gfaces + 1)));
@@ -2848,7 +3028,8 @@ int paths_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, co
         }
         drv.as_gfaces = gfaces;
     }
-    rc = drv.prepare_paths(ctx->d_code_f);
+    const CodeArray fcodes = drv.cf();
+    rc = drv.prepare_paths(&fcodes);
     if (rc == 0) rc = drv.detect_paths();
     if (gfaces) {
         (void)hipStreamSynchronize(ctx->stream);
@@ -2870,8 +3051,8 @@ int paths_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, co
         if (rc) return rc;
         if (nds + nas) {
             k_fix_paths<T><<<nblocks(nds + nas), BLOCK, 0, ctx->stream>>>(
-                pa.rec, nas, pd.rec, nds, nullptr, 0, (const T*)ctx->d_f, ctx->d_code_f, (const T*)ctx->d_g,
-                ctx->d_code_g, d, c, ctx->d_counter, 0.0, 0.0, fl.edit_type, drv.sink());
+                pa.rec, nas, pd.rec, nds, nullptr, 0, (const T*)ctx->d_f, drv.cf(), (const T*)ctx->d_g,
+                drv.cg(), d, c, ctx->d_counter, 0.0, 0.0, fl.edit_type, drv.sink());
             CK(hipGetLastError());
         }
         rc = sync_ctr(ctx);
@@ -2920,7 +3101,8 @@ int walls_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, do
     if (rc) return rc;
     rc = drv.g_codes();
     if (rc) return rc;
-    rc = drv.prepare_paths(ctx->d_code_f);
+    const CodeArray fcodes = drv.cf();
+    rc = drv.prepare_paths(&fcodes);
     if (rc) return rc;
     rc = drv.walls();
     if (rc) return rc;
@@ -2940,8 +3122,8 @@ int walls_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, do
         if (rc) return rc;
         if (nw) {
             k_fix_paths<T><<<nblocks(nw), BLOCK, 0, ctx->stream>>>(
-                nullptr, 0, nullptr, 0, pw.rec, nw, (const T*)ctx->d_f, ctx->d_code_f, (const T*)ctx->d_g,
-                ctx->d_code_g, d, c, ctx->d_counter, eps, range, fl.edit_type, drv.sink());
+                nullptr, 0, nullptr, 0, pw.rec, nw, (const T*)ctx->d_f, drv.cf(), (const T*)ctx->d_g,
+                drv.cg(), d, c, ctx->d_counter, eps, range, fl.edit_type, drv.sink());
             CK(hipGetLastError());
         }
         rc = sync_ctr(ctx);

@@ -42,17 +42,17 @@ DMTZ_HD void star_of(const T* fld, const Dims& d, i64 v, LowerStar& ls) {
     lower_star(val, ls);
 }
 
-// Pairing lookups over precomputed star codes (code[v] = encode_star(lower star of v)). Finding
+// Pairing lookups over precomputed star codes (of v: encode_star(lower star of v)). Finding
 // a cell's highest vertex needs only the cell's own values; the partner then comes from that
 // vertex's 32-byte code.
-template <class T>
+template <class T, class Code = const StarCode*>
 struct FieldGrad {
     const T* fld;
-    const StarCode* code;
+    Code code;
     Dims d;
     Counts c;
 
-    DMTZ_HD FieldGrad(const T* f, const StarCode* cd, const Dims& dd, const Counts& cc)
+    DMTZ_HD FieldGrad(const T* f, Code cd, const Dims& dd, const Counts& cc)
         : fld(f), code(cd), d(dd), c(cc) {}
 
     // compare_vertices main_3d.cu:1043-1049: a above b.
@@ -74,7 +74,7 @@ struct FieldGrad {
     // paired_vertices[v]
     DMTZ_HD i64 pv(i64 v) const {
         if (v < 0 || v >= c.N) return -1;
-        int s = code_s(code[v]);
+        int s = partner_slot_of(code, v);
         return s == 15 ? -1 : edge_of(v, s);
     }
 
@@ -85,7 +85,7 @@ struct FieldGrad {
         edge_verts(d, c, e, a, b);
         i64 m = above(a, b) ? a : b, o = (m == a) ? b : a;
         int sl = slot_between(d, m, o);
-        int nib = code_edge(code[m], sl);
+        int nib = partner_edge_of(code, m, sl);
         if (nib == 14) return m;
         if (nib == 15) return -1;
         return tri_id3(d, c, m, o, nb(m, nib));
@@ -102,7 +102,7 @@ struct FieldGrad {
         i64 o1 = (m == p) ? q : p;
         i64 o2 = (m == r) ? q : r;
         int lt = ST.tri_of[slot_between(d, m, o1)][slot_between(d, m, o2)];
-        int cc = code_tri(code[m], lt);
+        int cc = partner_tri_of(code, m, lt);
         int i = ST.tri_i[lt], j = ST.tri_j[lt];
         switch (cc) {
             case 0: return edge_of(m, i);
@@ -129,7 +129,7 @@ struct FieldGrad {
             uint32_t kk = (1u << ST.tet_s[k][0]) | (1u << ST.tet_s[k][1]) | (1u << ST.tet_s[k][2]);
             lq = (kk == key) ? k : lq;
         }
-        int cc = code_tet(code[m], lq);
+        int cc = partner_tet_of(code, m, lq);
         if (cc == 3) return -1;
         int s0 = ST.tet_s[lq][cc == 0 ? 1 : 0];
         int s1 = ST.tet_s[lq][cc == 2 ? 1 : 2];

@@ -315,6 +315,37 @@ struct StarCode {
     uint64_t w[4];
 };
 
+// Star codes of a field on the device, word by word: word k of vertex v at w[k n + v]. A lookup reads
+// one word, and neighbouring lookups of one kind share lines (eight vertices' words in 64 bytes where
+// whole codes hold two); the dense passes read and write only the words they need, in full lines.
+struct CodeArray {
+    uint64_t* w;
+    i64 n;
+};
+DMTZ_HD uint64_t code_word(const StarCode* c, i64 v, int k) { return c[v].w[k]; }
+DMTZ_HD uint64_t code_word(const CodeArray& c, i64 v, int k) { return c.w[(i64)k * c.n + v]; }
+template <class Code>
+DMTZ_HD StarCode code_at(const Code& c, i64 v) {
+    StarCode s;
+    for (int k = 0; k < 4; k++) s.w[k] = code_word(c, v, k);
+    return s;
+}
+DMTZ_HD void code_put(const CodeArray& c, i64 v, const StarCode& s) {
+    for (int k = 0; k < 4; k++) c.w[(i64)k * c.n + v] = s.w[k];
+}
+// One field of a vertex's code.
+template <class Code>
+DMTZ_HD int partner_slot_of(const Code& c, i64 v) { return (int)(code_word(c, v, 0) >> 56) & 15; }
+template <class Code>
+DMTZ_HD int partner_edge_of(const Code& c, i64 v, int a) { return (int)(code_word(c, v, 0) >> (4 * a)) & 15; }
+template <class Code>
+DMTZ_HD int partner_tri_of(const Code& c, i64 v, int t) {
+    const int k = t < 21 ? 0 : 1;
+    return (int)(code_word(c, v, 2 + k) >> (3 * (t - 21 * k))) & 7;
+}
+template <class Code>
+DMTZ_HD int partner_tet_of(const Code& c, i64 v, int q) { return (int)(code_word(c, v, 1) >> (14 + 2 * q)) & 3; }
+
 DMTZ_HD int code_edge(const StarCode& c, int a) { return (int)((c.w[0] >> (4 * a)) & 15u); }
 DMTZ_HD int code_s(const StarCode& c) { return (int)((c.w[0] >> 56) & 15u); }
 DMTZ_HD uint32_t code_L(const StarCode& c) { return (uint32_t)(c.w[1] & 0x3FFFu); }

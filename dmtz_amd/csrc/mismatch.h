@@ -38,8 +38,8 @@ DMTZ_HD i64 local_cell_id(const Dims& d, const Counts& c, i64 v, int lc) {
     return tet_id4(d, c, v, nb(ST.tet_s[q][0]), nb(ST.tet_s[q][1]), nb(ST.tet_s[q][2]));
 }
 
-template <class T>
-DMTZ_HD bool is_crit_lookup(const FieldGrad<T>& X, int type, i64 id) {
+template <class T, class Code>
+DMTZ_HD bool is_crit_lookup(const FieldGrad<T, Code>& X, int type, i64 id) {
     switch (type) {
         case 0: return X.pv(id) == -1;
         case 1: return X.pe(id) == -1;
@@ -71,11 +71,11 @@ DMTZ_HD void local_cells_exist(const Dims& d, i64 v, uint64_t& lo, uint32_t& hi)
 // Critical status in field F of every existing local cell of v: the bits of the cells v owns in
 // F come from v's star code, the others from a pairing lookup at their owner. F is fixed during
 // the correction, so this is evaluated once per run for f.
-template <class T>
-DMTZ_HD void local_crit(const FieldGrad<T>& F, i64 v, uint64_t& lo, uint32_t& hi) {
+template <class T, class Code>
+DMTZ_HD void local_crit(const FieldGrad<T, Code>& F, i64 v, uint64_t& lo, uint32_t& hi) {
     uint64_t c_lo, i_lo, e_lo;
     uint32_t c_hi, i_hi, e_hi;
-    code_masks(F.code[v], c_lo, c_hi, i_lo, i_hi);
+    code_masks(code_at(F.code, v), c_lo, c_hi, i_lo, i_hi);
     local_cells_exist(F.d, v, e_lo, e_hi);
     lo = c_lo & i_lo;
     hi = c_hi & i_hi;

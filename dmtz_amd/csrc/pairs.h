@@ -164,8 +164,8 @@ DMTZ_HD uint32_t cube_pairs(const T* val, const uint64_t* w1) {
 constexpr uint32_t PW_NO_CUBE = PW_NONE * 0x9249u;  // six unpaired tets
 
 // Pair word of vertex v (coordinates x, y, z) from a field and its star codes.
-template <class T>
-DMTZ_HD uint32_t pair_word(const T* fld, const StarCode* code, const Dims& d, i64 v, i64 x, i64 y, i64 z) {
+template <class T, class Code>
+DMTZ_HD uint32_t pair_word(const T* fld, const Code& code, const Dims& d, i64 v, i64 x, i64 y, i64 z) {
     uint32_t word = PW_NO_CUBE;
     if (x < d.W - 1 && y < d.H - 1 && z < d.D - 1) {
         T val[8];
@@ -174,11 +174,11 @@ DMTZ_HD uint32_t pair_word(const T* fld, const StarCode* code, const Dims& d, i6
         for (int k = 0; k < 8; k++) {
             const i64 u = v + (k & 1) + ((k >> 1) & 1) * d.W + ((k >> 2) & 1) * d.W * d.H;
             val[k] = fld[u];
-            w1[k] = code[u].w[1];
+            w1[k] = code_word(code, u, 1);
         }
         word = cube_pairs(val, w1);
     }
-    return word | ((uint32_t)(code[v].w[0] >> 56) & 15u) << PW_SLOT_SHIFT;
+    return word | (uint32_t)partner_slot_of(code, v) << PW_SLOT_SHIFT;
 }
 
 DMTZ_HD uint32_t pw_out(uint32_t word, int type) { return (word >> (3 * type)) & 7u; }

@@ -12,16 +12,16 @@
 
 namespace dmtz {
 
-template <class T, class Sink>
+template <class T, class Sink, class Code = const StarCode*>
 struct Repair {
-    FieldGrad<T> F;  // original field f ("type 0")
-    FieldGrad<T> G;  // decompressed field g ("type 1")
+    FieldGrad<T, Code> F;  // original field f ("type 0")
+    FieldGrad<T, Code> G;  // decompressed field g ("type 1")
     const uint8_t* counter;
     double eps, range;
     int edit_type;
     Sink sink;
 
-    DMTZ_HD Repair(const T* f, const StarCode* cf, const T* g, const StarCode* cg, const Dims& d, const Counts& c,
+    DMTZ_HD Repair(const T* f, Code cf, const T* g, Code cg, const Dims& d, const Counts& c,
                    const uint8_t* cnt, double e, double r, int et, Sink s)
         : F(f, cf, d, c), G(g, cg, d, c), counter(cnt), eps(e), range(r), edit_type(et), sink(s) {}
 
@@ -655,7 +655,7 @@ struct Repair {
     // get_paired_id main_3d.cu:4499-4537 on field which (0 = f, 1 = g): the tet reached by
     // following the ascending pairing from tet id.
     DMTZ_HD i64 paired_max(i64 id, int which, i64 cap, bool& overflow) const {
-        const FieldGrad<T>& X = which == 0 ? F : G;
+        const FieldGrad<T, Code>& X = which == 0 ? F : G;
         i64 cur = id;
         bool done = id < 0;
         i64 steps = 0;

@@ -96,12 +96,12 @@ constexpr RuleTables make_rule_tables() {
 constexpr RuleTables RT = detail::make_rule_tables();
 
 // tb and off (the index offset of every slot, off[14] = 0) lie in LDS on the device.
-template <class T, class Sink>
+template <class T, class Sink, class Code = const StarCode*>
 struct LocalRules {
     const T* f;
-    const StarCode* cf;
+    Code cf;
     const T* g;
-    const StarCode* cg;
+    Code cg;
     const uint8_t* counter;
     const RuleTables* tb;
     const int32_t* off;
@@ -161,13 +161,10 @@ struct LocalRules {
     // Partner fields at the owner: edge: 14 = the owner, < 14 = the triangle completed by that slot,
     // 15 = none; triangle: 0 / 1 = edge to tri_i / tri_j, 2 / 3 = tet through tri_k[0] / [1], 7 = none;
     // tet: the slot its face leaves out, 3 = none.
-    static DMTZ_HD int slot_of(const StarCode* cd, uint32_t v) { return (int)(cd[v].w[0] >> 56) & 15; }
-    static DMTZ_HD int edge_code(const StarCode* cd, At e) { return (int)(cd[e.v].w[0] >> (4 * e.l)) & 15; }
-    static DMTZ_HD int tri_code(const StarCode* cd, At t) {
-        const int k = t.l < 21 ? 0 : 1;
-        return (int)(cd[t.v].w[2 + k] >> (3 * (t.l - 21 * k))) & 7;
-    }
-    static DMTZ_HD int tet_code(const StarCode* cd, At q) { return (int)(cd[q.v].w[1] >> (14 + 2 * q.l)) & 3; }
+    static DMTZ_HD int slot_of(const Code& cd, uint32_t v) { return partner_slot_of(cd, (i64)v); }
+    static DMTZ_HD int edge_code(const Code& cd, At e) { return partner_edge_of(cd, (i64)e.v, e.l); }
+    static DMTZ_HD int tri_code(const Code& cd, At t) { return partner_tri_of(cd, (i64)t.v, t.l); }
+    static DMTZ_HD int tet_code(const Code& cd, At q) { return partner_tet_of(cd, (i64)q.v, q.l); }
 
     DMTZ_HD i64 tri_number(At t) const {
         i64 x, y, z;
