@@ -639,13 +639,20 @@ __global__ __launch_bounds__(BLOCK) void k_fcrit(MaskArray own, CodeArray cf, Co
     block_emit(base, lo, hi, out, ctr);
 }
 
+// The edit set of an epoch: the vertices whose stamp holds it. With a list, each vertex is also
+// appended to it once (an exchange of its stamp and a claim of a slot, both of which wait for the
+// memory side); without, the stamps are plain stores and k_apply_marked reads all of them.
 struct TargetSink {
     uint32_t* stamp;
     uint32_t epoch;
-    uint32_t* list;
+    uint32_t* list;  // null: mark only
     ull* ctr;
     ull cap;
     __device__ void operator()(i64 v) const {
+        if (!list) {
+            stamp[v] = epoch;
+            return;
+        }
         uint32_t old = atomicExch(stamp + v, epoch);
         if (old != epoch) {
             ull i = atomicAdd(ctr, 1ull);
@@ -676,6 +683,13 @@ struct HoldSink {
     // Every lane of the wave must call this. Adds the held targets not yet in this epoch's set.
     __device__ __forceinline__ void flush() const {
         const uint32_t e = direct.epoch;
+        if (!direct.list) {
+            if (n > 0) direct.stamp[t0] = e;
+            if (n > 1) direct.stamp[t1] = e;
+            if (n > 2) direct.stamp[t2] = e;
+            if (n > 3) direct.stamp[t3] = e;
+            return;
+        }
         uint32_t o0 = e, o1 = e, o2 = e, o3 = e;
         if (n > 0) o0 = atomicExch(direct.stamp + t0, e);
         if (n > 1) o1 = atomicExch(direct.stamp + t1, e);
@@ -747,9 +761,40 @@ __global__ __launch_bounds__(64) void k_zero_ctrs(ull* ctr, uint32_t mask) {
 static_assert(K_NCTR <= 32, "k_zero_ctrs takes a 32-bit mask");
 constexpr uint32_t ctr_bit(int k) { return 1u << k; }
 
-// Frozen vertices are never edited. moved counts the edits that changed a value or a counter.
-// The edit set's size is read on the device (*n_ptr, at most cap); the grid strides over the set
-// in block-uniform steps, so every lane takes part in the wave-wide appends.
+// The edit of vertex v (applyDeltaBuffer1 main_3d.cu:1122-1164; frozen vertices are never edited).
+// ch: its value changed (the order, hence every lower star, only sees value comparisons); mv: its
+// value or its counter did.
+template <class T>
+__device__ __forceinline__ void edit_vertex(i64 v, const T* f, T* g, uint8_t* counter, double eps, double range,
+                                            int preserve_type, int edit_type, bool& ch, bool& mv) {
+    const int k0 = counter[v];
+    ch = mv = false;
+    if (k0 == FROZEN) return;
+    const T fv = f[v];
+    const T g0 = g[v];
+    T gv = g0;
+    int k = k0;
+    const double dl = edit_type == 1 ? halving_delta(eps, k) : EditArith<T>::delta0(fv, gv, eps);
+    if (preserve_type == 0) {
+        if (fabs_d(dl) > 1e-15 * range && k < 5 && EditArith<T>::step(fv, gv, dl, eps)) {
+            k += 1;
+        } else {
+            k = 6;
+            gv = EditArith<T>::snap(fv, eps);
+        }
+    } else {
+        k = 6;
+        gv = EditArith<T>::snap(fv, eps);
+    }
+    g[v] = gv;
+    counter[v] = (uint8_t)k;
+    ch = !(gv == g0);
+    mv = ch || k != k0;
+}
+
+// moved counts the edits that changed a value or a counter. The edit set's size is read on the
+// device (*n_ptr, at most cap); the grid strides over the set in block-uniform steps, so every lane
+// takes part in the wave-wide appends.
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_apply(const uint32_t* list, const ull* n_ptr, ull cap, const T* f, T* g,
                                                  uint8_t* counter, double eps, double range, int preserve_type,
@@ -761,33 +806,48 @@ __global__ __launch_bounds__(BLOCK) void k_apply(const uint32_t* list, const ull
         i64 v = 0;
         if (i < n) {
             v = list[i];
-            const int k0 = counter[v];
-            if (k0 != FROZEN) {
-                const T fv = f[v];
-                const T g0 = g[v];
-                T gv = g0;
-                int k = k0;
-                const double dl = edit_type == 1 ? halving_delta(eps, k) : EditArith<T>::delta0(fv, gv, eps);
-                if (preserve_type == 0) {
-                    if (fabs_d(dl) > 1e-15 * range && k < 5 && EditArith<T>::step(fv, gv, dl, eps)) {
-                        k += 1;
-                    } else {
-                        k = 6;
-                        gv = EditArith<T>::snap(fv, eps);
-                    }
-                } else {
-                    k = 6;
-                    gv = EditArith<T>::snap(fv, eps);
-                }
-                g[v] = gv;
-                counter[v] = (uint8_t)k;
-                ch = !(gv == g0);  // the order (hence every lower star) only sees value comparisons
-                mv = ch || k != k0;
-            }
+            edit_vertex(v, f, g, counter, eps, range, preserve_type, edit_type, ch, mv);
         }
         ull at = block_alloc(chg_ctr, ch ? 1 : 0);
         if (ch) changed[at] = (uint32_t)v;
         block_add(moved, mv);
+    }
+}
+
+// The same for a marked edit set: one pass over the stamps, so the edits read and write the fields
+// in order and the changed list comes out in vertex order. APPLY_V vertices per thread and one claim
+// per block keep the claims, which the memory side serves one after the other, below the pass.
+constexpr int APPLY_V = 16;
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_apply_marked(const uint32_t* stamp, uint32_t epoch, i64 n, const T* f, T* g,
+                                                        uint8_t* counter, double eps, double range, int preserve_type,
+                                                        int edit_type, uint32_t* changed, ull* chg_ctr, ull* moved,
+                                                        ull* targets) {
+    __shared__ uint32_t sum[2];
+    if (threadIdx.x < 2) sum[threadIdx.x] = 0;
+    const i64 base = (i64)blockIdx.x * (BLOCK * APPLY_V) + threadIdx.x;
+    uint32_t in = 0;
+#pragma unroll
+    for (int k = 0; k < APPLY_V; k++) {
+        const i64 v = base + (i64)k * BLOCK;
+        in |= (uint32_t)(v < n && stamp[v] == epoch) << k;
+    }
+    if (!__syncthreads_or(in != 0u)) return;
+    uint32_t changes = 0, moves = 0;
+    for (uint32_t m = in; m; m &= m - 1) {
+        const int k = __builtin_ctz(m);
+        bool ch, mv;
+        edit_vertex(base + (i64)k * BLOCK, f, g, counter, eps, range, preserve_type, edit_type, ch, mv);
+        changes |= (uint32_t)ch << k;
+        moves += (uint32_t)mv;
+    }
+    atomicAdd(&sum[0], moves);
+    atomicAdd(&sum[1], (uint32_t)__popc(in));
+    ull at = block_alloc(chg_ctr, __popc(changes));
+    for (uint32_t m = changes; m; m &= m - 1) changed[at++] = (uint32_t)(base + (i64)__builtin_ctz(m) * BLOCK);
+    if (threadIdx.x == 0) {  // block_alloc's barriers order the sums
+        if (sum[0]) atomicAdd(moved, (ull)sum[0]);
+        atomicAdd(targets, (ull)sum[1]);
     }
 }
 
@@ -1906,11 +1966,11 @@ struct Driver {
         return 0;
     }
 
-    TargetSink sink() {
+    TargetSink sink(bool mark = false) {
         TargetSink s;
         s.stamp = ctx->d_stamp;
         s.epoch = ctx->epoch;
-        s.list = ctx->d_targets;
+        s.list = mark ? nullptr : ctx->d_targets;
         s.ctr = ctx->d_ctr + K_TGT;
         s.cap = (ull)ctx->cap_n;
         return s;
@@ -1943,25 +2003,34 @@ struct Driver {
     // reads overlap another's work. Two streams rather than one per kind: the process's streams
     // share four hardware queues, and two streams on one queue run one after the other.
 
+    // From N / TARGET_DENSE records on the edit set is marked and applied by a pass over all stamps
+    // instead of listed. Listing costs a returning atomic per target (about 0.4 ns of the whole chip's
+    // time each: 512^3 fBm's first list of 65 M 2-saddles 27.5 -> 13.2 ms with marks), the pass reads
+    // 4 N bytes (0.3 ms at 512^3 when it edits little).
+    static constexpr ull TARGET_DENSE = 256;
+    bool mark_targets(ull nrec) const { return nrec * TARGET_DENSE >= (ull)c.N; }
+
     int fix_cp(const ull counts[4]) {
         int rc = begin_edits(true);
         if (rc) return rc;
         ull nrec = 0;
-        rc = repair_records(counts, nrec);
+        for (int ty = 0; ty < 4; ty++)
+            if (rule_active(counts, ty)) nrec += counts[ty];
+        rc = repair_records(counts, mark_targets(nrec));
         if (rc) return rc;
-        return apply(nrec);
+        return apply(nrec, mark_targets(nrec));
+    }
+
+    bool rule_active(const ull counts[4], int ty) const {
+        return counts[ty] != 0 && !((ty == 1 || ty == 2) && fl.preserve_saddles != 1);
     }
 
     // The repair rules over the current mismatch lists (counts[ty] records of type ty) into the
-    // edit set of the current epoch; nrec receives the number of records repaired.
-    int repair_records(const ull counts[4], ull& nrec) {
+    // edit set of the current epoch, listed or marked.
+    int repair_records(const ull counts[4], bool mark) {
         Lists4 L = rec_lists(ctx);
         bool active[4];
-        nrec = 0;
-        for (int ty = 0; ty < 4; ty++) {
-            active[ty] = counts[ty] != 0 && !((ty == 1 || ty == 2) && fl.preserve_saddles != 1);
-            if (active[ty]) nrec += counts[ty];
-        }
+        for (int ty = 0; ty < 4; ty++) active[ty] = rule_active(counts, ty);
         const bool side = ctx->fix_concurrent && (active[1] || active[3]) && (active[0] || active[2]);
         if (side && !ctx->fix_stream) {
             // created on first use: batch lanes never run a second stream
@@ -1978,7 +2047,7 @@ struct Driver {
             hipStream_t st = side && (ty == 1 || ty == 3) ? ctx->fix_stream : ctx->stream;
             auto kern = ty == 0 ? k_fix_cp<T, 0> : ty == 1 ? k_fix_cp<T, 1> : ty == 2 ? k_fix_cp<T, 2> : k_fix_cp<T, 3>;
             kern<<<nblocks(counts[ty]), BLOCK, 0, st>>>(L.l[ty], counts[ty], f, cf(), g, cg(), d,
-                                                        c, ctx->d_counter, eps, range, fl.edit_type, sink());
+                                                        c, ctx->d_counter, eps, range, fl.edit_type, sink(mark));
             CK(hipGetLastError());
         }
         if (side) {  // the context's stream waits for the second stream's kinds before the edits apply
@@ -1995,9 +2064,17 @@ struct Driver {
     // launches, and the count of edits that changed a value or a counter (K_MOVED) is read with
     // the next detection's counters. Each vertex enters the edit set at most once per epoch, so
     // the set never exceeds the N entries of its buffer.
-    int apply(ull nrec) {  // its counters start at zero with the epoch (begin_edits(true))
-        if (!nrec) return 0;  // no record, no edit
+    int apply(ull nrec, bool marked) {  // its counters start at zero with the epoch (begin_edits(true))
+        if (!nrec) return 0;            // no record, no edit
         const ull est = nrec < (ull)c.N ? nrec : (ull)c.N;
+        if (marked) {
+            const ull per_block = (ull)BLOCK * APPLY_V;
+            k_apply_marked<T><<<(unsigned)(((ull)c.N + per_block - 1) / per_block), BLOCK, 0, ctx->stream>>>(
+                ctx->d_stamp, ctx->epoch, c.N, f, g, ctx->d_counter, eps, range, fl.preserve_type, fl.edit_type,
+                ctx->d_changed, ctx->d_ctr + K_CHG, ctx->d_ctr + K_MOVED, ctx->d_ctr + K_TGT);
+            CK(hipGetLastError());
+            return refresh(est);
+        }
         k_apply<T><<<stride_blocks(est), BLOCK, 0, ctx->stream>>>(
             ctx->d_targets, ctx->d_ctr + K_TGT, (ull)ctx->cap_n, f, g, ctx->d_counter, eps, range, fl.preserve_type,
             fl.edit_type, ctx->d_changed, ctx->d_ctr + K_CHG, ctx->d_ctr + K_MOVED);
@@ -2012,13 +2089,16 @@ struct Driver {
     // (both give the same codes).
     int refresh(ull est) {
         if (!est) return 0;
-        if (16 * est >= (ull)c.N) {  // many stars may change: decide on the exact count
+        // Dense from N / 64 changed vertices on where the pass runs over bit planes (512^3: 4.6 ms,
+        // where lists of a quarter of the stars took 5 to 8), from N / 16 with a thread per vertex.
+        const ull dense = c.N >= PLANE_MIN ? 64 : 16;
+        if (dense * est >= (ull)c.N) {  // many stars may change: decide on the exact count
             int rc = sync_ctr(ctx);
             if (rc) return rc;
             est = ctx->h_ctr[K_CHG];
             if (!est) return 0;
         }
-        if (16 * est >= (ull)c.N) {  // most stars change: re-evaluate all of them
+        if (dense * est >= (ull)c.N) {  // most stars change: re-evaluate all of them
             int rc = g_codes();
             if (rc) return rc;
             as_full = true;
@@ -2504,13 +2584,14 @@ struct Driver {
         int rc = begin_edits(true);
         if (rc) return rc;
         if (fl.preserve_connectors != 1) nw = 0;
+        const bool mark = mark_targets(nds + nas + nw);
         if (nds + nas + nw) {
             k_fix_paths<T><<<nblocks(nds + nas + nw), BLOCK, 0, ctx->stream>>>(
                 path_list(1).rec, nas, path_list(0).rec, nds, path_list(2).rec, nw, f, cf(), g,
-                cg(), d, c, ctx->d_counter, eps, range, fl.edit_type, sink());
+                cg(), d, c, ctx->d_counter, eps, range, fl.edit_type, sink(mark));
             CK(hipGetLastError());
         }
-        return apply(nds + nas + nw);
+        return apply(nds + nas + nw, mark);
     }
 
     int filtration() {
@@ -2971,8 +3052,7 @@ int targets_host(dmtz_ctx* ctx, const T* f, const T* g, i64 nx, i64 ny, i64 nz, 
     for (int k = 0; k < 4; k++) counts4[k] = (int64_t)cc[k];
     rc = drv.begin_edits();
     if (rc) return rc;
-    ull nrec = 0;
-    rc = drv.repair_records(cc, nrec);
+    rc = drv.repair_records(cc, false);
     if (rc) return rc;
     rc = sync_ctr(ctx);
     if (rc) return rc;
