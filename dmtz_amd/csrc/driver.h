@@ -51,6 +51,7 @@
 #include "repair.h"
 #include "rules.h"
 #include "star_planes.h"
+#include "walls.h"
 
 using namespace dmtz;
 typedef unsigned long long ull;
@@ -72,7 +73,8 @@ enum : int {
     K_ASNEXT = 19,                              // next face of the work-stealing path walk
     K_ASTOTAL = 20,                             // steps of the listed paths
     K_DTILES = 21,                              // tiles whose masks the last detection read
-    K_NCTR = 22
+    K_WOPEN = 22,                               // open faces of the wall checks
+    K_NCTR = 23
 };
 
 constexpr uint8_t FROZEN = 7;  // counter value of a vertex restored to f by the finisher
@@ -1230,10 +1232,6 @@ struct PathList {
     }
 };
 
-struct NoSink {
-    __device__ void operator()(i64) const {}
-};
-
 // The separatrix checks read the pairings of f and g from pair words (pairs.h). Where branches are
 // walked (connectivity mode), one thread per (start cell, branch) writes its result at a fixed
 // position and a combine step per start cell applies the reference's "first branch that fails"
@@ -1685,12 +1683,172 @@ __global__ __launch_bounds__(BLOCK) void k_ds_combine(const uint64_t* fce, ull n
     out.push_block(has, e, rec);
 }
 
-// 2-saddle walls, get_false_ds_wall main_3d.cu:5064-5133, made deterministic: from each
-// f-critical face, a depth-first walk over f's face -> edge -> paired-face steps with a stack and
-// a visited set of its own (the reference shares one stack between threads, defects D2-D5).
-// A face is marked when popped; its edges are taken in the order (v1,v2), (v1,v3), (v2,v3) and
-// pushed in that order, so the last is popped first. The first edge met whose f partner exists
-// and differs from its g partner is recorded as (face, edge), and the walk stops.
+// 2-saddle walls, get_false_ds_wall main_3d.cu:5064-5133, made deterministic: from each f-critical
+// face, a depth-first walk over f's face -> edge -> paired-face steps with a stack and a visited set
+// of its own (the reference shares one stack between threads, defects D2-D5), to the first edge met
+// whose f partner exists and differs from its g partner. The walks are not made: walls.h finds the
+// faces from which a mismatched edge is reached, backwards and once for all walls, and follows one
+// chain per open f-critical face. (A thread per face with its own visited set searched every wall, most
+// of them to their end; the longest of a few thousand faces set the time: 96 x 95 x 97 fBm, 7 ms per
+// launch and 28 ms per check; now 0.5 ms per check, 0.33 of it the serial levels of k_wall_levels.)
+//
+// Bit 16 v + kind of open: the face of that kind anchored at v is open.
+__device__ __forceinline__ bool wall_open(const uint32_t* open, uint32_t id) {
+    const uint64_t b = (uint64_t)(id / 12u) * 16u + id % 12u;
+    return ((open[b >> 5] >> (b & 31u)) & 1u) != 0;
+}
+// Newly opened faces gather in LDS and enter the queue with one claim per block (a claim per wave and
+// face made k_wall_seeds 765 us instead of 97 on average, 96 x 95 x 97); past WALL_BUF of them each claims a slot of its own.
+constexpr uint32_t WALL_BUF = 2048;
+struct WallQueue {
+    uint32_t n;
+    ull base;
+    uint32_t id[WALL_BUF];
+    // every thread of the block: before the first add
+    __device__ __forceinline__ void clear() {
+        if (threadIdx.x == 0) n = 0;
+        __syncthreads();
+    }
+    __device__ __forceinline__ void add(uint32_t* open, uint32_t face, uint32_t* queue, ull* ctr) {
+        const uint64_t b = (uint64_t)(face / 12u) * 16u + face % 12u;
+        const uint32_t bit = 1u << (b & 31u);
+        if (atomicOr(open + (b >> 5), bit) & bit) return;
+        const uint32_t k = atomicAdd(&n, 1u);
+        if (k < WALL_BUF) id[k] = face;
+        else queue[atomicAdd(ctr, 1ull)] = face;
+    }
+    // every thread of the block: after the last add. Returns the end of the queue.
+    __device__ __forceinline__ ull flush(uint32_t* queue, ull* ctr) {
+        __syncthreads();
+        const uint32_t m = n < WALL_BUF ? n : WALL_BUF;
+        if (threadIdx.x == 0) base = atomicAdd(ctr, (ull)m);
+        __syncthreads();
+        const ull b = base;
+        for (uint32_t k = threadIdx.x; k < m; k += blockDim.x) queue[b + k] = id[k];
+        return b + m;
+    }
+};
+
+// Tables of the wall kernels in LDS. Every thread of the block must call load().
+static_assert(sizeof(RuleTables) / 4 <= BLOCK && sizeof(WallTables) <= BLOCK, "one table word per thread");
+struct WallLds {
+    RuleTables tb;
+    WallTables wt;
+    int32_t off[15];
+    __device__ __forceinline__ void load(const Dims& d) {
+        if (threadIdx.x < sizeof(RuleTables) / 4)
+            reinterpret_cast<uint32_t*>(&tb)[threadIdx.x] = reinterpret_cast<const uint32_t*>(&RT)[threadIdx.x];
+        if (threadIdx.x < sizeof(WallTables))
+            reinterpret_cast<uint8_t*>(&wt)[threadIdx.x] = reinterpret_cast<const uint8_t*>(&WT)[threadIdx.x];
+        if (threadIdx.x < 15) off[threadIdx.x] = threadIdx.x == 14 ? 0 : (int32_t)slot_step(d, threadIdx.x);
+        __syncthreads();
+    }
+};
+template <class T>
+struct WallArgs {
+    const T* f;
+    const T* g;
+    CodeArray cf, cg;
+    Dims d;
+    Counts c;
+    uint32_t* open;
+    uint32_t* queue;
+    ull* ctr;  // faces in the queue
+};
+#define DMTZ_WALL_GRAPH(a, lds)                                                                                    \
+    NullSink none;                                                                                                 \
+    const LocalRules<T, NullSink, CodeArray> rules{(a).f, (a).cf, (a).g, (a).cg, nullptr, &(lds).tb, (lds).off,    \
+                                                   (a).d, (a).c,  0.0,   0,      none};                            \
+    const WallGraph<T, CodeArray> graph{rules, &(lds).wt};                                                         \
+    using At = typename WallGraph<T, CodeArray>::At
+
+// The faces of every mismatched edge, each edge taken at its owner in f.
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_wall_seeds(WallArgs<T> a) {
+    __shared__ WallLds lds;
+    __shared__ WallQueue next;
+    next.clear();
+    lds.load(a.d);
+    DMTZ_WALL_GRAPH(a, lds);
+    const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    if (v < a.c.N)
+        graph.mismatched_edges((uint32_t)v, [&](At e) {
+            graph.faces_of(e, [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.ctr); });
+        });
+    next.flush(a.queue, a.ctr);
+}
+
+// One level: the faces that lead on to the queue's faces [from, to).
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_wall_level(WallArgs<T> a, ull from, ull to) {
+    __shared__ WallLds lds;
+    __shared__ WallQueue next;
+    next.clear();
+    lds.load(a.d);
+    DMTZ_WALL_GRAPH(a, lds);
+    const ull i = from + (ull)blockIdx.x * BLOCK + threadIdx.x;
+    if (i < to)
+        graph.leading_to(graph.face_at(a.queue[i]),
+                         [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.ctr); });
+    next.flush(a.queue, a.ctr);
+}
+
+// All levels from there on in one block, which only has to wait for itself between them: levels are
+// many (as long as the longest chain) and small. Every face enters the queue at most once, so the
+// levels end.
+constexpr int WALL_BLOCK = 1024;
+constexpr ull WALL_LEVEL_MIN = 16384;  // larger levels get a launch of their own
+template <class T>
+__global__ __launch_bounds__(WALL_BLOCK) void k_wall_levels(WallArgs<T> a, ull from, ull to) {
+    __shared__ WallLds lds;
+    __shared__ WallQueue next;
+    lds.load(a.d);
+    DMTZ_WALL_GRAPH(a, lds);
+    while (from < to) {
+        next.clear();
+        for (ull i = from + threadIdx.x; i < to; i += WALL_BLOCK)
+            graph.leading_to(graph.face_at(a.queue[i]),
+                             [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.ctr); });
+        from = to;
+        to = next.flush(a.queue, a.ctr);
+        __threadfence();
+        __syncthreads();  // the block reads what it has queued
+    }
+}
+
+// The chain of every open f-critical face to its first mismatched edge; a face whose chain does not
+// end in WALL_CHAIN_CAP steps is listed in ovf for the search.
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_wall_chain(WallArgs<T> a, const uint64_t* starts, ull n, PathList out,
+                                                      uint32_t* ovf, ull* ovf_ctr) {
+    __shared__ WallLds lds;
+    lds.load(a.d);
+    DMTZ_WALL_GRAPH(a, lds);
+    const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
+    bool has = false;
+    i64 face = -1, edge = -1;
+    if (i < n) {
+        const uint64_t r = starts[i];
+        At t{(uint32_t)(r >> 7), (int)(r & 127u) - LC_TRI}, e{0, 0};
+        if (wall_open(a.open, graph.face_id(t))) {
+            int s = 0;
+            for (int k = 0; s == 0 && k < WALL_CHAIN_CAP; k++)
+                s = graph.chain_step(t, e, [&](uint32_t id) { return wall_open(a.open, id); });
+            if (s == 1) {
+                has = true;
+                face = local_cell_id(a.d, a.c, (i64)(r >> 7), (int)(r & 127u));
+                edge = rules.edge_number(e);
+            } else {
+                ovf[atomicAdd(ovf_ctr, 1ull)] = (uint32_t)i;
+            }
+        }
+    }
+    out.push_block(has, face, edge);
+}
+
+// The search itself, for the faces whose chain is capped, and for grids whose faces do not fit the
+// queue's numbers. A face is marked when popped; its edges are taken in the order (v1,v2), (v1,v3),
+// (v2,v3) and pushed in that order, so the last is popped first.
 //
 // Thread t of the launch walks start first + t (or sel[first + t]) with its own part of scratch
 // (2 * slots + 2 entries: the visited set and the stack of Repair::wall_walk). A walk that
@@ -1705,7 +1863,7 @@ __global__ __launch_bounds__(BLOCK) void k_ds_wall(const uint64_t* starts, const
     const ull s = sel ? (ull)sel[first + t] : first + t;
     const uint64_t r = starts[s];
     const i64 face = local_cell_id(d, c, (i64)(r >> 7), (int)(r & 127u));
-    Repair<T, NoSink, CodeArray> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NoSink{});
+    Repair<T, NullSink, CodeArray> R(f, cf, g, cg, d, c, nullptr, 0, 0, 0, NullSink{});
     uint32_t* set = scratch + (size_t)t * (2 * (size_t)slots + 2);
     i64 found = -1;
     const bool overflow = R.wall_walk(face, set, set + slots, slots, found);
@@ -1810,6 +1968,9 @@ struct dmtz_ctx {
     size_t wall_scr_cap = 0;
     uint32_t* d_wall_ovf = nullptr;  // wall walks to repeat with more slots (two lists)
     size_t wall_ovf_cap = 0;
+    uint32_t* d_wall_open = nullptr;   // open faces (16 bits per vertex) and their queue
+    uint32_t* d_wall_queue = nullptr;
+    size_t wall_open_cap = 0, wall_queue_cap = 0;
     int64_t* d_labels = nullptr;  // min labels (2 per f-critical edge), max labels (2 per face)
     int64_t* d_walk = nullptr;    // per-branch walk results (4 per start cell)
     ull* d_ctr = nullptr;
@@ -1890,8 +2051,10 @@ void free_paths(dmtz_ctx* ctx) {
     ctx->labels_cap = ctx->walk_cap = 0;
     (void)hipFree(ctx->d_wall_scr);
     (void)hipFree(ctx->d_wall_ovf);
-    ctx->d_wall_scr = ctx->d_wall_ovf = nullptr;
-    ctx->wall_scr_cap = ctx->wall_ovf_cap = 0;
+    (void)hipFree(ctx->d_wall_open);
+    (void)hipFree(ctx->d_wall_queue);
+    ctx->d_wall_scr = ctx->d_wall_ovf = ctx->d_wall_open = ctx->d_wall_queue = nullptr;
+    ctx->wall_scr_cap = ctx->wall_ovf_cap = ctx->wall_open_cap = ctx->wall_queue_cap = 0;
 }
 
 void free_fc(dmtz_ctx* ctx) {
@@ -2525,10 +2688,55 @@ struct Driver {
         return 0;
     }
 
-    // 2-saddle walls (preserve_connectors, main_3d.cu:5064-5133) from every f-critical face
-    // into the wall list. The walks run in tiers of visited-set size: every start with 256
-    // slots, the walks that outgrow them with 8192, then with 2^18; a wall of more than 2^17
-    // faces is a capacity error. Launches are chunked to keep the per-thread sets near 1 GiB.
+    size_t wall_words() const { return ((size_t)c.N + 1) / 2; }
+    bool wall_buffers() {
+        if (12 * c.N >= ((i64)1 << 32)) return false;
+        if (!grow_buf(ctx, ctx->d_wall_open, ctx->wall_open_cap, wall_words()) &&
+            !grow_buf(ctx, ctx->d_wall_queue, ctx->wall_queue_cap, (size_t)c.F))
+            return true;
+        (void)hipGetLastError();
+        return false;
+    }
+    // The walls by chains; left receives the number of faces to search, listed in the second half of
+    // d_wall_ovf.
+    int wall_chains(ull& left) {
+        int rc;
+        const size_t words = wall_words();
+        const WallArgs<T> a{f, g, cf(), cg(), d, c, ctx->d_wall_open, ctx->d_wall_queue, ctx->d_ctr + K_WOPEN};
+        CK(hipMemsetAsync(ctx->d_wall_open, 0, sizeof(uint32_t) * words, ctx->stream));
+        CK(hipMemsetAsync(ctx->d_ctr + K_WOPEN, 0, sizeof(ull), ctx->stream));
+        CK(hipMemsetAsync(ctx->d_ctr + K_WOVF, 0, sizeof(ull), ctx->stream));
+        k_wall_seeds<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(a);
+        CK(hipGetLastError());
+        ull from = 0, to = 0;
+        for (;;) {
+            rc = sync_ctr(ctx);
+            if (rc) return rc;
+            to = ctx->h_ctr[K_WOPEN];
+            if (to - from < WALL_LEVEL_MIN) break;
+            k_wall_level<T><<<nblocks(to - from), BLOCK, 0, ctx->stream>>>(a, from, to);
+            CK(hipGetLastError());
+            from = to;
+        }
+        left = 0;
+        if (to == 0) return 0;
+        k_wall_levels<T><<<1, WALL_BLOCK, 0, ctx->stream>>>(a, from, to);
+        CK(hipGetLastError());
+        k_wall_chain<T><<<nblocks(nfcf), BLOCK, 0, ctx->stream>>>(a, fcrit_lists(ctx).l[2], nfcf, path_list(2),
+                                                                   ctx->d_wall_ovf + nfcf, ctx->d_ctr + K_WOVF);
+        CK(hipGetLastError());
+        rc = sync_ctr(ctx);
+        if (rc) return rc;
+        left = ctx->h_ctr[K_WOVF];
+        return 0;
+    }
+
+    // 2-saddle walls (preserve_connectors, main_3d.cu:5064-5133) from every f-critical face into the
+    // wall list: the open faces (levels backwards from the mismatched edges), then a chain per open
+    // f-critical face. The faces left over (all of them, where the device has no memory for the queue)
+    // are searched in tiers of visited-set size: with 256 slots, the
+    // walks that outgrow them with 8192, then with 2^18; a search of more than 2^17 faces is a capacity
+    // error. Launches are chunked to keep the per-thread sets near 1 GiB.
     int walls() {
         CK(hipMemsetAsync(ctx->d_ctr + K_DSW, 0, sizeof(ull), ctx->stream));
         if (!nfcf) return 0;
@@ -2543,6 +2751,11 @@ struct Driver {
         Lists4 FL = fcrit_lists(ctx);
         const uint32_t* sel = nullptr;
         ull n = nfcf;
+        if (wall_buffers()) {
+            sel = ctx->d_wall_ovf + nfcf;
+            rc = wall_chains(n);
+            if (rc) return rc;
+        }
         for (int tier = 0; tier < 3 && n > 0; tier++) {
             const uint32_t slots = tiers[tier];
             const size_t per = 2 * (size_t)slots + 2;
