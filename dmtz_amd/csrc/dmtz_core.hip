@@ -43,12 +43,6 @@ void dmtz_ctx_destroy(dmtz_ctx* ctx) {
     free_fc(ctx);
     free_paths(ctx);
     (void)hipFree(ctx->d_ctr);
-    if (ctx->fix_stream) {
-        (void)hipStreamSynchronize(ctx->fix_stream);
-        (void)hipStreamDestroy(ctx->fix_stream);
-    }
-    if (ctx->fix_fork) (void)hipEventDestroy(ctx->fix_fork);
-    if (ctx->fix_join) (void)hipEventDestroy(ctx->fix_join);
     if (ctx->as_stream) {
         (void)hipStreamSynchronize(ctx->as_stream);
         (void)hipStreamDestroy(ctx->as_stream);

@@ -33,6 +33,7 @@
 // deterministic, the order is not, and every consumer is order independent.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 #include <hipcub/hipcub.hpp>
 
 #include <chrono>
@@ -795,7 +796,10 @@ struct HoldSink {
     }
 };
 
-// One kernel per cell type, so each holds only its own repair rule. The rule runs in vertex frames
+// The repair rules of all four cell types in one launch; a block holds records of one type. (A kernel per
+// type, the saddles and maxima on a second stream, cost a short sweep three launches and four event
+// packets more and gained nothing on long lists: 256^3 mixtures 68.9 ms per correction, together 61.8;
+// 512^3 fBm 105.0 either way.) The rule runs in vertex frames
 // (rules.h); a record whose numbers collide takes the rule over global ids, a wave-rare branch.
 // Bound by its two to five dependent reads (values, then a star code, then the partner's values and
 // code): a list of a few records takes 12 us (2-saddles; 80 over global ids). The records are taken in
@@ -803,32 +807,64 @@ struct HoldSink {
 // they read, which is worth more than waves of one branch. (Over global ids, where a wave paid for
 // every branch body with thousands of instructions, the records were grouped by branch first; with
 // these rules the grouping costs 512^3 fBm 19 ms of 195 and 256^3 mixtures 13 of 122.)
+template <class T>
+struct FixArgs {
+    const T* f;
+    CodeArray cf;
+    const T* g;
+    CodeArray cg;
+    Dims d;
+    Counts c;
+    const uint8_t* counter;
+    double eps, range;
+    int edit_type;
+};
+// Tables of the rules in LDS. Every thread of the block must call load().
+struct RuleLds {
+    RuleTables tb;
+    int32_t off[15];
+    __device__ __forceinline__ void load(const Dims& d) {
+        if (threadIdx.x < sizeof(RuleTables) / 4)
+            reinterpret_cast<uint32_t*>(&tb)[threadIdx.x] = reinterpret_cast<const uint32_t*>(&RT)[threadIdx.x];
+        if (threadIdx.x < 15) off[threadIdx.x] = threadIdx.x == 14 ? 0 : (int32_t)slot_step(d, threadIdx.x);
+        __syncthreads();
+    }
+};
 template <class T, int TYPE>
-__global__ __launch_bounds__(BLOCK) void k_fix_cp(const uint64_t* recs, ull n, const T* f, CodeArray cf,
-                                                  const T* g, CodeArray cg, Dims d, Counts c,
-                                                  const uint8_t* counter, double eps, double range, int edit_type,
-                                                  TargetSink sink) {
-    __shared__ RuleTables tb;
-    __shared__ int32_t off[15];
-    if (threadIdx.x < sizeof(RuleTables) / 4)
-        reinterpret_cast<uint32_t*>(&tb)[threadIdx.x] = reinterpret_cast<const uint32_t*>(&RT)[threadIdx.x];
-    if (threadIdx.x < 15) off[threadIdx.x] = threadIdx.x == 14 ? 0 : (int32_t)slot_step(d, threadIdx.x);
-    __syncthreads();
-    const ull i = (ull)blockIdx.x * BLOCK + threadIdx.x;
+__device__ __forceinline__ void fix_record(const FixArgs<T>& a, const RuleLds& lds, uint64_t r, HoldSink& hold) {
+    const uint32_t v = (uint32_t)(r >> 7);
+    const int lc = (int)(r & 127u);
+    LocalRules<T, HoldSink, CodeArray> L{a.f, a.cf, a.g, a.cg, a.counter, &lds.tb, lds.off,
+                                         a.d, a.c, a.eps, a.edit_type, hold};
+    if (__builtin_expect(!L.template run<TYPE>(v, lc), 0)) {
+        Repair<T, HoldSink, CodeArray> R(a.f, a.cf, a.g, a.cg, a.d, a.c, a.counter, a.eps, a.range, a.edit_type, hold);
+        const i64 id = local_cell_id(a.d, a.c, (i64)v, lc);
+        if (TYPE == 1) R.fix_saddle(id);
+        else if (TYPE == 2) R.fix_2saddle(id);
+        else if (TYPE == 3) R.fix_maximum(id);
+        hold = R.sink;
+    }
+}
+// The blocks from first[k] on take the list of type 2, 0, 1, 3 (k = 0 to 3; an empty list has no block).
+struct FixLists {
+    const uint64_t* recs[4];
+    ull n[4];
+    unsigned first[5];
+};
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_fix_cp(FixLists q, FixArgs<T> a, TargetSink sink) {
+    __shared__ RuleLds lds;
+    lds.load(a.d);
+    const unsigned b = blockIdx.x;
+    const int k = b < q.first[1] ? 0 : b < q.first[2] ? 1 : b < q.first[3] ? 2 : 3;
+    const ull i = (ull)(b - q.first[k]) * BLOCK + threadIdx.x;
     HoldSink hold{sink, 0u, 0u, 0u, 0u, 0};
-    if (i < n) {
-        const uint64_t r = recs[i];
-        const uint32_t v = (uint32_t)(r >> 7);
-        const int lc = (int)(r & 127u);
-        LocalRules<T, HoldSink, CodeArray> L{f, cf, g, cg, counter, &tb, off, d, c, eps, edit_type, hold};
-        if (__builtin_expect(!L.template run<TYPE>(v, lc), 0)) {
-            Repair<T, HoldSink, CodeArray> R(f, cf, g, cg, d, c, counter, eps, range, edit_type, hold);
-            const i64 id = local_cell_id(d, c, (i64)v, lc);
-            if (TYPE == 1) R.fix_saddle(id);
-            else if (TYPE == 2) R.fix_2saddle(id);
-            else if (TYPE == 3) R.fix_maximum(id);
-            hold = R.sink;
-        }
+    if (i < q.n[k]) {
+        const uint64_t r = q.recs[k][i];
+        if (k == 0) fix_record<T, 2>(a, lds, r, hold);
+        else if (k == 1) fix_record<T, 0>(a, lds, r, hold);
+        else if (k == 2) fix_record<T, 1>(a, lds, r, hold);
+        else fix_record<T, 3>(a, lds, r, hold);
     }
     hold.flush();
 }
@@ -841,6 +877,15 @@ __global__ __launch_bounds__(64) void k_zero_ctrs(ull* ctr, uint32_t mask) {
 }
 static_assert(K_NCTR <= 32, "k_zero_ctrs takes a 32-bit mask");
 constexpr uint32_t ctr_bit(int k) { return 1u << k; }
+constexpr uint32_t DETECT_CTRS = ctr_bit(K_MIN) | ctr_bit(K_MIN + 1) | ctr_bit(K_MIN + 2) | ctr_bit(K_MIN + 3) |
+                                 ctr_bit(K_DTILES);
+
+// The counters into the host's pinned copy: a launch costs the host a third of the copy command that
+// would do it.
+__global__ __launch_bounds__(64) void k_read_ctrs(const ull* ctr, ull* host) {
+    const int k = (int)threadIdx.x;
+    if (k < K_NCTR) host[k] = ctr[k];
+}
 
 // The edit of vertex v (applyDeltaBuffer1 main_3d.cu:1122-1164; frozen vertices are never edited).
 // ch: its value changed (the order, hence every lower star, only sees value comparisons); mv: its
@@ -1952,9 +1997,7 @@ struct dmtz_ctx {
     uint64_t* d_fc = nullptr;     // 4 f-critical lists of fc_cap entries
     int64_t* d_path = nullptr;    // ds id/rec, as id/rec, wall id/rec (fc_cap each)
     // The second stream of the repair phase.
-    bool fix_concurrent = true;  // off in batch lanes: no second stream (repairs, path precompute)
-    hipStream_t fix_stream = nullptr;
-    hipEvent_t fix_fork = nullptr, fix_join = nullptr;
+    bool side_stream = true;  // off in batch lanes: no second stream for the path precompute
     uint32_t* d_pairf = nullptr;     // pair words of f and, where branches are walked, of g
     uint32_t* d_pairg = nullptr;
     uint8_t* d_mis = nullptr;        // per vertex: where the pairings of f and g differ
@@ -2174,7 +2217,8 @@ ull max4(const ull* x) {
 }
 
 int sync_ctr(dmtz_ctx* ctx) {
-    CK(hipMemcpyAsync(ctx->h_ctr, ctx->d_ctr, sizeof(ull) * K_NCTR, hipMemcpyDeviceToHost, ctx->stream));
+    k_read_ctrs<<<1, 64, 0, ctx->stream>>>(ctx->d_ctr, ctx->h_ctr);
+    CK(hipGetLastError());
     CK(hipStreamSynchronize(ctx->stream));
     return 0;
 }
@@ -2229,16 +2273,20 @@ struct Driver {
         return overflow_check(ctx);
     }
 
+    bool det_clear = false;  // the detection counters were zeroed with the epoch's (begin_edits(true))
+
     int detect_once() {
-        k_zero_ctrs<<<1, 64, 0, ctx->stream>>>(ctx->d_ctr, ctr_bit(K_MIN) | ctr_bit(K_MIN + 1) | ctr_bit(K_MIN + 2) |
-                                                        ctr_bit(K_MIN + 3) | ctr_bit(K_DTILES));
-        CK(hipGetLastError());
-        CK(hipEventRecord(ctx->ev0, ctx->stream));
+        if (!det_clear) {
+            k_zero_ctrs<<<1, 64, 0, ctx->stream>>>(ctx->d_ctr, DETECT_CTRS);
+            CK(hipGetLastError());
+        }
+        det_clear = false;
         const ull ntiles = (ull)((c.N + EMIT_TILE - 1) / EMIT_TILE);
-        k_detect<<<(unsigned)(ntiles < DETECT_BLOCKS ? ntiles : DETECT_BLOCKS), BLOCK, 0, ctx->stream>>>(
-            ctx->d_mm, c.N, ctx->d_tile_nz, rec_lists(ctx), ctx->d_ctr + K_MIN, ctx->d_ctr + K_DTILES);
+        // the events take the kernel's own time stamps: recorded around it they are two packets more
+        hipExtLaunchKernelGGL(k_detect, dim3((unsigned)(ntiles < DETECT_BLOCKS ? ntiles : DETECT_BLOCKS)), dim3(BLOCK),
+                              0, ctx->stream, ctx->ev0, ctx->ev1, 0, ctx->d_mm, c.N, ctx->d_tile_nz, rec_lists(ctx),
+                              ctx->d_ctr + K_MIN, ctx->d_ctr + K_DTILES);
         CK(hipGetLastError());
-        CK(hipEventRecord(ctx->ev1, ctx->stream));
         int rc = sync_ctr(ctx);
         if (rc) return rc;
         float ms = 0;
@@ -2276,20 +2324,18 @@ struct Driver {
             if (zone_from) zone_from = 1;
         }
         // the edit set; with for_apply also the counters of its apply (changed and dirty lists,
-        // moved edits), whose last values the host has read before this epoch begins (the
-        // finisher keeps its changed list across its epochs, so it zeroes those itself)
+        // moved edits) and of the detection after it, whose last values the host has read before this
+        // epoch begins (the finisher keeps its changed list across its epochs, so it zeroes those itself)
         k_zero_ctrs<<<1, 64, 0, ctx->stream>>>(
-            ctx->d_ctr, ctr_bit(K_TGT) | (for_apply ? ctr_bit(K_CHG) | ctr_bit(K_DIRTY) | ctr_bit(K_MOVED) : 0u));
+            ctx->d_ctr, ctr_bit(K_TGT) |
+                            (for_apply ? ctr_bit(K_CHG) | ctr_bit(K_DIRTY) | ctr_bit(K_MOVED) | DETECT_CTRS : 0u));
+        if (for_apply) det_clear = true;
         CK(hipGetLastError());
         return 0;
     }
 
     // Repair phase of one critical-point sweep (main_3d.cu:6801-6833) + apply (:6837). The kinds are
-    // repaired concurrently
-    // (the edits form a set: their order does not matter): minima and 2-saddles on the context's
-    // stream, saddles then maxima on a second one, so that one kind's longest chains of dependent
-    // reads overlap another's work. Two streams rather than one per kind: the process's streams
-    // share four hardware queues, and two streams on one queue run one after the other.
+    // repaired by one launch (the edits form a set: their order does not matter).
 
     // From N / TARGET_DENSE records on the edit set is marked and applied by a pass over all stamps
     // instead of listed. Listing costs a returning atomic per target (about 0.4 ns of the whole chip's
@@ -2316,32 +2362,32 @@ struct Driver {
     // The repair rules over the current mismatch lists (counts[ty] records of type ty) into the
     // edit set of the current epoch, listed or marked.
     int repair_records(const ull counts[4], bool mark) {
-        Lists4 L = rec_lists(ctx);
-        bool active[4];
-        for (int ty = 0; ty < 4; ty++) active[ty] = rule_active(counts, ty);
-        const bool side = ctx->fix_concurrent && (active[1] || active[3]) && (active[0] || active[2]);
-        if (side && !ctx->fix_stream) {
-            // created on first use: batch lanes never run a second stream
-            CK(hipStreamCreateWithFlags(&ctx->fix_stream, hipStreamNonBlocking));
-            CK(hipEventCreateWithFlags(&ctx->fix_fork, hipEventDisableTiming));
-            CK(hipEventCreateWithFlags(&ctx->fix_join, hipEventDisableTiming));
+        const Lists4 L = rec_lists(ctx);
+        const FixArgs<T> args{f, cf(), g, cg(), d, c, ctx->d_counter, eps, range, fl.edit_type};
+        const int order[4] = {2, 0, 1, 3};
+        FixLists q{};
+        for (int k = 0; k < 4; k++) {
+            const int ty = order[k];
+            const ull n = rule_active(counts, ty) ? counts[ty] : 0;
+            if ((ull)q.first[k] + nblocks(n) >= FIX_BLOCKS) {  // more threads than a launch takes: the lists so far
+                int rc = launch_fix(q, q.first[k], args, mark);
+                if (rc) return rc;
+                q = FixLists{};
+            }
+            q.recs[k] = L.l[ty];
+            q.n[k] = n;
+            q.first[k + 1] = q.first[k] + nblocks(n);
         }
-        if (side) {
-            CK(hipEventRecord(ctx->fix_fork, ctx->stream));
-            CK(hipStreamWaitEvent(ctx->fix_stream, ctx->fix_fork, 0));
-        }
-        for (int ty : {2, 0, 1, 3}) {
-            if (!active[ty]) continue;
-            hipStream_t st = side && (ty == 1 || ty == 3) ? ctx->fix_stream : ctx->stream;
-            auto kern = ty == 0 ? k_fix_cp<T, 0> : ty == 1 ? k_fix_cp<T, 1> : ty == 2 ? k_fix_cp<T, 2> : k_fix_cp<T, 3>;
-            kern<<<nblocks(counts[ty]), BLOCK, 0, st>>>(L.l[ty], counts[ty], f, cf(), g, cg(), d,
-                                                        c, ctx->d_counter, eps, range, fl.edit_type, sink(mark));
-            CK(hipGetLastError());
-        }
-        if (side) {  // the context's stream waits for the second stream's kinds before the edits apply
-            CK(hipEventRecord(ctx->fix_join, ctx->fix_stream));
-            CK(hipStreamWaitEvent(ctx->stream, ctx->fix_join, 0));
-        }
+        return launch_fix(q, q.first[4], args, mark);
+    }
+    static constexpr ull FIX_BLOCKS = ((ull)1 << 32) / BLOCK;
+    int launch_fix(const FixLists& q, unsigned blocks, const FixArgs<T>& args, bool mark) {
+        if (blocks == 0) return 0;
+        FixLists all = q;
+        for (int k = 1; k < 5; k++)
+            if (all.first[k] < all.first[k - 1]) all.first[k] = all.first[k - 1];
+        k_fix_cp<T><<<blocks, BLOCK, 0, ctx->stream>>>(all, args, sink(mark));
+        CK(hipGetLastError());
         return 0;
     }
 
@@ -2379,7 +2425,11 @@ struct Driver {
         // Dense from N / 64 changed vertices on where the pass runs over bit planes (512^3: 4.6 ms,
         // where lists of a quarter of the stars took 5 to 8), from N / 16 with a thread per vertex.
         const ull dense = c.N >= PLANE_MIN ? 64 : 16;
-        if (dense * est >= (ull)c.N) {  // many stars may change: decide on the exact count
+        // Up to CODE_SMALL vertices (a wave per SIMD) the pass over all of them takes as long as the
+        // shortest list (32^3: 17 us both), and neither the list nor its length is needed.
+        if (c.N <= CODE_SMALL) {
+            est = (ull)c.N;
+        } else if (dense * est >= (ull)c.N) {  // many stars may change: decide on the exact count
             int rc = sync_ctr(ctx);
             if (rc) return rc;
             est = ctx->h_ctr[K_CHG];
@@ -2516,6 +2566,7 @@ struct Driver {
     // idle and its 55 us of work (float32; 80 in float64) is the time of the pass, against 0.12 us per
     // thousand vertices with a thread per vertex (64^3: 47 us, 129 x 96 x 111 float64: 172).
     static constexpr i64 PLANE_MIN = (i64)1 << 19;
+    static constexpr i64 CODE_SMALL = (i64)1 << 16;
     unsigned plane_blocks() const { return (unsigned)((c.N + PLANE_TILE - 1) / PLANE_TILE); }
 
     // Star codes of every vertex of a field.
@@ -2820,7 +2871,7 @@ struct Driver {
     int as_stage = 0;
 
     int as_start_async() {
-        if (!ctx->fix_concurrent || !as_listable() || as_ready || !nfcf) return 0;
+        if (!ctx->side_stream || !as_listable() || as_ready || !nfcf) return 0;
         if (!ctx->as_stream) {
             CK(hipStreamCreateWithFlags(&ctx->as_stream, hipStreamNonBlocking));
             CK(hipEventCreateWithFlags(&ctx->as_ev_fork, hipEventDisableTiming));
@@ -3272,7 +3323,7 @@ int correct_batch(dmtz_ctx* ctx, const Field* fields, int32_t n, const dmtz_flag
             ctx->err = "batch lane context creation failed";
             return rc;
         }
-        w->fix_concurrent = false;  // one stream per lane: more would share the four hardware queues
+        w->side_stream = false;  // one stream per lane: more would share the four hardware queues
         ctx->workers.push_back(w);
     }
     for (dmtz_ctx* w : ctx->workers) w->err.clear();
