@@ -164,6 +164,8 @@ def _single_runtime():
     runtime. torch bundles its own libamdhip64; when torch is imported first, the library binds
     to that copy (same soname), otherwise the process holds two runtimes whose streams do not
     order against each other."""
+    if N.lib().dmtz_hip_runtimes() < 2:  # 0.5 ms less per tensor than reading the maps
+        return
     paths = set()
     with open("/proc/self/maps") as fh:
         for line in fh:

@@ -82,6 +82,9 @@ typedef struct dmtz_ctx dmtz_ctx;
 int dmtz_ctx_create(dmtz_ctx** out, int device);
 void dmtz_ctx_destroy(dmtz_ctx* ctx);
 const char* dmtz_last_error(const dmtz_ctx* ctx);
+/* HIP runtime libraries loaded in the process; with more than one, device buffers of the other do
+ * not order against this library's streams. */
+int dmtz_hip_runtimes(void);
 
 /* eps = rel * (max f - min f) and range = max f - min f, main_3d.cu:6301-6309. */
 int dmtz_eps_from_rel_f32(const float* f, int64_t n, double rel, double* eps_out, double* range_out);
