@@ -70,6 +70,8 @@ def lib():
     L.dmtz_ctx_destroy.restype = None
     L.dmtz_last_error.argtypes = [P]
     L.dmtz_last_error.restype = ctypes.c_char_p
+    L.dmtz_hip_runtimes.argtypes = []
+    L.dmtz_hip_runtimes.restype = ctypes.c_int
     for t in ("f32", "f64"):
         getattr(L, "dmtz_eps_from_rel_" + t).argtypes = [P, I64, D, ctypes.POINTER(D), ctypes.POINTER(D)]
         for name in ("dmtz_correct_", "dmtz_correct_dev_"):
@@ -121,7 +123,7 @@ def lib():
 
 # Every symbol declared in include/dmtz.h and include/dmtz_learned.h.
 EXPORTS = (
-    "dmtz_ctx_create", "dmtz_ctx_destroy", "dmtz_last_error",
+    "dmtz_ctx_create", "dmtz_ctx_destroy", "dmtz_last_error", "dmtz_hip_runtimes",
     "dmtz_eps_from_rel_f32", "dmtz_eps_from_rel_f64",
     "dmtz_correct_f32", "dmtz_correct_f64", "dmtz_correct_dev_f32", "dmtz_correct_dev_f64",
     "dmtz_trajectory", "dmtz_phase_times", "dmtz_kernel_stats", "dmtz_run_info",
