@@ -21,25 +21,30 @@ DMTZ_HD float pos_inf<float>() { return __builtin_huge_valf(); }
 template <>
 DMTZ_HD double pos_inf<double>() { return __builtin_huge_val(); }
 
-// Closed-star values of vertex v (val[14] = v), +inf for off-grid neighbours.
+// Closed-star values of vertex v (val[14] = v), +inf for off-grid neighbours. Returns the slots inside
+// the grid.
 template <class T>
-DMTZ_HD void gather_star(const T* fld, const Dims& d, i64 v, T* val) {
+DMTZ_HD uint32_t gather_star(const T* fld, const Dims& d, i64 v, T* val) {
     i64 x, y, z;
     vxyz(d, v, x, y, z);
+    uint32_t grid = 0;
 #pragma unroll
     for (int k = 0; k < 14; k++) {
         i64 nx = x + DIR[k][0], ny = y + DIR[k][1], nz = z + DIR[k][2];
-        val[k] = inb(d, nx, ny, nz) ? fld[vidx(d, nx, ny, nz)] : pos_inf<T>();
+        const bool in = inb(d, nx, ny, nz);
+        val[k] = in ? fld[vidx(d, nx, ny, nz)] : pos_inf<T>();
+        grid |= (uint32_t)in << k;
     }
     val[14] = fld[v];
+    return grid;
 }
 
 // Lower star of vertex v from the field values (the dense classification step).
 template <class T>
 DMTZ_HD void star_of(const T* fld, const Dims& d, i64 v, LowerStar& ls) {
     T val[15];
-    gather_star(fld, d, v, val);
-    lower_star(val, ls);
+    const uint32_t grid = gather_star(fld, d, v, val);
+    lower_star(val, ls, grid);
 }
 
 // Pairing lookups over precomputed star codes (of v: encode_star(lower star of v)). Finding

@@ -18,7 +18,9 @@
 //
 // Order: u < w  <=>  val[u] < val[w] or (val[u] == val[w] and index u < index w)
 // (main_3d.cu:1043-1049). Inside one star the index order of two slots is the fixed rank TB[].
-// Absent (off-grid) neighbours carry +inf and so are never below anything; fields are finite.
+// Absent (off-grid) neighbours carry +inf and so are below nothing finite; the caller also names the
+// slots inside the grid, since a vertex whose own value is +inf is tied with the absent ones and would
+// be paired across the grid's boundary.
 #pragma once
 #include "stencil.h"
 
@@ -113,14 +115,15 @@ DMTZ_HD uint32_t bit1(uint64_t x, int k) { return (uint32_t)(x >> k) & 1u; }
 
 }  // namespace detail
 
-// Evaluate the five passes on the lower star of the centre of val[15] (val[14] = centre).
+// Evaluate the five passes on the lower star of the centre of val[15] (val[14] = centre); grid holds
+// the slots inside the grid.
 // Every per-cell condition is computed as 0/1 integer arithmetic on the slot masks, with the
 // selections resolved at compile time: "below both n_i and n_j" is blw[i] & blw[j], "strictly
 // between them" is blw[i] ^ blw[j] (the order is total, so whatever is below the lower of the
 // two is below the higher), and the triangles paired in E0 / E1 are set from the slot each edge
 // chose, through the compile-time triangle index of (edge slot, chosen slot).
 template <class T>
-DMTZ_HD void lower_star(const T* val, LowerStar& r) {
+DMTZ_HD void lower_star(const T* val, LowerStar& r, uint32_t grid = 0x3FFFu) {
     using detail::bit1;
     uint32_t blw[14];
 #pragma unroll
@@ -128,6 +131,7 @@ DMTZ_HD void lower_star(const T* val, LowerStar& r) {
     detail::PairLoop<0, 1>::run(val, blw);
     uint32_t L = 0;
     detail::CentreLoop<0>::run(val, L);
+    L &= grid;
 #pragma unroll
     for (int i = 0; i < 14; i++) DMTZ_OPAQUE(blw[i]);
     DMTZ_OPAQUE(L);
