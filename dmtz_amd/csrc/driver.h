@@ -365,78 +365,7 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const
 // the spills cost more than the second wave gives (15 ms). Codes and masks are stored word by word
 // (CodeArray, MaskArray): as 32-byte structs, whose words leave a tile at different times, the lines
 // were written to memory several times over (23.5 GB instead of 6.4 at 512^3, 10.7 ms).
-constexpr int PLANE_ROWS = 32;
-constexpr i64 PLANE_TILE = 64 * PLANE_ROWS;
 static_assert(PLANE_TILE == EMIT_TILE, "a wave's count of nonzero masks is its tile's");
-
-// 64 vertices further in coordinates: at most one carry per axis.
-struct Step64 {
-    int x, y, z;
-    explicit Step64(const Dims& d)
-        : x((int)(64 % d.W)), y((int)(64 / d.W % d.H)), z((int)(64 / (d.W * d.H))) {}
-};
-
-// The comparison words of a wave's tile. The next row's values are loaded while a row is compared;
-// a neighbour's index is only kept inside the field, since finish() drops the slots outside the grid.
-template <class T>
-__device__ __forceinline__ void tile_words(const T* fld, const Dims& d, const Step64& st, i64 n, i64 v0, StarWords& w) {
-    const int W = (int)d.W, H = (int)d.H, D = (int)d.D, last = (int)(n - 1);
-    i64 x64, y64, z64;
-    vxyz(d, v0 <= last ? v0 : last, x64, y64, z64);
-    int x = (int)x64, y = (int)y64, z = (int)z64;
-    uint32_t v = (uint32_t)v0;  // v0 < n + PLANE_TILE < 2^32
-    int32_t off[14];
-#pragma unroll
-    for (int k = 0; k < 14; k++) off[k] = (int32_t)slot_step(d, k);
-    uint32_t side[6] = {0, 0, 0, 0, 0, 0};
-    auto load = [&](T* val) {
-        const uint32_t u = v < (uint32_t)last ? v : (uint32_t)last;
-#pragma unroll
-        for (int k = 0; k < 14; k++) {
-            uint32_t q;
-            if (k & 1) {  // odd slots lead down
-                const int t = (int)u + off[k];
-                q = t < 0 ? 0u : (uint32_t)t;
-            } else {
-                const uint32_t t = u + (uint32_t)off[k];
-                q = t < (uint32_t)last ? t : (uint32_t)last;
-            }
-            val[k] = fld[q];
-        }
-        val[14] = fld[u];
-        v += 64;
-    };
-    auto sides = [&]() {
-        side[0] = (side[0] << 1) | (uint32_t)(x > 0);
-        side[1] = (side[1] << 1) | (uint32_t)(x < W - 1);
-        side[2] = (side[2] << 1) | (uint32_t)(y > 0);
-        side[3] = (side[3] << 1) | (uint32_t)(y < H - 1);
-        side[4] = (side[4] << 1) | (uint32_t)(z > 0);
-        side[5] = (side[5] << 1) | (uint32_t)(z < D - 1);
-        x += st.x;
-        const int cx = x >= W;
-        x -= cx ? W : 0;
-        y += st.y + cx;
-        const int cy = y >= H;
-        y -= cy ? H : 0;
-        z += st.z + cy;
-    };
-#pragma unroll
-    for (int k = 0; k < N_PAIRS; k++) w.p[k] = 0;
-#pragma unroll
-    for (int k = 0; k < 14; k++) w.l[k] = 0;
-    T cur[15], nxt[15];
-    load(cur);
-#pragma unroll 1
-    for (int b = 0; b < PLANE_ROWS; b++) {
-        load(nxt);  // past the last row: not used
-        sides();
-        add_vertex(cur, w);
-#pragma unroll
-        for (int k = 0; k < 15; k++) cur[k] = nxt[k];
-    }
-    finish(w, side);
-}
 
 // Stores of a tile: codes, and per vertex its owned critical cells (crit_f null) or the mismatch
 // with f's critical cells.

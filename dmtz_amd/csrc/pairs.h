@@ -297,10 +297,6 @@ DMTZ_HD bool path_mismatch(const Dims& d, const uint32_t* pf, const uint32_t* pg
     return found;
 }
 
-DMTZ_HD i64 slot_step(const Dims& d, uint32_t slot) {  // index offset of a star slot
-    return DIR[slot][0] + (i64)DIR[slot][1] * d.W + (i64)DIR[slot][2] * d.W * d.H;
-}
-
 // get_orginal_saddle_min_pairs (main_3d.cu:4613-4687): the minimum reached from vertex v. step[s] =
 // slot_step of slot s.
 DMTZ_HD i64 paired_min(const uint32_t* pw, const i64* step, i64 v, i64 cap, bool& overflow) {

@@ -36,6 +36,9 @@ struct StarWords {
     }
 };
 
+DMTZ_HD float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+DMTZ_HD double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // The sign bit of a - b: a < b (a, b finite, neither -0; subnormal differences are kept).
 DMTZ_HD uint32_t sign_word(float a, float b) {
     const float x = a - b;
@@ -78,6 +81,27 @@ struct WordCentreLoop {
     }
 };
 
+// The same two for values of which some are infinite or NaN: their differences have no sign to go by, so
+// the bits are the comparisons of lower_star.h (below).
+template <int I, int J>
+struct WordLoopAny {
+    template <class T>
+    DMTZ_HD static void run(const T* val, StarWords& w) {
+        uint32_t& x = w.p[pair_index(I, J)];
+        x = (x << 1) | (uint32_t)(below<T, I, J>(val) != (TB[I] < TB[J]));
+        if constexpr (J + 1 < 14) WordLoopAny<I, J + 1>::run(val, w);
+        else if constexpr (I + 2 < 14) WordLoopAny<I + 1, I + 2>::run(val, w);
+    }
+};
+template <int I>
+struct WordCentreLoopAny {
+    template <class T>
+    DMTZ_HD static void run(const T* val, StarWords& w) {
+        w.l[I] = (w.l[I] << 1) | (uint32_t)(below<T, I, 14>(val) != (TB[I] < TB[14]));
+        if constexpr (I + 1 < 14) WordCentreLoopAny<I + 1>::run(val, w);
+    }
+};
+
 // fn(0), ..., fn(N - 1) with compile-time arguments: the passes below are too long for the unroller,
 // and an index that is not a constant would put their words into memory.
 #if defined(__HIPCC__)
@@ -108,7 +132,7 @@ DMTZ_HD void transpose_step(uint32_t* a) {
 }  // namespace detail
 
 // Shift the comparisons of one more vertex's values into the words (the last vertex is bit 0). The
-// values are finite; a slot outside the grid may hold any finite value.
+// values are finite; a slot outside the grid may hold any of them.
 template <class T>
 DMTZ_HD void add_vertex(const T* val, StarWords& w) {
     T v[15];
@@ -116,6 +140,13 @@ DMTZ_HD void add_vertex(const T* val, StarWords& w) {
     for (int k = 0; k < 15; k++) v[k] = val[k] + (T)0;  // -0 to +0: equal values have no sign
     detail::WordLoop<0, 1>::run(v, w);
     detail::WordCentreLoop<0>::run(v, w);
+}
+
+// The same for any values, by comparisons.
+template <class T>
+DMTZ_HD void add_vertex_any(const T* val, StarWords& w) {
+    detail::WordLoopAny<0, 1>::run(val, w);
+    detail::WordCentreLoopAny<0>::run(val, w);
 }
 
 // After the last vertex: side[2 a] and side[2 a + 1] say for which vertices the grid goes on down and
@@ -129,6 +160,93 @@ DMTZ_HD void finish(StarWords& w, const uint32_t* side) {
             if (DIR[k][a] != 0) x &= side[2 * a + (DIR[k][a] > 0)];
         w.l[k] = x;
     }
+}
+
+constexpr int PLANE_ROWS = 32;
+constexpr i64 PLANE_TILE = 64 * PLANE_ROWS;
+
+// 64 vertices further in coordinates: at most one carry per axis.
+struct Step64 {
+    int x, y, z;
+    DMTZ_HD explicit Step64(const Dims& d)
+        : x((int)(64 % d.W)), y((int)(64 / d.W % d.H)), z((int)(64 / (d.W * d.H))) {}
+};
+
+// The comparison words of one lane of a wave's tile: lane l of the tile at vertex base takes the vertices
+// v0 + 64 b, v0 = base + l. The next row's values are loaded while a row is compared; a neighbour's
+// index is only kept inside the field, since finish() drops the slots outside the grid. The tile's values
+// gather in a sum of zeros, which an infinity or a NaN makes a NaN: a lane that met one takes its rows
+// again with comparisons (15 multiply-adds a row, 2 % of the pass's instructions).
+template <class T>
+DMTZ_HD void tile_words(const T* fld, const Dims& d, const Step64& st, i64 n, i64 v0, StarWords& w) {
+    const int W = (int)d.W, H = (int)d.H, D = (int)d.D, last = (int)(n - 1);
+    i64 x64, y64, z64;
+    vxyz(d, v0 <= last ? v0 : last, x64, y64, z64);
+    int x = (int)x64, y = (int)y64, z = (int)z64;
+    uint32_t v = (uint32_t)v0;  // v0 < n + PLANE_TILE < 2^32
+    int32_t off[14];
+#pragma unroll
+    for (int k = 0; k < 14; k++) off[k] = (int32_t)slot_step(d, k);
+    uint32_t side[6] = {0, 0, 0, 0, 0, 0};
+    auto load = [&](T* val) {
+        const uint32_t u = v < (uint32_t)last ? v : (uint32_t)last;
+#pragma unroll
+        for (int k = 0; k < 14; k++) {
+            uint32_t q;
+            if (k & 1) {  // odd slots lead down
+                const int t = (int)u + off[k];
+                q = t < 0 ? 0u : (uint32_t)t;
+            } else {
+                const uint32_t t = u + (uint32_t)off[k];
+                q = t < (uint32_t)last ? t : (uint32_t)last;
+            }
+            val[k] = fld[q];
+        }
+        val[14] = fld[u];
+        v += 64;
+    };
+    T zero = 0;
+    auto sides = [&]() {
+        side[0] = (side[0] << 1) | (uint32_t)(x > 0);
+        side[1] = (side[1] << 1) | (uint32_t)(x < W - 1);
+        side[2] = (side[2] << 1) | (uint32_t)(y > 0);
+        side[3] = (side[3] << 1) | (uint32_t)(y < H - 1);
+        side[4] = (side[4] << 1) | (uint32_t)(z > 0);
+        side[5] = (side[5] << 1) | (uint32_t)(z < D - 1);
+        x += st.x;
+        const int cx = x >= W;
+        x -= cx ? W : 0;
+        y += st.y + cx;
+        const int cy = y >= H;
+        y -= cy ? H : 0;
+        z += st.z + cy;
+    };
+#pragma unroll
+    for (int k = 0; k < N_PAIRS; k++) w.p[k] = 0;
+#pragma unroll
+    for (int k = 0; k < 14; k++) w.l[k] = 0;
+    T cur[15], nxt[15];
+    load(cur);
+#pragma unroll 1
+    for (int b = 0; b < PLANE_ROWS; b++) {
+        load(nxt);  // past the last row: not used
+        sides();
+        add_vertex(cur, w);
+#pragma unroll
+        for (int k = 0; k < 15; k++) {
+            zero = fma_of(cur[k], (T)0, zero);
+            cur[k] = nxt[k];
+        }
+    }
+    if (__builtin_expect(zero != zero, 0)) {
+        v = (uint32_t)v0;
+#pragma unroll 1
+        for (int b = 0; b < PLANE_ROWS; b++) {  // 32 bits are pushed: nothing of the words before is left
+            load(cur);
+            add_vertex_any(cur, w);
+        }
+    }
+    finish(w, side);
 }
 
 // 32 x 32 bit transpose in place: bit p of a[r] becomes bit r of a[p].

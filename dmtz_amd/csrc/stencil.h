@@ -461,6 +461,10 @@ DMTZ_HD void tet_verts(const Dims& d, i64 q, i64& v1, i64& v2, i64& v3, i64& v4)
     sort_desc4(v1, v2, v3, v4);
 }
 
+DMTZ_HD i64 slot_step(const Dims& d, uint32_t slot) {  // index offset of a star slot
+    return DIR[slot][0] + (i64)DIR[slot][1] * d.W + (i64)DIR[slot][2] * d.W * d.H;
+}
+
 // Slot of vertex u in the star of vertex m (u must be a 14-neighbour of m), else -1.
 DMTZ_HD int slot_between(const Dims& d, i64 m, i64 u) {
     i64 mx, my, mz, ux, uy, uz;
