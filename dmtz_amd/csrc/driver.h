@@ -1790,8 +1790,8 @@ __global__ __launch_bounds__(WALL_BLOCK) void k_wall_levels(WallArgs<T> a, ull f
     }
 }
 
-// The chain of every open f-critical face to its first mismatched edge; a face whose chain does not
-// end in WALL_CHAIN_CAP steps is listed in ovf for the search.
+// The chain of every open f-critical face to its first mismatched edge; a face whose chain runs in a
+// circle is listed in ovf for the search.
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_wall_chain(WallArgs<T> a, const uint64_t* starts, ull n, PathList out,
                                                       uint32_t* ovf, ull* ovf_ctr) {
@@ -1803,12 +1803,11 @@ __global__ __launch_bounds__(BLOCK) void k_wall_chain(WallArgs<T> a, const uint6
     i64 face = -1, edge = -1;
     if (i < n) {
         const uint64_t r = starts[i];
-        At t{(uint32_t)(r >> 7), (int)(r & 127u) - LC_TRI}, e{0, 0};
+        const At t{(uint32_t)(r >> 7), (int)(r & 127u) - LC_TRI};
+        At e{0, 0};
         if (wall_open(a.open, graph.face_id(t))) {
-            int s = 0;
-            for (int k = 0; s == 0 && k < WALL_CHAIN_CAP; k++)
-                s = graph.chain_step(t, e, [&](uint32_t id) { return wall_open(a.open, id); });
-            if (s == 1) {
+            i64 steps;
+            if (graph.follow(t, e, [&](uint32_t id) { return wall_open(a.open, id); }, steps) == 1) {
                 has = true;
                 face = local_cell_id(a.d, a.c, (i64)(r >> 7), (int)(r & 127u));
                 edge = rules.edge_number(e);
@@ -1820,7 +1819,7 @@ __global__ __launch_bounds__(BLOCK) void k_wall_chain(WallArgs<T> a, const uint6
     out.push_block(has, face, edge);
 }
 
-// The search itself, for the faces whose chain is capped, and for grids whose faces do not fit the
+// The search itself, for the faces whose chain runs in a circle, and for grids whose faces do not fit the
 // queue's numbers. A face is marked when popped; its edges are taken in the order (v1,v2), (v1,v3),
 // (v2,v3) and pushed in that order, so the last is popped first.
 //

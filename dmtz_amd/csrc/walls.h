@@ -12,7 +12,8 @@
 // As in rules.h, the reference compares partners as plain numbers: a vertex and a face with one
 // number count as equal partners, and an edge paired with a vertex leads on to the face that has the
 // vertex's number if that face is paired with the tet that has the edge's number. Such links can close
-// a cycle, so chains are capped; a face whose chain is longer takes the search of repair.h.
+// a circle (about one chain in 150 thousand over random fields of a few dozen vertices); a face whose
+// chain comes back to itself takes the search of repair.h.
 #pragma once
 #include "repair.h"
 #include "rules.h"
@@ -190,8 +191,26 @@ struct WallGraph {
         t = next;
         return 0;
     }
-};
 
-constexpr int WALL_CHAIN_CAP = 1 << 17;  // faces of a chain, as of a search
+    // The chain from open face t to its end: 1 with the mismatched edge in e, -1 from a face that is not
+    // open, 0 when it runs in a circle. The next face depends on the face alone, so a chain that meets the
+    // face it was at 1, 2, 4, 8, ... steps before never ends; one that ends is followed however long it
+    // is. n receives the number of steps.
+    template <class Open>
+    DMTZ_HD int follow(At t, At& e, Open open, i64& n) const {
+        uint32_t mark = face_id(t);
+        i64 next = 1;
+        for (n = 1;; n++) {
+            const int s = chain_step(t, e, open);
+            if (s != 0) return s;
+            const uint32_t id = face_id(t);
+            if (id == mark) return 0;
+            if (n == next) {
+                mark = id;
+                next *= 2;
+            }
+        }
+    }
+};
 
 }  // namespace dmtz
