@@ -5,6 +5,7 @@
 #include <cstring>
 
 #include "driver.h"
+#include "testing.h"
 
 namespace dmtz_internal {
 int noalloc_setup(int device);  // dmtz_noalloc.hip: device address of its scratch array
@@ -125,6 +126,35 @@ int device(dmtz_ctx* ctx) { return ctx->device; }
 void set_error(dmtz_ctx* ctx, const char* msg) { ctx->err = msg; }
 }  // namespace dmtz_internal
 
+
+extern "C" {
+
+void dmtz_testing_limits(dmtz_ctx* ctx, const int64_t* v) {
+    const decltype(ctx->lim) own{};
+    ctx->lim = own;
+    if (v[0] >= 0) ctx->lim.plane_min = v[0];
+    if (v[1] >= 0) ctx->lim.code_small = v[1];
+    if (v[2] >= 0) ctx->lim.target_dense = (ull)v[2];
+    if (v[3] >= 0) ctx->lim.path_steps = (ull)v[3];
+    if (v[4] >= 0) ctx->lim.wall_level = (ull)v[4];
+}
+
+int dmtz_testing_state(dmtz_ctx* ctx, int64_t n, uint64_t* code_f, uint64_t* code_g, uint64_t* critf_lo,
+                       uint32_t* critf_hi, uint64_t* mm_lo, uint32_t* mm_hi, uint32_t* tile_nz) {
+    if (!ctx || n <= 0 || n > ctx->cap_n) return DMTZ_E_ARG;
+    CK(hipStreamSynchronize(ctx->stream));
+    CK(hipMemcpy(code_f, ctx->d_code_f, 4 * sizeof(uint64_t) * (size_t)n, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(code_g, ctx->d_code_g, 4 * sizeof(uint64_t) * (size_t)n, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(critf_lo, ctx->d_critf.lo, sizeof(uint64_t) * (size_t)n, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(critf_hi, ctx->d_critf.hi, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(mm_lo, ctx->d_mm.lo, sizeof(uint64_t) * (size_t)n, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(mm_hi, ctx->d_mm.hi, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(tile_nz, ctx->d_tile_nz, sizeof(uint32_t) * (size_t)((n + EMIT_TILE - 1) / EMIT_TILE),
+                 hipMemcpyDeviceToHost));
+    return 0;
+}
+
+}  // extern "C"
 
 // Field files (getdata2 main_3d.cu:153-181, saveVectorToBin main_3d.cu:1315-1327). Host code.
 namespace {

@@ -1771,7 +1771,6 @@ __global__ __launch_bounds__(BLOCK) void k_wall_level(WallArgs<T> a, ull from, u
 // many (as long as the longest chain) and small. Every face enters the queue at most once, so the
 // levels end.
 constexpr int WALL_BLOCK = 1024;
-constexpr ull WALL_LEVEL_MIN = 16384;  // larger levels get a launch of their own
 template <class T>
 __global__ __launch_bounds__(WALL_BLOCK) void k_wall_levels(WallArgs<T> a, ull from, ull to) {
     __shared__ WallLds lds;
@@ -1950,6 +1949,15 @@ struct dmtz_ctx {
     ull rec_cap = 0;
     ull fc_cap = 0;
     uint32_t epoch = 0;
+    // Sizes at which the driver changes its route; the reasons stand where each is used. (The tests lower
+    // them, so that small grids take every route: testing.h.)
+    struct {
+        i64 plane_min = (i64)1 << 19;   // vertices from which the dense classification runs over bit planes
+        i64 code_small = (i64)1 << 16;  // vertices up to which every star is re-evaluated
+        ull target_dense = 256;         // records from which an edit set is marked: N over this
+        ull path_steps = (ull)1 << 32;  // steps from which ascending paths are walked, not listed
+        ull wall_level = 16384;         // faces from which a wall level gets a launch of its own
+    } lim;
     std::vector<int64_t> traj;
     double phase[6] = {0, 0, 0, 0, 0, 0};
     // live timing of the dense detection kernel on the context stream (HIP events)
@@ -2265,12 +2273,11 @@ struct Driver {
     // Repair phase of one critical-point sweep (main_3d.cu:6801-6833) + apply (:6837). The kinds are
     // repaired by one launch (the edits form a set: their order does not matter).
 
-    // From N / TARGET_DENSE records on the edit set is marked and applied by a pass over all stamps
+    // From N / lim.target_dense records on the edit set is marked and applied by a pass over all stamps
     // instead of listed. Listing costs a returning atomic per target (about 0.4 ns of the whole chip's
     // time each: 512^3 fBm's first list of 65 M 2-saddles 27.5 -> 13.2 ms with marks), the pass reads
     // 4 N bytes (0.3 ms at 512^3 when it edits little).
-    static constexpr ull TARGET_DENSE = 256;
-    bool mark_targets(ull nrec) const { return nrec * TARGET_DENSE >= (ull)c.N; }
+    bool mark_targets(ull nrec) const { return nrec * ctx->lim.target_dense >= (ull)c.N; }
 
     int fix_cp(const ull counts[4]) {
         int rc = begin_edits(true);
@@ -2352,10 +2359,10 @@ struct Driver {
         if (!est) return 0;
         // Dense from N / 64 changed vertices on where the pass runs over bit planes (512^3: 4.6 ms,
         // where lists of a quarter of the stars took 5 to 8), from N / 16 with a thread per vertex.
-        const ull dense = c.N >= PLANE_MIN ? 64 : 16;
-        // Up to CODE_SMALL vertices (a wave per SIMD) the pass over all of them takes as long as the
+        const ull dense = c.N >= ctx->lim.plane_min ? 64 : 16;
+        // Up to lim.code_small vertices (a wave per SIMD) the pass over all of them takes as long as the
         // shortest list (32^3: 17 us both), and neither the list nor its length is needed.
-        if (c.N <= CODE_SMALL) {
+        if (c.N <= ctx->lim.code_small) {
             est = (ull)c.N;
         } else if (dense * est >= (ull)c.N) {  // many stars may change: decide on the exact count
             int rc = sync_ctr(ctx);
@@ -2476,7 +2483,7 @@ struct Driver {
     // g star codes and mismatch masks of every vertex (the g gradient, main_3d.cu:6624-6638);
     // needs the f-critical masks.
     int g_codes() {
-        if (c.N >= PLANE_MIN) {
+        if (c.N >= ctx->lim.plane_min) {
             k_code_planes<T><<<plane_blocks(), 64, 0, ctx->stream>>>(g, d, Step64(d), c.N, cg(), ctx->d_mm, ctx->d_critf,
                                                                      ctx->d_tile_nz);
             CK(hipGetLastError());
@@ -2490,16 +2497,14 @@ struct Driver {
         return 0;
     }
 
-    // Grids from here on classify over bit planes: below, a wave per 2048 vertices leaves most of the chip
+    // Grids of lim.plane_min vertices or more classify over bit planes: below, a wave per 2048 vertices leaves most of the chip
     // idle and its 55 us of work (float32; 80 in float64) is the time of the pass, against 0.12 us per
     // thousand vertices with a thread per vertex (64^3: 47 us, 129 x 96 x 111 float64: 172).
-    static constexpr i64 PLANE_MIN = (i64)1 << 19;
-    static constexpr i64 CODE_SMALL = (i64)1 << 16;
     unsigned plane_blocks() const { return (unsigned)((c.N + PLANE_TILE - 1) / PLANE_TILE); }
 
     // Star codes of every vertex of a field.
     int codes(const T* fld, CodeArray out, MaskArray own) {
-        if (c.N >= PLANE_MIN) {
+        if (c.N >= ctx->lim.plane_min) {
             k_code_planes<T><<<plane_blocks(), 64, 0, ctx->stream>>>(fld, d, Step64(d), c.N, out, own, MaskArray{nullptr, nullptr}, nullptr);
             CK(hipGetLastError());
             return 0;
@@ -2692,7 +2697,7 @@ struct Driver {
             rc = sync_ctr(ctx);
             if (rc) return rc;
             to = ctx->h_ctr[K_WOPEN];
-            if (to - from < WALL_LEVEL_MIN) break;
+            if (to - from < ctx->lim.wall_level || to == from) break;
             k_wall_level<T><<<nblocks(to - from), BLOCK, 0, ctx->stream>>>(a, from, to);
             CK(hipGetLastError());
             from = to;
@@ -2878,7 +2883,7 @@ struct Driver {
     // Second half, with the number of steps on the host.
     int as_fill(hipStream_t st) {
         as_total = *ctx->h_as_total;
-        as_listed = as_listed && as_total < ((ull)1 << 32);
+        as_listed = as_listed && as_total < ctx->lim.path_steps;
         if (!as_listed || !nfcf || !as_total) return 0;
         int rc = grow_buf(ctx, ctx->d_as_steps, ctx->as_steps_cap, as_total);
         if (rc) return rc;
