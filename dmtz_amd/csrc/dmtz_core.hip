@@ -137,6 +137,7 @@ void dmtz_testing_limits(dmtz_ctx* ctx, const int64_t* v) {
     if (v[2] >= 0) ctx->lim.target_dense = (ull)v[2];
     if (v[3] >= 0) ctx->lim.path_steps = (ull)v[3];
     if (v[4] >= 0) ctx->lim.wall_level = (ull)v[4];
+    if (v[5] >= 0) ctx->lim.wall_queue = (ull)v[5];
 }
 
 int dmtz_testing_state(dmtz_ctx* ctx, int64_t n, uint64_t* code_f, uint64_t* code_g, uint64_t* critf_lo,

@@ -1683,22 +1683,28 @@ struct WallQueue {
         if (threadIdx.x == 0) n = 0;
         __syncthreads();
     }
-    __device__ __forceinline__ void add(uint32_t* open, uint32_t face, uint32_t* queue, ull* ctr) {
+    __device__ __forceinline__ void add(uint32_t* open, uint32_t face, uint32_t* queue, ull cap, ull* ctr) {
         const uint64_t b = (uint64_t)(face / 12u) * 16u + face % 12u;
         const uint32_t bit = 1u << (b & 31u);
         if (atomicOr(open + (b >> 5), bit) & bit) return;
         const uint32_t k = atomicAdd(&n, 1u);
-        if (k < WALL_BUF) id[k] = face;
-        else queue[atomicAdd(ctr, 1ull)] = face;
+        if (k < WALL_BUF) {
+            id[k] = face;
+        } else {
+            const ull at = atomicAdd(ctr, 1ull);
+            if (at < cap) queue[at] = face;
+        }
     }
-    // every thread of the block: after the last add. Returns the end of the queue.
-    __device__ __forceinline__ ull flush(uint32_t* queue, ull* ctr) {
+    // every thread of the block: after the last add. Returns the end of the queue; past cap the faces are
+    // counted but not kept.
+    __device__ __forceinline__ ull flush(uint32_t* queue, ull cap, ull* ctr) {
         __syncthreads();
         const uint32_t m = n < WALL_BUF ? n : WALL_BUF;
         if (threadIdx.x == 0) base = atomicAdd(ctr, (ull)m);
         __syncthreads();
         const ull b = base;
-        for (uint32_t k = threadIdx.x; k < m; k += blockDim.x) queue[b + k] = id[k];
+        for (uint32_t k = threadIdx.x; k < m; k += blockDim.x)
+            if (b + k < cap) queue[b + k] = id[k];
         return b + m;
     }
 };
@@ -1727,6 +1733,7 @@ struct WallArgs {
     Counts c;
     uint32_t* open;
     uint32_t* queue;
+    ull cap;
     ull* ctr;  // faces in the queue
 };
 #define DMTZ_WALL_GRAPH(a, lds)                                                                                    \
@@ -1747,9 +1754,9 @@ __global__ __launch_bounds__(BLOCK) void k_wall_seeds(WallArgs<T> a) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (v < a.c.N)
         graph.mismatched_edges((uint32_t)v, [&](At e) {
-            graph.faces_of(e, [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.ctr); });
+            graph.faces_of(e, [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.cap, a.ctr); });
         });
-    next.flush(a.queue, a.ctr);
+    next.flush(a.queue, a.cap, a.ctr);
 }
 
 // One level: the faces that lead on to the queue's faces [from, to).
@@ -1763,13 +1770,13 @@ __global__ __launch_bounds__(BLOCK) void k_wall_level(WallArgs<T> a, ull from, u
     const ull i = from + (ull)blockIdx.x * BLOCK + threadIdx.x;
     if (i < to)
         graph.leading_to(graph.face_at(a.queue[i]),
-                         [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.ctr); });
-    next.flush(a.queue, a.ctr);
+                         [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.cap, a.ctr); });
+    next.flush(a.queue, a.cap, a.ctr);
 }
 
 // All levels from there on in one block, which only has to wait for itself between them: levels are
 // many (as long as the longest chain) and small. Every face enters the queue at most once, so the
-// levels end.
+// levels end; a queue that is full ends them too.
 constexpr int WALL_BLOCK = 1024;
 template <class T>
 __global__ __launch_bounds__(WALL_BLOCK) void k_wall_levels(WallArgs<T> a, ull from, ull to) {
@@ -1777,13 +1784,13 @@ __global__ __launch_bounds__(WALL_BLOCK) void k_wall_levels(WallArgs<T> a, ull f
     __shared__ WallQueue next;
     lds.load(a.d);
     DMTZ_WALL_GRAPH(a, lds);
-    while (from < to) {
+    while (from < to && to <= a.cap) {
         next.clear();
         for (ull i = from + threadIdx.x; i < to; i += WALL_BLOCK)
             graph.leading_to(graph.face_at(a.queue[i]),
-                             [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.ctr); });
+                             [&](At t) { next.add(a.open, graph.face_id(t), a.queue, a.cap, a.ctr); });
         from = to;
-        to = next.flush(a.queue, a.ctr);
+        to = next.flush(a.queue, a.cap, a.ctr);
         __threadfence();
         __syncthreads();  // the block reads what it has queued
     }
@@ -1957,6 +1964,7 @@ struct dmtz_ctx {
         ull target_dense = 256;         // records from which an edit set is marked: N over this
         ull path_steps = (ull)1 << 32;  // steps from which ascending paths are walked, not listed
         ull wall_level = 16384;         // faces from which a wall level gets a launch of its own
+        ull wall_queue = 0;             // open faces a wall queue holds at first, 0: one per vertex
     } lim;
     std::vector<int64_t> traj;
     double phase[6] = {0, 0, 0, 0, 0, 0};
@@ -2107,14 +2115,14 @@ int grow_fc(dmtz_ctx* ctx, ull need) {
     return 0;
 }
 
-// Grow a device buffer of P to at least need elements (by x1.25 + 4096).
+// Grow a device buffer of P to at least need elements (by x1.25 + 4096, or to need exactly).
 template <class P>
-int grow_buf(dmtz_ctx* ctx, P*& p, size_t& cap, size_t need) {
+int grow_buf(dmtz_ctx* ctx, P*& p, size_t& cap, size_t need, bool exact = false) {
     if (need <= cap) return 0;
     (void)hipFree(p);
     p = nullptr;
     cap = 0;
-    const size_t n = need + need / 4 + 4096;
+    const size_t n = exact ? need : need + need / 4 + 4096;
     CK(hipMalloc(&p, sizeof(P) * n));
     cap = n;
     return 0;
@@ -2673,54 +2681,71 @@ struct Driver {
     }
 
     size_t wall_words() const { return ((size_t)c.N + 1) / 2; }
-    bool wall_buffers() {
-        if (12 * c.N >= ((i64)1 << 32)) return false;
-        if (!grow_buf(ctx, ctx->d_wall_open, ctx->wall_open_cap, wall_words()) &&
-            !grow_buf(ctx, ctx->d_wall_queue, ctx->wall_queue_cap, (size_t)c.F))
+    bool wall_search = false;  // no memory for the open faces: the run searches its walls
+
+    // Room for the open faces' bits and a queue of so many. Most checks open a small part of the 12 faces
+    // per vertex, so the queue begins with one per vertex (both together 6 bytes a vertex, 0.8 GB at 512^3; a
+    // queue of all faces 6.4 GB) and grows when a check opens more.
+    bool wall_room(ull faces) {
+        if (wall_search || 12 * c.N >= ((i64)1 << 32)) return false;
+        if (!grow_buf(ctx, ctx->d_wall_open, ctx->wall_open_cap, wall_words(), true) &&
+            !grow_buf(ctx, ctx->d_wall_queue, ctx->wall_queue_cap, (size_t)faces, true))
             return true;
         (void)hipGetLastError();
+        ctx->err.clear();  // not an error of the call: the search needs neither
+        wall_search = true;
         return false;
     }
     // The walls by chains; left receives the number of faces to search, listed in the second half of
-    // d_wall_ovf.
-    int wall_chains(ull& left) {
-        int rc;
+    // d_wall_ovf. done = false: there was no room, and all faces are to be searched.
+    int wall_chains(bool& done, ull& left) {
         const size_t words = wall_words();
-        const WallArgs<T> a{f, g, cf(), cg(), d, c, ctx->d_wall_open, ctx->d_wall_queue, ctx->d_ctr + K_WOPEN};
-        CK(hipMemsetAsync(ctx->d_wall_open, 0, sizeof(uint32_t) * words, ctx->stream));
-        CK(hipMemsetAsync(ctx->d_ctr + K_WOPEN, 0, sizeof(ull), ctx->stream));
-        CK(hipMemsetAsync(ctx->d_ctr + K_WOVF, 0, sizeof(ull), ctx->stream));
-        k_wall_seeds<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(a);
-        CK(hipGetLastError());
-        ull from = 0, to = 0;
-        for (;;) {
-            rc = sync_ctr(ctx);
-            if (rc) return rc;
-            to = ctx->h_ctr[K_WOPEN];
-            if (to - from < ctx->lim.wall_level || to == from) break;
-            k_wall_level<T><<<nblocks(to - from), BLOCK, 0, ctx->stream>>>(a, from, to);
+        done = wall_room(ctx->lim.wall_queue ? ctx->lim.wall_queue : (ull)c.N);
+        while (done) {
+            const ull cap = (ull)ctx->wall_queue_cap;
+            const WallArgs<T> a{f, g, cf(), cg(), d, c, ctx->d_wall_open, ctx->d_wall_queue, cap, ctx->d_ctr + K_WOPEN};
+            CK(hipMemsetAsync(ctx->d_wall_open, 0, sizeof(uint32_t) * words, ctx->stream));
+            k_zero_ctrs<<<1, 64, 0, ctx->stream>>>(ctx->d_ctr, ctr_bit(K_WOPEN) | ctr_bit(K_WOVF) | ctr_bit(K_DSW));
             CK(hipGetLastError());
-            from = to;
+            k_wall_seeds<T><<<nblocks(c.N), BLOCK, 0, ctx->stream>>>(a);
+            CK(hipGetLastError());
+            ull from = 0, to = 0;
+            for (;;) {
+                int rc = sync_ctr(ctx);
+                if (rc) return rc;
+                to = ctx->h_ctr[K_WOPEN];
+                if (to > cap || to - from < ctx->lim.wall_level || to == from) break;
+                k_wall_level<T><<<nblocks(to - from), BLOCK, 0, ctx->stream>>>(a, from, to);
+                CK(hipGetLastError());
+                from = to;
+            }
+            left = 0;
+            if (to == 0) return 0;
+            if (to <= cap) {
+                k_wall_levels<T><<<1, WALL_BLOCK, 0, ctx->stream>>>(a, from, to);
+                CK(hipGetLastError());
+                k_wall_chain<T><<<nblocks(nfcf), BLOCK, 0, ctx->stream>>>(
+                    a, fcrit_lists(ctx).l[2], nfcf, path_list(2), ctx->d_wall_ovf + nfcf, ctx->d_ctr + K_WOVF);
+                CK(hipGetLastError());
+                int rc = sync_ctr(ctx);
+                if (rc) return rc;
+                to = ctx->h_ctr[K_WOPEN];
+                left = ctx->h_ctr[K_WOVF];
+                if (to <= cap) return 0;
+            }
+            // more faces than the queue holds: again, with room for at least those counted so far
+            const ull want = to > 4 * cap ? to : 4 * cap;
+            done = wall_room(want < (ull)c.F ? want : (ull)c.F);
         }
-        left = 0;
-        if (to == 0) return 0;
-        k_wall_levels<T><<<1, WALL_BLOCK, 0, ctx->stream>>>(a, from, to);
-        CK(hipGetLastError());
-        k_wall_chain<T><<<nblocks(nfcf), BLOCK, 0, ctx->stream>>>(a, fcrit_lists(ctx).l[2], nfcf, path_list(2),
-                                                                   ctx->d_wall_ovf + nfcf, ctx->d_ctr + K_WOVF);
-        CK(hipGetLastError());
-        rc = sync_ctr(ctx);
-        if (rc) return rc;
-        left = ctx->h_ctr[K_WOVF];
         return 0;
     }
 
     // 2-saddle walls (preserve_connectors, main_3d.cu:5064-5133) from every f-critical face into the
     // wall list: the open faces (levels backwards from the mismatched edges), then a chain per open
     // f-critical face. The faces left over (all of them, where the device has no memory for the queue)
-    // are searched in tiers of visited-set size: with 256 slots, the
-    // walks that outgrow them with 8192, then with 2^18; a search of more than 2^17 faces is a capacity
-    // error. Launches are chunked to keep the per-thread sets near 1 GiB.
+    // are searched in tiers of visited-set size: with 256 slots, the walks that outgrow them with 8192,
+    // then with 2^18; a search of more than 2^17 faces is a capacity error. Launches are chunked to keep
+    // the per-thread sets near 1 GiB.
     int walls() {
         CK(hipMemsetAsync(ctx->d_ctr + K_DSW, 0, sizeof(ull), ctx->stream));
         if (!nfcf) return 0;
@@ -2735,10 +2760,15 @@ struct Driver {
         Lists4 FL = fcrit_lists(ctx);
         const uint32_t* sel = nullptr;
         ull n = nfcf;
-        if (wall_buffers()) {
+        bool done = false;
+        ull left = 0;
+        rc = wall_chains(done, left);
+        if (rc) return rc;
+        if (done) {
             sel = ctx->d_wall_ovf + nfcf;
-            rc = wall_chains(n);
-            if (rc) return rc;
+            n = left;
+        } else {  // a check that ran out of room may have listed some
+            CK(hipMemsetAsync(ctx->d_ctr + K_DSW, 0, sizeof(ull), ctx->stream));
         }
         for (int tier = 0; tier < 3 && n > 0; tier++) {
             const uint32_t slots = tiers[tier];

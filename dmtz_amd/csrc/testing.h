@@ -8,7 +8,7 @@
 extern "C" {
 
 // The sizes of dmtz_ctx::lim, in its order; a negative value restores the library's own.
-constexpr int DMTZ_TESTING_LIMITS = 5;
+constexpr int DMTZ_TESTING_LIMITS = 6;
 void dmtz_testing_limits(dmtz_ctx* ctx, const int64_t* values);
 
 // Star codes of f and g (4 n words each, word by word), the f-critical and the mismatch masks (n each) and

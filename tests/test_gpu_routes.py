@@ -13,7 +13,9 @@ context's (dmtz_amd/csrc/testing.h), so that these tests can move them:
     listed and with edit sets marked;
   - separatrix checks that walk the ascending paths instead of listing them;
   - whole corrections of grids just above the sizes of the rules as they are, bit-exact with the oracle;
-  - the wall lists with every level in a launch of its own, and with every level in one block.
+  - the wall lists with every level in a launch of its own, and with every level in one block;
+  - the wall lists from a queue that has to grow, and without memory for one, where all walls are searched;
+    the memory that a wall check keeps.
 """
 import ctypes
 
@@ -31,7 +33,7 @@ NEVER = 1 << 32
 
 class Limits:
     """The context's sizes within a with block; those not named stay the library's own."""
-    NAMES = ("plane_min", "code_small", "target_dense", "path_steps", "wall_level")
+    NAMES = ("plane_min", "code_small", "target_dense", "path_steps", "wall_level", "wall_queue")
 
     def __init__(self, ctx, **values):
         assert set(values) <= set(self.NAMES)
@@ -184,3 +186,49 @@ def test_wall_levels(oracle, dev):
     for level in (-1, NEVER):
         with Limits(dev, wall_level=level):
             assert _wall_set(dmtz_amd.walls(f, g, 1.0, 1.0, ctx=dev)) == want
+
+
+def _wall_pairs():
+    """Noise, whose mismatched edges open most faces; a smooth field with a few vertices lowered, whose walls
+    are large: some outgrow the first two tiers of the search's visited sets."""
+    r = np.random.default_rng(6)
+    f = r.standard_normal((40, 41, 42)).astype(np.float32)
+    yield "noise", f, (f + 0.3 * r.standard_normal(f.shape)).astype(np.float32)
+    f = fields.gaussian_mixture((64, 60, 62), 6, seed=2, noise=0.0)
+    g = f.copy()
+    g.flat[r.integers(0, f.size, 40)] -= np.float32(0.05)
+    yield "smooth", f, g
+
+
+@pytest.mark.parametrize("level", [-1, 1, NEVER])
+@pytest.mark.parametrize("queue", [1, 1 << 60], ids=["grows", "no_memory"])
+def test_wall_queue(oracle, queue, level):
+    fl = oracle.flags(preserve_vpath=1, preserve_geometry=1, preserve_connectors=1)
+    with dmtz_amd.Context(0) as ctx:  # a context of its own: a queue is kept once it has grown
+        for name, f, g in _wall_pairs():
+            print("wall queue", queue, level, name, flush=True)
+            want = oracle.paths(f, g, fl)
+            want = sorted(zip(want["wall"].tolist(), want["wall_rec"].tolist()))
+            assert len(want) > 0
+            with Limits(ctx, wall_queue=queue, wall_level=level):
+                for _ in range(2):
+                    assert _wall_set(dmtz_amd.walls(f, g, 1.0, 1.0, ctx=ctx)) == want
+            assert ctx.error() == ""  # the search is no error
+
+
+def test_wall_memory():
+    """A check that opens few faces keeps at most 16 bytes a vertex for them, not room for all 12 faces."""
+    import torch
+
+    f = fields.fbm((160, 160, 160), seed=3)
+    eps, rng = fields.eps_from_rel(f, 1e-3)
+    fl = dmtz_amd.CorrectionFlags(preserve_vpath=1, preserve_geometry=1, max_sweeps=200)
+    with dmtz_amd.Context(0) as ctx:
+        g = dmtz_amd.correct(f, fields.quantize(f, eps), eps, rng, fl, ctx=ctx).g
+        dmtz_amd.paths(f, g, dmtz_amd.CorrectionFlags(preserve_geometry=0), ctx=ctx)  # what the checks share
+        free = torch.cuda.mem_get_info()[0]
+        print("wall memory", f.shape, flush=True)
+        assert len(dmtz_amd.walls(f, g, eps, rng, fl, ctx=ctx)["face"]) > 0
+        kept = free - torch.cuda.mem_get_info()[0]
+        print("kept", kept / f.size, "bytes a vertex", flush=True)
+        assert kept <= 16 * f.size
