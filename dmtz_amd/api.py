@@ -118,7 +118,7 @@ class Context:
 
     def run_info(self):
         """Last correction: dict(stalls, finished, radius, stars) (finisher outcome and the
-        number of lower stars re-evaluated incrementally)."""
+        number of lower stars re-evaluated after edits; small grids re-evaluate all of theirs)."""
         out = np.zeros(4, np.int64)
         self._lib.dmtz_run_info(self._h, out.ctypes.data_as(ctypes.c_void_p))
         return dict(zip(("stalls", "finished", "radius", "stars"), (int(x) for x in out)))

@@ -6,21 +6,27 @@
 // MI355X (gfx950) implementation of the DMTz topology-correction path behind include/dmtz.h.
 //
 // Device work (one HIP stream per context):
-//   k_code        lower star of every vertex -> 32-byte star code (the gradient of
-//                 main_3d.cu:1930-2316 restricted to each vertex's lower star)
+//   k_code, k_code_g, k_code_planes
+//                 lower star of every vertex -> 32-byte star code (the gradient of
+//                 main_3d.cu:1930-2316 restricted to each vertex's lower star), a thread per vertex
+//                 or, on large grids, over bit planes
 //   k_critf_gather  f-critical status of the 75 local cells of every vertex (once per run)
 //   k_detect      mismatch records from the g star codes and the f-critical masks
 //                 (get_false_* main_3d.cu:2492-2550), 4 typed lists
 //   k_fix_cp      repair rules over a record list -> edit set (main_3d.cu:2554-4303)
-//   k_apply       epsilon-checked edit of the edit set (applyDeltaBuffer1 main_3d.cu:1122-1164)
-//   k_dirty, k_code_list
+//   k_apply, k_apply_marked
+//                 epsilon-checked edit of the edit set (applyDeltaBuffer1 main_3d.cu:1122-1164),
+//                 listed or marked
+//   k_dirty (or k_dirty_mark + k_dirty_collect), k_code_list_g
 //                 re-evaluation of the g star codes around the vertices whose value changed
 //   k_fcrit       f-critical cells (for separatrix checks and filtration)
 //   k_pairs, k_as_walk, k_mism_full / k_mism_marked, k_as_bad + k_as_list, k_ds_list
 //                 separatrix checks, geometry (main_3d.cu:4437-4497, 4837-4959)
 //   k_labels, k_as_branch + k_as_combine, k_ds_branch + k_ds_combine
 //                 separatrix checks, connectivity (main_3d.cu:4499-4835, 4961-5062)
-//   k_fix_paths   separatrix repairs (main_3d.cu:5135-5295)
+//   k_wall_seeds, k_wall_level, k_wall_levels, k_wall_chain, k_ds_wall
+//                 2-saddle walls (main_3d.cu:5064-5133)
+//   k_fix_paths   separatrix and wall repairs (main_3d.cu:5135-5413)
 //   k_pin         filtration (main_3d.cu:2405-2490)
 //   k_zone_cells, k_zone, k_snap_boxes, k_tie_mark, k_tie_raise, k_freeze_all
 //                 the optional finisher at stalls (no counterpart in the reference)
@@ -233,7 +239,6 @@ __device__ __forceinline__ void block_emit(i64 base, const uint64_t (&lo)[EMIT_V
 // ------------------------------------------------------------------------------------------------
 // Kernels
 // ------------------------------------------------------------------------------------------------
-// Star codes of every vertex (dense) or of the listed vertices.
 // 75-bit mask over the local cells of a vertex: the f-critical status of every local cell
 // (mismatch.h: local_crit), or the mismatched cells a vertex owns in g.
 struct CritMask {
@@ -257,8 +262,8 @@ constexpr double MASK_BYTES = sizeof(uint64_t) + sizeof(uint32_t);
 // the code kernels at 128 VGPRs: four waves per SIMD to hide the loads of the star values.
 constexpr int CODE_BLOCKS_PER_CU = 4;
 
-// own (lo nullable) receives the critical cells each vertex owns, from the lower star itself (the
-// first pass of the f-critical masks, without reading the codes back).
+// Star codes of every vertex. own (lo nullable) receives the critical cells each vertex owns, from the
+// lower star itself (the first pass of the f-critical masks, without reading the codes back).
 template <class T>
 __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code(const T* fld, Dims d, Counts c, CodeArray code,
                                                                     MaskArray own) {
@@ -358,13 +363,14 @@ __global__ __launch_bounds__(BLOCK, CODE_BLOCKS_PER_CU) void k_code_list_g(const
 
 // The dense classifications over bit planes (star_planes.h): a wave takes PLANE_TILE consecutive
 // vertices, lane l and bit 31 - b the vertex base + 64 b + l, so that a row of a tile is 64
-// consecutive vertices, read and written coalesced. About 23 thousand instructions per tile, a third of
-// them comparisons; the words of the passes take all 512 registers, so one wave runs per SIMD and
-// the instruction issue of that wave is the bound. 512^3 float32: 15.2 ms with a thread per vertex,
-// now 4.6 (the bytes alone take about 1.5 ms); 256^3: 1.99 -> 0.61 ms. With 256 registers and two waves
-// the spills cost more than the second wave gives (15 ms). Codes and masks are stored word by word
-// (CodeArray, MaskArray): as 32-byte structs, whose words leave a tile at different times, the lines
-// were written to memory several times over (23.5 GB instead of 6.4 at 512^3, 10.7 ms).
+// consecutive vertices, read and written coalesced. About 21 thousand vector instructions per tile, a
+// third of them comparisons; the words of the passes take all 512 registers, so one wave runs per SIMD. It
+// issues half of its time and waits for its loads and stores most of the rest, with no second wave to
+// cover that (counters at 512^3: 50 % issuing, 44 % waiting). 512^3 float32: 15.2 ms with a thread per
+// vertex, now 4.75 (9.4 GB, 2.0 TB/s; at the issue limit it would be 2.3); 256^3: 1.99 -> 0.61 ms. With 256
+// registers and two waves the spills cost more than the second wave gives (15 ms). Codes and masks are
+// stored word by word (CodeArray, MaskArray): as 32-byte structs, whose words leave a tile at different
+// times, the lines were written to memory several times over (23.5 GB instead of 6.4 at 512^3, 10.7 ms).
 static_assert(PLANE_TILE == EMIT_TILE, "a wave's count of nonzero masks is its tile's");
 
 // Stores of a tile: codes, and per vertex its owned critical cells (crit_f null) or the mismatch
@@ -439,8 +445,8 @@ __global__ __launch_bounds__(64, 1) void k_code_planes(const T* fld, Dims d, Ste
 
 // f-critical status of the local cells of every vertex (once per run), in two passes: each
 // vertex writes the critical cells it owns (k_code's own output, or k_critf_own from the codes),
-// then gathers the ones its 14 neighbours own that contain it (k_critf_gather: 15 coalesced
-// 16-byte reads and one store per vertex; the reverse, each owner spreading its cells with
+// then gathers the ones its 14 neighbours own that contain it (k_critf_gather: 15 coalesced reads
+// of 12 bytes and one store per vertex; the reverse, each owner spreading its cells with
 // atomics, wrote five times the masks' size to memory and took twice as long).
 __global__ __launch_bounds__(BLOCK) void k_critf_own(CodeArray cf, i64 n, MaskArray out) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
@@ -491,8 +497,7 @@ __global__ __launch_bounds__(BLOCK) void k_critf_gather(MaskArray own, Dims d, i
 }
 
 // Dense mismatch detection: every vertex lists the mismatched cells it owns in g, from the
-// per-vertex mismatch masks kept with the g star codes (16 bytes per vertex). Waves without a
-// mismatch skip the list appends.
+// per-vertex mismatch masks kept with the g star codes (12 bytes per vertex).
 // A tile whose count of nonzero masks is zero is skipped without reading its masks; tiles_read
 // counts the tiles whose masks were read. A grid of at most DETECT_BLOCKS blocks strides over
 // the tiles: block b takes tiles b, b + grid, ..., reads the counts of 64 of them at once and
@@ -730,8 +735,9 @@ struct HoldSink {
 // packets more and gained nothing on long lists: 256^3 mixtures 68.9 ms per correction, together 61.8;
 // 512^3 fBm 105.0 either way.) The rule runs in vertex frames
 // (rules.h); a record whose numbers collide takes the rule over global ids, a wave-rare branch.
-// Bound by its two to five dependent reads (values, then a star code, then the partner's values and
-// code): a list of a few records takes 12 us (2-saddles; 80 over global ids). The records are taken in
+// A record is two to five dependent reads (values, then a star code, then the partner's values and
+// code), and a list of a few records takes their latency: 12 us (2-saddles; 80 over global ids). Long lists
+// are bound by the lines they touch: 512^3 fBm, 90 lists, 78 GB in 19 ms, 4.1 TB/s. The records are taken in
 // the order of their lists: neighbouring records share the lines
 // they read, which is worth more than waves of one branch. (Over global ids, where a wave paid for
 // every branch body with thousands of instructions, the records were grouped by branch first; with
@@ -1211,8 +1217,8 @@ struct PathList {
 // position and a combine step per start cell applies the reference's "first branch that fails"
 // rule and appends to the list in convergent code.
 
-// Pair words (pairs.h) of every vertex of a field. Bound by the reads of the values and of the
-// codes' first two words (the whole 32-byte codes, as lines go).
+// Pair words (pairs.h) of every vertex of a field. Bound by memory: the values, the codes' words 0 and 1
+// and the pair word, 24 bytes a vertex (512^3: 0.94 ms, 5.3 TB/s by the counters).
 template <class T>
 __global__ __launch_bounds__(BLOCK) void k_pairs(const T* fld, CodeArray code, Dims d, i64 n, uint32_t* out) {
     const i64 v = (i64)blockIdx.x * BLOCK + threadIdx.x;
@@ -1930,7 +1936,6 @@ struct dmtz_ctx {
     uint64_t* d_rec = nullptr;    // 4 mismatch record lists of rec_cap entries
     uint64_t* d_fc = nullptr;     // 4 f-critical lists of fc_cap entries
     int64_t* d_path = nullptr;    // ds id/rec, as id/rec, wall id/rec (fc_cap each)
-    // The second stream of the repair phase.
     bool side_stream = true;  // off in batch lanes: no second stream for the path precompute
     uint32_t* d_pairf = nullptr;     // pair words of f and, where branches are walked, of g
     uint32_t* d_pairg = nullptr;
@@ -1972,7 +1977,7 @@ struct dmtz_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double det_launches = 0, det_ms = 0, det_bytes = 0, det_voxels = 0;
     std::vector<dmtz_ctx*> workers;  // batch lanes: contexts of their own (stream, buffers)
-    double dirty_total = 0;  // star codes re-evaluated incrementally in the last correction
+    double dirty_total = 0;  // star codes re-evaluated after edits in the last correction
     int64_t stalls = 0, finished = 0, radius = 0;  // finisher outcome of the last correction
     // precomputed ascending separatrix paths of f (geometry mode)
     uint32_t* d_as_cnt = nullptr;  // steps per f-critical face, then scanned into d_as_off
@@ -2368,8 +2373,10 @@ struct Driver {
         // Dense from N / 64 changed vertices on where the pass runs over bit planes (512^3: 4.6 ms,
         // where lists of a quarter of the stars took 5 to 8), from N / 16 with a thread per vertex.
         const ull dense = c.N >= ctx->lim.plane_min ? 64 : 16;
-        // Up to lim.code_small vertices (a wave per SIMD) the pass over all of them takes as long as the
-        // shortest list (32^3: 17 us both), and neither the list nor its length is needed.
+        // Up to lim.code_small vertices (a wave per SIMD) the pass over all of them takes no longer than
+        // the shortest list (32^3: 17 us both), and neither the list nor its length is needed: whole
+        // corrections of 2 to 65 thousand vertices, both types, are 2 to 10 % faster than over lists (40^3
+        // mixture 7.70 against 8.58 ms); at 110 thousand 2 % faster, at 176 thousand 7 % slower.
         if (c.N <= ctx->lim.code_small) {
             est = (ull)c.N;
         } else if (dense * est >= (ull)c.N) {  // many stars may change: decide on the exact count
@@ -2505,9 +2512,10 @@ struct Driver {
         return 0;
     }
 
-    // Grids of lim.plane_min vertices or more classify over bit planes: below, a wave per 2048 vertices leaves most of the chip
-    // idle and its 55 us of work (float32; 80 in float64) is the time of the pass, against 0.12 us per
-    // thousand vertices with a thread per vertex (64^3: 47 us, 129 x 96 x 111 float64: 172).
+    // Grids of lim.plane_min vertices or more classify over bit planes: below, a wave per 2048 vertices
+    // leaves most of the chip idle and its 50 to 60 us of work are the time of the pass, in both types,
+    // against 0.125 us per thousand vertices with a thread per vertex (393 k vertices: 51 and 54 us, the same
+    // over planes; 524 k: 65 and 71 against 50 and 60; 1.4 M: 165 against 57 and 68).
     unsigned plane_blocks() const { return (unsigned)((c.N + PLANE_TILE - 1) / PLANE_TILE); }
 
     // Star codes of every vertex of a field.

@@ -351,7 +351,6 @@ template <class Code>
 DMTZ_HD int partner_tet_of(const Code& c, i64 v, int q) { return (int)(code_word(c, v, 1) >> (14 + 2 * q)) & 3; }
 
 DMTZ_HD int code_edge(const StarCode& c, int a) { return (int)((c.w[0] >> (4 * a)) & 15u); }
-DMTZ_HD int code_s(const StarCode& c) { return (int)((c.w[0] >> 56) & 15u); }
 DMTZ_HD uint32_t code_L(const StarCode& c) { return (uint32_t)(c.w[1] & 0x3FFFu); }
 DMTZ_HD int code_tet(const StarCode& c, int q) { return (int)((c.w[1] >> (14 + 2 * q)) & 3u); }
 DMTZ_HD int code_tri(const StarCode& c, int t) {

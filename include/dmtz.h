@@ -239,7 +239,7 @@ int dmtz_phase_times(const dmtz_ctx* ctx, double* out6);
 int dmtz_kernel_stats(dmtz_ctx* ctx, double* out4, int reset);
 
 /* Outcome of the last correction on ctx beyond the counts: out4 = {stalls, vertices changed by
- * the finisher, finisher radius reached, lower stars re-evaluated incrementally}. No reference
+ * the finisher, finisher radius reached, lower stars re-evaluated after edits}. No reference
  * counterpart (the reference neither detects stalls nor finishes them). */
 int dmtz_run_info(const dmtz_ctx* ctx, int64_t* out4);
 
