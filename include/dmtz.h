@@ -280,7 +280,8 @@ int dmtz_paths_f64(dmtz_ctx* ctx, const double* f, const double* g, int64_t nx, 
  * id) pairs, as many as cap allows (in no particular order). When targets is non-null it
  * receives the edit set of fix_ds_wall (main_3d.cu:5297-5413) over the list; eps and range enter
  * its threshold, and flags (nullable) its edit_type. DMTZ_E_CAPACITY if a walk that has to be searched
- * (one whose chain of open faces runs in a circle) visits more than 2^17 faces. */
+ * (its chain of open faces runs in a circle, or the device has no memory for the open faces) visits
+ * more than 2^17 faces. */
 int dmtz_walls_f32(dmtz_ctx* ctx, const float* f, const float* g, int64_t nx, int64_t ny, int64_t nz, double eps,
                    double range, const dmtz_flags* flags, int64_t* count, int64_t* face, int64_t* edge, int64_t cap,
                    uint8_t* targets);
